@@ -30,6 +30,7 @@
 #include <cstring>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 
 namespace cg = cooperative_groups;
 
@@ -41,10 +42,12 @@ constexpr float kRealtimeDamping = 0.05f;
 constexpr float kSurfaceTolerance = 1.0e-5f;
 constexpr float kRestOffset = 1.0e-3f;
 constexpr uint32_t kSideFirst = 0x80000000u;
-// Colour-ordered entry, second word: the other body, and this flag when it
-// is dynamic and of a lower colour (the dataflow sweep waits for it).
+// Colour-ordered entry, second word: the other body, and a flag when it is
+// dynamic and of a lower colour (the dataflow sweep waits for it) or not
+// dynamic (no sweep moves it).
 constexpr uint32_t kEntryLower = 0x80000000u;
-constexpr uint32_t kEntryBody = 0x7fffffffu;
+constexpr uint32_t kEntryFixed = 0x40000000u;
+constexpr uint32_t kEntryBody = kMaxBodies;
 
 __device__ __forceinline__ uint32_t ld_relaxed(const uint32_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -53,27 +56,58 @@ __device__ __forceinline__ void st_relaxed(uint32_t *p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Agent-coherent 64-bit words: relaxed agent-scope atomics, issued as
-// global_load/global_store with the sc1 bit.  The dataflow sweep hands
-// displacements between the wavefronts of one launch with them: inside a
-// kernel the L2 caches of the eight XCDs are not coherent with each other
-// for ordinary accesses.
-__device__ __forceinline__ uint64_t ld64_co(const float *p) {
-    return __hip_atomic_load(reinterpret_cast<const uint64_t *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// A lane exchange inside the wavefront as an operand modifier (DPP): the add
+// or multiply that uses it takes no extra instruction, where __shfl goes
+// through the LDS pipe (ds_bpermute).  Every lane must be active.
+enum : int { kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140, kDppRowShr = 0x110,
+             kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143, kDppNewBcast = 0x150 };
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
+    return uint32_t(__builtin_amdgcn_update_dpp(0, int(x), kCtrl, 0xf, 0xf, true));
 }
-__device__ __forceinline__ void st64_co(float *p, float x, float y) {
-    const uint64_t v = uint64_t(__float_as_uint(x)) | (uint64_t(__float_as_uint(y)) << 32);
-    __hip_atomic_store(reinterpret_cast<uint64_t *>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+template <int kCtrl>
+__device__ __forceinline__ float dpp_f32(float x) { return __uint_as_float(dpp_u32<kCtrl>(__float_as_uint(x))); }
+// The value of lane kLane of each 16-lane row.
+template <int kLane>
+__device__ __forceinline__ float row_bcast(float x) { return dpp_f32<kDppNewBcast + kLane>(x); }
+// The value of the odd row of each pair of rows, in both.
+__device__ __forceinline__ float odd_row(float x) {
+    return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);
 }
-__device__ __forceinline__ float lo_f(uint64_t v) { return __uint_as_float(uint32_t(v)); }
-__device__ __forceinline__ float hi_f(uint64_t v) { return __uint_as_float(uint32_t(v >> 32)); }
-__device__ __forceinline__ float4 ld4_co(const float4 *p) {
-    const uint64_t a = ld64_co(&p->x), b = ld64_co(&p->z);
-    return make_float4(lo_f(a), hi_f(a), lo_f(b), hi_f(b));
+
+// Combines a value over the wavefront; the result is in lane 63 (zero is
+// neutral in every use: sums and maxima of unsigned values).
+template <class T, class F>
+__device__ __forceinline__ T wave_fold(T x, F f) {
+    auto step = [&](auto moved) { x = f(x, moved); };
+    auto move = [](auto ctrl, T v) -> T {
+        if constexpr (sizeof(T) == 8)
+            return (T(dpp_u32<decltype(ctrl)::value>(uint32_t(v >> 32))) << 32) | dpp_u32<decltype(ctrl)::value>(uint32_t(v));
+        else
+            return dpp_u32<decltype(ctrl)::value>(v);
+    };
+    step(move(std::integral_constant<int, kDppRowShr + 1>{}, x));
+    step(move(std::integral_constant<int, kDppRowShr + 2>{}, x));
+    step(move(std::integral_constant<int, kDppRowShr + 4>{}, x));
+    step(move(std::integral_constant<int, kDppRowShr + 8>{}, x));
+    step(move(std::integral_constant<int, kDppRowBcast15>{}, x));
+    step(move(std::integral_constant<int, kDppRowBcast31>{}, x));
+    return x;
 }
-__device__ __forceinline__ void st4_co(float4 *p, float4 v) {
-    st64_co(&p->x, v.x, v.y);
-    st64_co(&p->z, v.z, v.w);
+
+// Mailboxes of the dataflow sweep: eight 64-bit words per body, each a float
+// and the stamp of the sweep that wrote it (displacement, then the rotation
+// delta's w).  A reader needs no second look at a flag and the writer no wait
+// between data and flag: a word whose stamp is this sweep's holds this
+// sweep's value.  Written by 64-bit agent-scope stores, read two words per
+// 16-byte agent-scope load (the sc1 bit: the L2 caches of the eight XCDs are
+// not coherent with each other inside a kernel); each word is consistent in
+// itself and the stamps tell whether all of them have arrived.
+constexpr uint32_t kFlowUsed = 7;
+constexpr int kLoadAgent = 16;   // buffer load cache policy: sc1
+typedef uint32_t flow_pair __attribute__((ext_vector_type(4)));   // two words: value, stamp, value, stamp
+__device__ __forceinline__ flow_pair flow_load(__amdgpu_buffer_rsrc_t box, uint32_t body, int pair) {
+    return __builtin_amdgcn_raw_buffer_load_b128(box, int(body * (kFlowWords * 8u)), 16 * pair, kLoadAgent);
 }
 
 // Sum over a converged wavefront (every lane active).
@@ -851,8 +885,9 @@ __global__ void k_bp_fill(const StepCounters *ctr, const uint32_t *start, const 
         const uint2 p = ab[m];
         const bool first = p.x == i;
         const uint32_t other = first ? p.y : p.x;
-        // Static bodies hold no colour (kInvalid): never lower.
-        const uint32_t tag = other | (color[other] < ci ? kEntryLower : 0u);
+        // Only dynamic bodies hold a colour.
+        const uint32_t co = color[other];
+        const uint32_t tag = other | (co == kInvalid ? kEntryFixed : co < ci ? kEntryLower : 0u);
         for (uint32_t q = 0; q < m_count[m]; ++q) {
             c_entry[2 * (m_start[m] + q) + (first ? 0u : 1u)] = o;
             entries[o++] = make_uint2((m_start[m] + q) | (first ? kSideFirst : 0u), tag);
@@ -956,10 +991,10 @@ struct SolveArgs {
     uint32_t nj;
     const uint32_t *jstart, *jadj;       // per-body incident joints, descending index
     const PmhRigidBodyState *prev;
-    // dataflow sweep: colours, published stamps, this sweep's stamp (0: not
-    // in a dataflow sweep) and the poll limit of its waits
+    // dataflow sweep: colours, the mailboxes, this sweep's stamp and the poll
+    // limit of its waits
     const uint32_t *color;
-    uint32_t *done;
+    unsigned long long *flow;
     uint32_t flow_stamp, flow_limit;
 };
 
@@ -994,28 +1029,25 @@ __device__ __forceinline__ void load_disp(const float4 *disp, uint32_t i, float 
     const float4 a = disp[2 * i], b = disp[2 * i + 1];
     d[0] = a.x; d[1] = a.y; d[2] = a.z; d[3] = b.x; d[4] = b.y; d[5] = b.z;
 }
-// Another body's displacement inside a dataflow sweep (agent-coherent).
-__device__ __forceinline__ void load_disp_co(const float4 *disp, uint32_t i, float *d) {
-    const float *p = &disp[2 * i].x;
-    const uint64_t t = ld64_co(p), tz = ld64_co(p + 2), r = ld64_co(p + 4), rz = ld64_co(p + 6);
-    d[0] = lo_f(t); d[1] = hi_f(t); d[2] = lo_f(tz); d[3] = lo_f(r); d[4] = hi_f(r); d[5] = lo_f(rz);
-}
-__device__ __forceinline__ void load_disp_a(const SolveArgs &a, uint32_t i, float *d) {
-    if (a.flow_stamp) load_disp_co(a.disp, i, d);
-    else load_disp(a.disp, i, d);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t flow_box(const SolveArgs &a) {
+    return __builtin_amdgcn_make_buffer_rsrc(a.flow, 0, int(a.n * (kFlowWords * 8u)), 0x00020000);
 }
 
-// Dataflow sweep: waits until body j has published this sweep's
-// displacement.  Bounded: a wait that runs out raises the abort flag, which
-// ends every other wait of the step, and marks the status, so the step
-// fails instead of hanging.
-// A wait that runs out also marks the sweep failed (kept until the host
-// reports it): the step then keeps its states and fails.  The abort flag
-// is read every 256th poll only: thousands of waiting lanes reading one
-// address on every poll would queue on one memory channel, and the waits
-// would slow down the bodies they wait for.
-__device__ __forceinline__ void wait_published(const SolveArgs &a, uint32_t j) {
-    for (uint32_t polls = 1; int32_t(ld_relaxed(&a.done[j]) - a.flow_stamp) < 0; ++polls) {
+// Dataflow sweep: waits until body j has published this sweep's displacement
+// and takes it.  Bounded: a wait that runs out raises the abort flag, which
+// ends every other wait of the step, and marks the status and the sweep
+// (kept until the host reports it), so the step keeps its states and fails
+// instead of hanging.  The abort flag is read every 256th poll only:
+// thousands of waiting lanes reading one address on every poll would queue on
+// one memory channel, and the waits would slow down the bodies they wait for.
+__device__ __forceinline__ void flow_take(const SolveArgs &a, __amdgpu_buffer_rsrc_t box, uint32_t j, float *d) {
+    flow_pair w0, w1, w2;
+    for (uint32_t polls = 1;; ++polls) {
+        w0 = flow_load(box, j, 0);
+        w1 = flow_load(box, j, 1);
+        w2 = flow_load(box, j, 2);
+        const uint32_t s = a.flow_stamp;
+        if (((w0[1] ^ s) | (w0[3] ^ s) | (w1[1] ^ s) | (w1[3] ^ s) | (w2[1] ^ s) | (w2[3] ^ s)) == 0u) break;
         if (polls > a.flow_limit) {
             st_relaxed(&a.ctr->color_abort, 1u);
             st_relaxed(&a.ctr->sweep_failed, 1u);
@@ -1023,15 +1055,21 @@ __device__ __forceinline__ void wait_published(const SolveArgs &a, uint32_t j) {
             break;
         }
         if ((polls & 255u) == 0u && ld_relaxed(&a.ctr->color_abort) != 0u) break;
-        __builtin_amdgcn_s_sleep(2);
+        // The mailbox is read again, not kept from the last poll.
+        asm volatile("s_sleep 1" ::: "memory");
     }
-    asm volatile("" ::: "memory");   // the displacement reads stay after the wait
+    d[0] = __uint_as_float(w0[0]); d[1] = __uint_as_float(w0[2]); d[2] = __uint_as_float(w1[0]);
+    d[3] = __uint_as_float(w1[2]); d[4] = __uint_as_float(w2[0]); d[5] = __uint_as_float(w2[2]);
 }
-// Dataflow sweep: body i's displacement stores (agent-coherent) have
-// completed before the stamp that releases its waiters is stored.
-__device__ __forceinline__ void publish_done(const SolveArgs &a, uint32_t i) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    st_relaxed(&a.done[i], a.flow_stamp);
+// The rotation delta's w of a body whose displacement has been taken.
+__device__ __forceinline__ float flow_take_w(const SolveArgs &a, __amdgpu_buffer_rsrc_t box, uint32_t j) {
+    flow_pair w3;
+    for (uint32_t polls = 1;; ++polls) {
+        w3 = flow_load(box, j, 3);
+        if (w3[1] == a.flow_stamp || polls > a.flow_limit || ld_relaxed(&a.ctr->color_abort) != 0u) break;
+        asm volatile("s_sleep 1" ::: "memory");
+    }
+    return __uint_as_float(w3[0]);
 }
 
 // err = e0 + dot6(JA, dA) + dot6(JB, dB) with JA = (-axis, angA),
@@ -1043,18 +1081,136 @@ __device__ __forceinline__ float row_error(float e0, float4 axis, float4 angA, f
     return e0 + dot6(ja, dA) + dot6(jb, dB);
 }
 
-__device__ void body_joint_rows(const SolveArgs &a, uint32_t i, uint32_t phase, Block &blk, uint32_t sub_lane,
-                                uint32_t L);
+template <bool kFlow>
+__device__ __forceinline__ void body_joint_rows(const SolveArgs &a, uint32_t i, uint32_t phase, Block &blk,
+                                                uint32_t sub_lane, uint32_t L, const float *dI, float wI);
 
+// A value the optimiser does not look through: a choice between such values
+// stays a choice between registers (a choice between elements of one array is
+// otherwise made into an indexed load, and the array goes to scratch).
+__device__ __forceinline__ float held(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+
+// Sums over the L lanes of a group, pairwise as an xor butterfly does (lane
+// k with k ^ 1, then ^ 2, ^ 4, ...): once four lanes agree, mirroring a row
+// half gives the partner quad's value, and so on, so every level is an add
+// with a DPP operand.  The totals are in every lane for L = 8 and 16, in the
+// odd 16-lane rows for 32 and in the last row for 64 (the row broadcasts go
+// one way only): sum_row().  Level by level over all 27 values: a DPP operand
+// may not be read right after it was written.
+template <int kCtrl>
+__device__ __forceinline__ void reduce_level(Block &b) {
+#pragma unroll
+    for (int k = 0; k < 21; ++k) b.h[k] = b.h[k] + dpp_f32<kCtrl>(b.h[k]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) b.g[k] = b.g[k] + dpp_f32<kCtrl>(b.g[k]);
+}
 template <int L>
 __device__ __forceinline__ void group_reduce(Block &b) {
+    reduce_level<kDppXor1>(b);
+    reduce_level<kDppXor2>(b);
+    reduce_level<kDppHalfMirror>(b);
+    if constexpr (L >= 16) reduce_level<kDppMirror>(b);
+    if constexpr (L >= 32) reduce_level<kDppRowBcast15>(b);
+    if constexpr (L >= 64) reduce_level<kDppRowBcast31>(b);
+}
+// First lane of the row that holds the group's totals.
+template <int L>
+__device__ __forceinline__ uint32_t sum_row(uint32_t lane) {
+    return L == 8 ? lane & ~7u : L == 16 ? lane & ~15u : L == 32 ? (lane & 32u) | 16u : 48u;
+}
+// A value of that row, the same in all its lanes, in every lane of the group.
+template <int L>
+__device__ __forceinline__ float from_sum_row(float x) {
+    if constexpr (L == 32) return odd_row(x);
+    if constexpr (L == 64) return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), 63));
+    return x;
+}
+
+// block_solve's first attempt with the rows of the block spread over the
+// lanes of each 16-lane row (lane r holds row r; lanes past 5 repeat row 5):
+// every element meets the same operations in the same order, but a column's
+// divisions run side by side, so a solve takes 6 divisions of latency and
+// issue instead of 21 (an IEEE division is 11 instructions), about 190
+// instructions instead of 510.  False where the first attempt is not the
+// result (a pivot at its floor, an entry out of range): block_solve decides
+// then.  The result is the same in all lanes of the row.
+__device__ __forceinline__ bool solve_rows(const Block &in, uint32_t lane, float *x) {
+    const float largest = 3.402823466e38f, pivot_floor = 8.0f * 1.1920928955078125e-7f;
+    const uint32_t r = lane & 15u;
+    const bool r0 = r == 0u, r1 = r == 1u, r2 = r == 2u, r3 = r == 3u, r4 = r == 4u;
+    float h[21], gr[6];
 #pragma unroll
-    for (int s = 1; s < L; s <<= 1) {
+    for (int k = 0; k < 21; ++k) h[k] = held(in.h[k]);
 #pragma unroll
-        for (int k = 0; k < 21; ++k) b.h[k] = b.h[k] + __shfl_xor(b.h[k], s, 64);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) b.g[k] = b.g[k] + __shfl_xor(b.g[k], s, 64);
+    for (int k = 0; k < 6; ++k) gr[k] = held(in.g[k]);
+    float a0 = r0 ? h[0] : r1 ? h[1] : r2 ? h[3] : r3 ? h[6] : r4 ? h[10] : h[15];
+    float a1 = r2 ? h[4] : r3 ? h[7] : r4 ? h[11] : h[16];
+    float a2 = r3 ? h[8] : r4 ? h[12] : h[17];
+    float a3 = r4 ? h[13] : h[18];
+    float a4 = h[19];
+    const float diag = r0 ? h[0] : r1 ? h[2] : r2 ? h[5] : r3 ? h[9] : r4 ? h[14] : h[20];
+    const float g = r0 ? gr[0] : r1 ? gr[1] : r2 ? gr[2] : r3 ? gr[3] : r4 ? gr[4] : gr[5];
+    bool ok = diag > 0.0f && diag < largest && fabsf(g) < largest && fabsf(a0) < largest && fabsf(a1) < largest &&
+              fabsf(a2) < largest && fabsf(a3) < largest && fabsf(a4) < largest;
+    float d = diag, f = -g;
+    // Column j: the multipliers of the rows below it, then those rows.
+#define PMH_COLUMN(j, aj, REST)                                    \
+    {                                                              \
+        const float dj = row_bcast<j>(d), fj = row_bcast<j>(f);    \
+        const float l = aj / dj;                                   \
+        const float nd = d - l * l * dj, nf = f - l * fj;          \
+        const float t = l * dj;                                    \
+        aj = l;                                                    \
+        d = r > j ? nd : d;                                        \
+        f = r > j ? nf : f;                                        \
+        REST                                                       \
+        (void)t;                                                   \
     }
+    PMH_COLUMN(0, a0, a1 = a1 - t * row_bcast<1>(l); a2 = a2 - t * row_bcast<2>(l); a3 = a3 - t * row_bcast<3>(l);
+               a4 = a4 - t * row_bcast<4>(l);)
+    PMH_COLUMN(1, a1, a2 = a2 - t * row_bcast<2>(l); a3 = a3 - t * row_bcast<3>(l); a4 = a4 - t * row_bcast<4>(l);)
+    PMH_COLUMN(2, a2, a3 = a3 - t * row_bcast<3>(l); a4 = a4 - t * row_bcast<4>(l);)
+    PMH_COLUMN(3, a3, a4 = a4 - t * row_bcast<4>(l);)
+    PMH_COLUMN(4, a4, )
+#undef PMH_COLUMN
+    ok = ok && d > pivot_floor * diag && d < largest;
+    const float q = f / d;
+    x[5] = row_bcast<5>(q);
+    x[4] = row_bcast<4>(q) - row_bcast<5>(a4) * x[5];
+    x[3] = row_bcast<3>(q) - row_bcast<4>(a3) * x[4] - row_bcast<5>(a3) * x[5];
+    x[2] = row_bcast<2>(q) - row_bcast<3>(a2) * x[3] - row_bcast<4>(a2) * x[4] - row_bcast<5>(a2) * x[5];
+    x[1] = row_bcast<1>(q) - row_bcast<2>(a1) * x[2] - row_bcast<3>(a1) * x[3] - row_bcast<4>(a1) * x[4] -
+           row_bcast<5>(a1) * x[5];
+    x[0] = row_bcast<0>(q) - row_bcast<1>(a0) * x[1] - row_bcast<2>(a0) * x[2] - row_bcast<3>(a0) * x[3] -
+           row_bcast<4>(a0) * x[4] - row_bcast<5>(a0) * x[5];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) ok = ok && fabsf(x[i]) < largest;
+    return ok;
+}
+
+// Solves the group's block (its totals in the sum row); the update is in
+// every lane of the group, and so is whether there is one.  Converged
+// wavefront; `live` marks the lanes of groups that hold a body.
+template <int L>
+__device__ __forceinline__ bool group_solve(const Block &blk, uint32_t lane, bool live, float *x) {
+    if constexpr (L < 16) return block_solve(blk, x) && live;
+    const uint32_t row = sum_row<L>(lane);
+    bool ok = ((__ballot(solve_rows(blk, lane, x)) >> row) & 0xffffull) == 0xffffull;
+    if (__ballot(live && !ok) != 0ull) {
+        float y[6];
+        const bool solved = ((__ballot(block_solve(blk, y)) >> row) & 1ull) != 0ull;
+        if (!ok) {
+#pragma unroll
+            for (int q = 0; q < 6; ++q) x[q] = y[q];
+            ok = solved;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 6; ++q) x[q] = from_sum_row<L>(x[q]);
+    return ok && live;
 }
 
 // apply_pose_update, geometry_constraints.slang:386-408: the translation
@@ -1085,15 +1241,11 @@ struct ResidualAcc {
 // Combines the lanes of a converged wavefront into the log's slot with one
 // atomic per field (non-negative floats order like their bit patterns).
 __device__ __forceinline__ void residual_commit(ResidualLog *log, uint32_t slot, const ResidualAcc &acc) {
-    uint32_t bits = __float_as_uint(acc.max), count = acc.count;
-    unsigned long long sum = acc.sum;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        bits = max(bits, uint32_t(__shfl_xor(bits, d, 64)));
-        count += uint32_t(__shfl_xor(count, d, 64));
-        sum += (unsigned long long)__shfl_xor((long long)sum, d, 64);
-    }
-    if ((threadIdx.x & 63) == 0 && count) {
+    const uint32_t bits = wave_fold(__float_as_uint(acc.max), [](uint32_t p, uint32_t q) { return max(p, q); });
+    const uint32_t count = wave_fold(acc.count, [](uint32_t p, uint32_t q) { return p + q; });
+    const unsigned long long sum =
+        wave_fold(acc.sum, [](unsigned long long p, unsigned long long q) { return p + q; });
+    if ((threadIdx.x & 63) == 63 && count) {
         const uint32_t bank = blockIdx.x & (kResidualBanks - 1);
         atomicMax(&log->bits[slot][bank], bits);
         atomicAdd(&log->sum[slot][bank], sum);
@@ -1101,11 +1253,19 @@ __device__ __forceinline__ void residual_commit(ResidualLog *log, uint32_t slot,
     }
 }
 
+// A point's new duals.
+struct DualStep {
+    Force3 f;
+    bool stick;
+};
 // One contact point's dual update (advance_duals, solve.slang:492-566)
 // from both ends' displacements and the point's rows; defined with
 // advance_duals below.
-__device__ void dual_point(const SolveArgs &a, uint32_t c, uint32_t phase, const float *dA, const float *dB,
-                           const float4 *Jx, bool last, ResidualAcc &residual);
+__device__ DualStep dual_point(const SolveArgs &a, uint32_t c, const float *dA, const float *dB, const float4 *Jx,
+                               ResidualAcc &residual);
+__device__ void publish_flow(const SolveArgs &a, uint32_t c, uint32_t phase, uint32_t ia, uint32_t ib,
+                             const DualStep &s, const float *dA, float wA, const float *dB, float wB, V3 t0, V3 t1);
+constexpr uint32_t kFlagSlipping = 4u;   // point flag, see below
 
 // The bodies at colour-ordered positions k = base + group of one wavefront
 // (solve_color, geometry_constraints_solve.slang:331-491).  Each body is
@@ -1114,9 +1274,13 @@ __device__ void dual_point(const SolveArgs &a, uint32_t c, uint32_t phase, const
 // crossing safeguard run on the whole group.
 // kJoints: the world has joints.  Joint-free worlds run the false
 // instance, which carries none of the joint code (registers, stack).
-// kFlow: inside a dataflow sweep (one launch for every colour): a body
-// waits for the lower-colour neighbours it reads, reads other bodies'
-// displacements agent-coherently, and publishes its own with a stamp.
+// kFlow: inside a dataflow sweep (one launch for every colour): a body takes
+// the displacements of its lower-colour neighbours from their mailboxes,
+// waiting for this sweep's, and publishes its own.  Every other body it reads
+// is not written before it publishes (a higher colour waits for it) or not at
+// all, so ordinary loads serve: they see the previous launch's values.
+// In the velocity phase a dynamic neighbour is solved whenever the body is:
+// neighbours share an island, and the impact flag is the island's.
 template <int L, bool kJoints, bool kFlow>
 __device__ __forceinline__ void solve_group(const SolveArgs &a, uint32_t base, uint32_t end, uint32_t phase,
                                             uint32_t it = 0u) {
@@ -1129,14 +1293,17 @@ __device__ __forceinline__ void solve_group(const SolveArgs &a, uint32_t base, u
         i = a.color_bodies[k];
         if (i == kInvalid || (phase != 0 && a.impact[i] == 0)) active = false;
     }
+    const __amdgpu_buffer_rsrc_t box = flow_box(a);
     Block blk;
     block_zero(blk);
     float dI[6] = {0, 0, 0, 0, 0, 0};
+    float4 dq = make_float4(0.0f, 0.0f, 0.0f, 1.0f);
     uint32_t eb = 0, ee = 0;
     if (active) {
         load_disp(a.disp, i, dI);
         eb = a.bp_start[k];
         ee = a.bp_start[k + 1];
+        if (phase == 0) dq = a.dq[i];
         if (sub_lane == 0) {
             const float4 i0 = a.inertia[2 * i], i1 = a.inertia[2 * i + 1];
             // Full packed block of the body: diag(m/dt^2) and the
@@ -1155,11 +1322,10 @@ __device__ __forceinline__ void solve_group(const SolveArgs &a, uint32_t base, u
                     blk.g[r] += h[r > c ? r * (r + 1) / 2 + c : c * (c + 1) / 2 + r] * dI[c];
         }
     }
-    // The crossing safeguard revisits the lane's rows: the first one's
-    // values stay in registers (a lane holds one row in most bodies).
-    float4 keep_axis = make_float4(0.0f, 0.0f, 0.0f, 0.0f), keep_angA = keep_axis, keep_angB = keep_axis;
-    float keep_lam = 0.0f, keep_pen = 0.0f, keep_dO[6] = {0, 0, 0, 0, 0, 0};
-    bool keep_first = false;
+    // The crossing safeguard and the dual update revisit the lane's rows: of
+    // the first one (a lane holds one row in most bodies) the normal row, its
+    // trial force and the other end stay in registers.
+    float keep_row[6] = {0, 0, 0, 0, 0, 0}, keep_trial = 0.0f, keep_pen = 0.0f, keep_dO[6] = {0, 0, 0, 0, 0, 0};
     for (uint32_t e = eb + sub_lane; e < ee; e += L) {
         const uint2 ent = a.entries[e];
         const uint32_t c = ent.x & 0x7fffffffu;
@@ -1170,22 +1336,8 @@ __device__ __forceinline__ void solve_group(const SolveArgs &a, uint32_t base, u
 #pragma unroll
         for (int q = 0; q < 9; ++q) Jx[q] = a.erec[q * a.ecap + e];
         float dO[6];
-        if (kFlow) {
-            if ((ent.y & kEntryLower) != 0u && (phase == 0 || a.impact[other] != 0u)) wait_published(a, other);
-            load_disp_co(a.disp, other, dO);
-        } else {
-            load_disp(a.disp, other, dO);
-        }
-        if (e == eb + sub_lane) {
-            keep_axis = Jx[0];
-            keep_angA = Jx[3];
-            keep_angB = Jx[6];
-            keep_lam = lam.x;
-            keep_pen = pen.x;
-            keep_first = first;
-#pragma unroll
-            for (int q = 0; q < 6; ++q) keep_dO[q] = dO[q];
-        }
+        if (kFlow && (ent.y & kEntryLower) != 0u) flow_take(a, box, other, dO);
+        else load_disp(a.disp, other, dO);
         const float *dA = first ? dI : dO;
         const float *dB = first ? dO : dI;
         const float err0 = row_error(Jx[0].w, Jx[0], Jx[3], Jx[6], dA, dB);
@@ -1204,139 +1356,152 @@ __device__ __forceinline__ void solve_group(const SolveArgs &a, uint32_t base, u
             const float row[6] = {first ? -axis.x : axis.x, first ? -axis.y : axis.y,
                                   first ? -axis.z : axis.z, ang.x, ang.y, ang.z};
             add_row(blk, row, stiff[ax], force[ax]);
+            if (ax == 0 && e == eb + sub_lane) {
+#pragma unroll
+                for (int q = 0; q < 6; ++q) {
+                    keep_row[q] = row[q];
+                    keep_dO[q] = dO[q];
+                }
+                keep_trial = trial.n;
+                keep_pen = pen.x;
+            }
         }
     }
+    // From here to the mailbox the wavefront is on the chain over the
+    // colours; wavefronts that wait or update duals give way.
+    if constexpr (kFlow && L >= 16) __builtin_amdgcn_s_setprio(3);
     // Joint rows follow the contact rows (solve.slang:401-430), each
     // joint in one lane's partial block.
-    if (kJoints && active) body_joint_rows(a, i, phase, blk, sub_lane, L);
+    if (kJoints && active) body_joint_rows<kFlow>(a, i, phase, blk, sub_lane, L, dI, dq.w);
     group_reduce<L>(blk);
     float update[6];
-    const bool solved = active && block_solve(blk, update);
-    // Crossing safeguard (solve.slang:433-475).
-    Block cross_blk;
-    block_zero(cross_blk);
-    bool crossing = false;
-    if (solved) {
-        for (uint32_t e = eb + sub_lane; e < ee; e += L) {
-            float4 axis, angA, angB;
-            float lam0, k0, dO[6];
-            bool first;
-            if (e == eb + sub_lane) {
-                axis = keep_axis;
-                first = keep_first;
-                angA = keep_angA;
-                angB = keep_angB;
-                lam0 = keep_lam;
-                k0 = keep_pen;
+    bool solved = false;
+    // Crossing safeguard (solve.slang:433-475): rows that the first update
+    // would carry across their surface join the block for a second solve.
+#pragma unroll 1
+    for (uint32_t pass = 0;; ++pass) {
+        float x[6];
+        const bool got = group_solve<L>(blk, lane, active, x);
+        if (pass == 0u || got) {
 #pragma unroll
-                for (int q = 0; q < 6; ++q) dO[q] = keep_dO[q];
-            } else {
-                const uint2 ent = a.entries[e];
-                const uint32_t c = ent.x & 0x7fffffffu;
-                first = (ent.x & kSideFirst) != 0u;
-                const uint32_t other = ent.y & kEntryBody;
-                if (kFlow) load_disp_co(a.disp, other, dO);
-                else load_disp(a.disp, other, dO);
-                axis = a.erec[e];
-                angA = a.erec[3 * a.ecap + e];
-                angB = a.erec[6 * a.ecap + e];
-                lam0 = a.c_lam[c].x;
-                k0 = a.c_pen[c].x;
-            }
-            const float *dA = first ? dI : dO;
-            const float *dB = first ? dO : dI;
-            const float err = row_error(axis.w, axis, angA, angB, dA, dB);
-            const float4 ang = first ? angA : angB;
-            const float row[6] = {first ? -axis.x : axis.x, first ? -axis.y : axis.y,
-                                  first ? -axis.z : axis.z, ang.x, ang.y, ang.z};
-            const float trial = lam0 + k0 * err;
-            if (trial <= 0.0f && trial + k0 * dot6(row, update) > k0 * 1.0e-6f) {
-                add_row(cross_blk, row, k0, trial);
-                crossing = true;
+            for (int q = 0; q < 6; ++q) update[q] = x[q];
+        }
+        if (pass != 0u) break;
+        solved = got;
+        Block cross_blk;
+        block_zero(cross_blk);
+        bool crossing = false;
+        if (solved) {
+            for (uint32_t e = eb + sub_lane; e < ee; e += L) {
+                float row[6], trial = keep_trial, k0 = keep_pen;
+#pragma unroll
+                for (int q = 0; q < 6; ++q) row[q] = keep_row[q];
+                if (e != eb + sub_lane) {
+                    const uint2 ent = a.entries[e];
+                    const uint32_t c = ent.x & 0x7fffffffu;
+                    const bool first = (ent.x & kSideFirst) != 0u;
+                    const uint32_t other = ent.y & kEntryBody;
+                    float dO[6];
+                    if (kFlow && (ent.y & kEntryLower) != 0u) flow_take(a, box, other, dO);
+                    else load_disp(a.disp, other, dO);
+                    const float4 axis = a.erec[e], angA = a.erec[3 * a.ecap + e], angB = a.erec[6 * a.ecap + e];
+                    const float err = row_error(axis.w, axis, angA, angB, first ? dI : dO, first ? dO : dI);
+                    const float4 ang = first ? angA : angB;
+                    row[0] = first ? -axis.x : axis.x;
+                    row[1] = first ? -axis.y : axis.y;
+                    row[2] = first ? -axis.z : axis.z;
+                    row[3] = ang.x;
+                    row[4] = ang.y;
+                    row[5] = ang.z;
+                    k0 = a.c_pen[c].x;
+                    trial = a.c_lam[c].x + k0 * err;
+                }
+                if (trial <= 0.0f && trial + k0 * dot6(row, update) > k0 * 1.0e-6f) {
+                    add_row(cross_blk, row, k0, trial);
+                    crossing = true;
+                }
             }
         }
-    }
-    // Group-wide "any crossing" (uniform across the group's lanes).
-    uint64_t bal = __ballot(crossing);
-    const uint64_t gmask = (L == 64 ? ~0ull : ((1ull << L) - 1ull)) << (grp * L);
-    const bool group_crossing = (bal & gmask) != 0ull;
-    if (bal != 0ull) {
+        const uint64_t bal = __ballot(crossing);
+        if (bal == 0ull) break;
         group_reduce<L>(cross_blk);
-        if (group_crossing && solved) {
+        // Group-wide "any crossing" (uniform across the group's lanes); a
+        // group without one solves its block again unchanged.
+        const uint64_t gmask = (~0ull >> (64 - L)) << (grp * L);
+        if ((bal & gmask) != 0ull) {
 #pragma unroll
             for (int q = 0; q < 21; ++q) blk.h[q] += cross_blk.h[q];
 #pragma unroll
             for (int q = 0; q < 6; ++q) blk.g[q] += cross_blk.g[q];
-            float safe[6];
-            if (block_solve(blk, safe))
-#pragma unroll
-                for (int q = 0; q < 6; ++q) update[q] = safe[q];
         }
     }
-    // The body's displacement after this update (the group's first lane
-    // writes it).
-    float nd[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) nd[q] = dI[q];
-    if (active && sub_lane == 0) {
-        if (solved) {
-            float4 t = a.disp[2 * i], r = a.disp[2 * i + 1];
-            if (phase == 0) {
-                float4 q = a.dq[i];
-                const bool turned = pose_update(t, r, q, update);
-                if (kFlow) {
-                    st4_co(&a.disp[2 * i], t);
-                    if (turned) {
-                        st4_co(&a.dq[i], q);
-                        st4_co(&a.disp[2 * i + 1], r);
-                    }
-                } else {
-                    a.disp[2 * i] = t;
-                    if (turned) {
-                        a.dq[i] = q;
-                        a.disp[2 * i + 1] = r;
-                    }
-                }
-            } else {
-                t.x += update[0]; t.y += update[1]; t.z += update[2];
-                r.x += update[3]; r.y += update[4]; r.z += update[5];
-                if (kFlow) {
-                    st4_co(&a.disp[2 * i], t);
-                    st4_co(&a.disp[2 * i + 1], r);
-                } else {
-                    a.disp[2 * i] = t;
-                    a.disp[2 * i + 1] = r;
-                }
-            }
-            nd[0] = t.x; nd[1] = t.y; nd[2] = t.z; nd[3] = r.x; nd[4] = r.y; nd[5] = r.z;
+    // The body's displacement after this update, in every lane of the group.
+    float4 t = make_float4(dI[0], dI[1], dI[2], 0.0f), r = make_float4(dI[3], dI[4], dI[5], 0.0f);
+    bool turned = false;
+    if (solved) {
+        if (phase == 0) {
+            turned = pose_update(t, r, dq, update);
+        } else {
+            t.x += update[0]; t.y += update[1]; t.z += update[2];
+            r.x += update[3]; r.y += update[4]; r.z += update[5];
+            turned = true;
         }
-        if (kFlow) publish_done(a, i);
+    }
+    const float nd[6] = {t.x, t.y, t.z, r.x, r.y, r.z};
+    if (kFlow && active && sub_lane < kFlowUsed) {
+        // One word per lane: the body's mailbox goes out as one transaction.
+        const uint32_t q = sub_lane;
+        float v = held(dq.w);
+#pragma unroll
+        for (uint32_t w = 0; w < 6; ++w) v = q == w ? held(nd[w]) : v;
+        __hip_atomic_store(&a.flow[size_t(i) * kFlowWords + q],
+                           (unsigned long long)(__float_as_uint(v)) | ((unsigned long long)(a.flow_stamp) << 32),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if constexpr (kFlow && L >= 16) __builtin_amdgcn_s_setprio(0);
+    if (solved && sub_lane == 0) {
+        a.disp[2 * i] = t;
+        if (turned) {
+            a.disp[2 * i + 1] = r;
+            if (phase == 0) a.dq[i] = dq;
+        }
     }
     if (kFlow) {
         // This update's duals (advance_duals) of the points whose other end
-        // is solved before this body in the sweep (a lower colour) or not in
-        // it (not dynamic, or not an impact body in the velocity phase):
-        // both ends' displacements are final here, and the points' duals are
-        // read again only by the next update's launch.  Every point has one
-        // such end, so each is updated once, as the separate dual pass did.
-#pragma unroll
-        for (int q = 0; q < 6; ++q) nd[q] = __shfl(nd[q], int(grp * L), 64);
+        // is solved before this body in the sweep (a lower colour) or never
+        // (not dynamic): both ends' displacements are final here, and the
+        // points' duals are read again only by the next update's launch.
+        // Every point has one such end, so each is updated once.
         const bool last = a.tol <= 0.0f && it + 1u == a.budget;
         ResidualAcc residual;
         if (active) {
             for (uint32_t e = eb + sub_lane; e < ee; e += L) {
                 const uint2 ent = a.entries[e];
+                const bool lower = (ent.y & kEntryLower) != 0u;
+                if (!lower && (ent.y & kEntryFixed) == 0u) continue;
                 const uint32_t other = ent.y & kEntryBody;
-                const bool other_solved = a.P[other].motion == kDynamic && (phase == 0 || a.impact[other] != 0u);
-                if (other_solved && (ent.y & kEntryLower) == 0u) continue;
                 const uint32_t c = ent.x & 0x7fffffffu;
                 const bool first = (ent.x & kSideFirst) != 0u;
                 float dO[6];
-                load_disp_co(a.disp, other, dO);
+                if (e == eb + sub_lane) {
+#pragma unroll
+                    for (int q = 0; q < 6; ++q) dO[q] = keep_dO[q];
+                } else if (lower) {
+                    flow_take(a, box, other, dO);
+                } else {
+                    load_disp(a.disp, other, dO);
+                }
                 float4 Jx[9];
 #pragma unroll
                 for (int q = 0; q < 9; ++q) Jx[q] = a.erec[q * a.ecap + e];
-                dual_point(a, c, phase, first ? nd : dO, first ? dO : nd, Jx, last, residual);
+                const DualStep s = dual_point(a, c, first ? nd : dO, first ? dO : nd, Jx, residual);
+                if (last) {
+                    const float wO = s.stick || phase != 0 ? 1.0f : lower ? flow_take_w(a, box, other) : a.dq[other].w;
+                    publish_flow(a, c, phase, first ? i : other, first ? other : i, s, first ? nd : dO,
+                                 first ? dq.w : wO, first ? dO : nd, first ? wO : dq.w, v3(Jx[1]), v3(Jx[2]));
+                } else if (a.tol > 0.0f) {
+                    a.c_flags[c] = (a.c_flags[c] & ~kFlagSlipping) | (s.stick ? 0u : kFlagSlipping);
+                }
             }
         }
         if (it < kResidualSlots) residual_commit(a.log, phase * kResidualSlots + it, residual);
@@ -1353,16 +1518,22 @@ __device__ void solve_color(const SolveArgs &a, uint32_t begin, uint32_t end, ui
         solve_group<L, kJoints, false>(a, base, end, phase);
 }
 
-__device__ __forceinline__ PmhRigidBodyState avbd_pose(const SolveArgs &a, uint32_t i) {
+// The pose of body i with displacement d and rotation delta q.
+__device__ __forceinline__ PmhRigidBodyState pose_with(const SolveArgs &a, uint32_t i, V3 d, Q dq) {
     PmhRigidBodyState s;
-    const V3 t = v3(a.tpos[i]);
-    const float4 d = a.flow_stamp ? ld4_co(&a.disp[2 * i]) : a.disp[2 * i];
-    s.position = pv(add(t, {d.x, d.y, d.z}));
+    s.position = pv(add(v3(a.tpos[i]), d));
     Q o = q4(a.tq[i]);
-    const Q dq = q4(a.flow_stamp ? ld4_co(&a.dq[i]) : a.dq[i]);
     if (dq.x != 0.0f || dq.y != 0.0f || dq.z != 0.0f) o = qnormalize(qmul(dq, o));
     s.orientation = pq(o);
     return s;
+}
+__device__ __forceinline__ PmhRigidBodyState avbd_pose(const SolveArgs &a, uint32_t i) {
+    return pose_with(a, i, v3(a.disp[2 * i]), q4(a.dq[i]));
+}
+// Pose phase: the displacement's rotation part is twice the delta's vector
+// part (exactly: pose_update doubles it), so six floats and w are a pose.
+__device__ __forceinline__ PmhRigidBodyState pose_from(const SolveArgs &a, uint32_t i, const float *d, float w) {
+    return pose_with(a, i, {d[0], d[1], d[2]}, {0.5f * d[3], 0.5f * d[4], 0.5f * d[5], w});
 }
 
 // ---------------------------------------------------------------------
@@ -1372,6 +1543,20 @@ __device__ __forceinline__ PmhRigidBodyState avbd_pose(const SolveArgs &a, uint3
 // dual update, the velocity-phase rows).  Same operations and order as the
 // reference.
 // ---------------------------------------------------------------------
+// Both ends of a joint as a visit sees them: displacements and the rotation
+// deltas' w.
+struct JointEnds {
+    float da[6], db[6], wa, wb;
+};
+__device__ __forceinline__ JointEnds joint_ends(const SolveArgs &a, uint32_t ia, uint32_t ib) {
+    JointEnds e;
+    load_disp(a.disp, ia, e.da);
+    load_disp(a.disp, ib, e.db);
+    e.wa = a.dq[ia].w;
+    e.wb = a.dq[ib].w;
+    return e;
+}
+
 enum : uint32_t { kVisitInitialize = 0, kVisitAccumulate = 1, kVisitAdvance = 2, kVisitImpact = 3 };
 constexpr float kLimitStabilization = 0.8f;
 
@@ -1440,14 +1625,13 @@ __device__ __forceinline__ void set6(float *d, V3 l, V3 r) {
 
 // rigid_avbd_visit_joint_row, :626-713.
 __device__ void visit_joint_row(const SolveArgs &a, PmhRigidConstraint &j, Block &blk, uint32_t &index,
-                                float &impulse, bool first, const JointRowArgs &r, uint32_t visit) {
+                                float &impulse, bool first, const JointRowArgs &r, uint32_t visit,
+                                const JointEnds &ends) {
     if (index >= 18u) return;
     const uint32_t ri = index++;
     PmhAvbdRow row = j.rows[ri];
     const uint32_t ia = j.dense_a, ib = j.dense_b;
-    float da[6], db[6];
-    load_disp_a(a, ia, da);
-    load_disp_a(a, ib, db);
+    const float *da = ends.da, *db = ends.db;
     const float linearized = dot6(r.ja, da) + dot6(r.jb, db);
 #pragma unroll
     for (int k = 0; k < 6; ++k) { row.a[k] = r.ja[k]; row.b[k] = r.jb[k]; }
@@ -1499,12 +1683,12 @@ __device__ void visit_joint_row(const SolveArgs &a, PmhRigidConstraint &j, Block
 
 // rigid_avbd_visit_joint, :715-926.
 __device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstraint &j, Block &blk, bool first,
-                                          uint32_t visit) {
+                                          uint32_t visit, const JointEnds &ends) {
     uint32_t index = 0;
     float impulse = 0.0f;
     const PmhRigidConstraintOptions &o = j.options;
     const uint32_t ia = j.dense_a, ib = j.dense_b;
-    const PmhRigidBodyState sa = avbd_pose(a, ia), sb = avbd_pose(a, ib);
+    const PmhRigidBodyState sa = pose_from(a, ia, ends.da, ends.wa), sb = pose_from(a, ib, ends.db, ends.wb);
     const PmhRigidBodyState pa = a.prev[ia], pb = a.prev[ib];
     const Q qa = sq(sa.orientation), qb = sq(sb.orientation);
     const V3 armA = rotate(qa, sv(o.local_anchor_a)), armB = rotate(qb, sv(o.local_anchor_b));
@@ -1576,7 +1760,7 @@ __device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstra
                 r.current = current; r.previous = old_current; r.penalty = lock_penalty;
                 r.stiffness = kMaxPenalty; r.damping = 0.0f; r.lower = -kMaxPenalty; r.upper = kMaxPenalty;
                 r.stabilization = kAlpha;
-                visit_joint_row(a, j, blk, index, impulse, first, r, visit);
+                visit_joint_row(a, j, blk, index, impulse, first, r, visit, ends);
             }
             const bool free_limit = angular ? (type == kJointHinge && axis == 2u) || (type == kJointPiston && axis == 0u)
                                             : (type == kJointSlider || type == kJointPiston) && axis == 0u;
@@ -1599,15 +1783,15 @@ __device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstra
                     l.current = limit_current - lower; l.previous = old_limit_current - lower;
                     l.penalty = equal_penalty; l.lower = -kMaxPenalty; l.upper = kMaxPenalty;
                     l.stabilization = kAlpha;
-                    visit_joint_row(a, j, blk, index, impulse, first, l, visit);
+                    visit_joint_row(a, j, blk, index, impulse, first, l, visit, ends);
                 } else if (lower < upper) {
                     l.current = limit_current - upper; l.previous = smax(old_limit_current - upper, 0.0f);
                     l.penalty = penalty; l.lower = 0.0f; l.upper = kMaxPenalty;
                     l.stabilization = kLimitStabilization;
-                    visit_joint_row(a, j, blk, index, impulse, first, l, visit);
+                    visit_joint_row(a, j, blk, index, impulse, first, l, visit, ends);
                     l.current = limit_current - lower; l.previous = smin(old_limit_current - lower, 0.0f);
                     l.lower = -kMaxPenalty; l.upper = 0.0f;
-                    visit_joint_row(a, j, blk, index, impulse, first, l, visit);
+                    visit_joint_row(a, j, blk, index, impulse, first, l, visit, ends);
                 }
             }
             if (type == kJointGenericSpring && (springs.axes & (1u << axis)) != 0u) {
@@ -1615,7 +1799,7 @@ __device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstra
                 sr.current = current; sr.previous = old_current; sr.penalty = penalty;
                 sr.stiffness = comp(sv(springs.stiffness), axis); sr.damping = comp(sv(springs.damping), axis);
                 sr.lower = -kMaxPenalty; sr.upper = kMaxPenalty; sr.stabilization = kAlpha;
-                visit_joint_row(a, j, blk, index, impulse, first, sr, visit);
+                visit_joint_row(a, j, blk, index, impulse, first, sr, visit, ends);
             }
             if (motor_type && axis == 0u && (angular ? o.motor.angular_enabled != 0u : o.motor.linear_enabled != 0u)) {
                 const float speed = angular ? o.motor.angular_target_velocity : o.motor.linear_target_velocity;
@@ -1634,7 +1818,7 @@ __device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstra
                 mr.current = travel - speed * a.dt; mr.previous = 0.0f; mr.penalty = penalty;
                 mr.stiffness = kMaxPenalty; mr.damping = 0.0f; mr.lower = -bound; mr.upper = bound;
                 mr.motor = true; mr.motor_speed = speed; mr.stabilization = kAlpha;
-                visit_joint_row(a, j, blk, index, impulse, first, mr, visit);
+                visit_joint_row(a, j, blk, index, impulse, first, mr, visit, ends);
             }
         }
     }
@@ -1648,28 +1832,43 @@ __device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstra
 // The body's enabled joints are dealt round-robin over the L lanes of its
 // group (the k-th enabled joint of the list to lane k mod L) and added to
 // that lane's partial block before the group reduction.
-__device__ void body_joint_rows(const SolveArgs &a, uint32_t i, uint32_t phase, Block &blk, uint32_t sub_lane,
-                                uint32_t L) {
+// The body's own displacement and rotation delta come in registers, the
+// other end's from its mailbox where this sweep has moved it already.
+template <bool kFlow>
+__device__ __forceinline__ void body_joint_rows(const SolveArgs &a, uint32_t i, uint32_t phase, Block &blk,
+                                                uint32_t sub_lane, uint32_t L, const float *dI, float wI) {
     uint32_t pos = 0;
     for (uint32_t e = a.jstart[i]; e < a.jstart[i + 1]; ++e) {
         PmhRigidConstraint &j = a.joints[a.jadj[e]];
         if (j.state_enabled == 0u) continue;
         if (pos++ % L != sub_lane) continue;
         const bool first = i == j.dense_a;
-        if (a.flow_stamp) {
-            const uint32_t other = first ? j.dense_b : j.dense_a;
-            if (a.color[other] < a.color[i] && (phase == 0u || a.impact[other] != 0u)) wait_published(a, other);
+        const uint32_t other = first ? j.dense_b : j.dense_a;
+        float dO[6], wO = 1.0f;
+        // Bodies without a colour hold kInvalid: never lower.
+        if (kFlow && a.color[other] < a.color[i]) {
+            const __amdgpu_buffer_rsrc_t box = flow_box(a);
+            flow_take(a, box, other, dO);
+            if (phase == 0u) wO = flow_take_w(a, box, other);
+        } else {
+            load_disp(a.disp, other, dO);
+            if (phase == 0u) wO = a.dq[other].w;
         }
+        JointEnds ends;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+            ends.da[q] = first ? dI[q] : dO[q];
+            ends.db[q] = first ? dO[q] : dI[q];
+        }
+        ends.wa = first ? wI : wO;
+        ends.wb = first ? wO : wI;
         if (phase == 0u) {
-            visit_joint(a, j, blk, first, kVisitAccumulate);
+            visit_joint(a, j, blk, first, kVisitAccumulate, ends);
             continue;
         }
-        float da[6], db[6];
-        load_disp_a(a, j.dense_a, da);
-        load_disp_a(a, j.dense_b, db);
         for (uint32_t r = 0; r < j.avbd_count; ++r) {
             const PmhAvbdRow row = j.rows[r];
-            if (row.stiffness >= kMaxPenalty) jrow_accumulate(blk, row, first, da, db, a.dt);
+            if (row.stiffness >= kMaxPenalty) jrow_accumulate(blk, row, first, ends.da, ends.db, a.dt);
         }
     }
 }
@@ -1685,7 +1884,7 @@ __device__ void advance_joint(const SolveArgs &a, uint32_t k, uint32_t phase) {
     if (phase == 0u) {
         Block scratch;
         block_zero(scratch);
-        impulse = visit_joint(a, j, scratch, true, kVisitAdvance);
+        impulse = visit_joint(a, j, scratch, true, kVisitAdvance, joint_ends(a, ia, ib));
     } else {
         float da[6], db[6];
         load_disp(a.disp, ia, da);
@@ -1722,33 +1921,47 @@ __device__ float joint_residual(const SolveArgs &a, const PmhRigidConstraint &j)
     return r;
 }
 
-// Point flag: the point slid at the last dual update (to-residual mode,
+// kFlagSlipping: the point slid at the last dual update (to-residual mode,
 // where the impulses are published after the loop).
-constexpr uint32_t kFlagSlipping = 4u;
 
-// The impulses of the last dual update and the re-anchoring of a sliding
-// contact (solve.slang:540-562).
-__device__ void publish_point(const SolveArgs &a, uint32_t c, uint32_t phase, uint2 p, float fn, float ft0,
-                              float ft1, bool stick, V3 t0, V3 t1) {
+// The impulses of the last dual update (solve.slang:540-562).
+__device__ __forceinline__ void publish_impulse(const SolveArgs &a, uint32_t c, float fn, float ft0, float ft1, V3 t0,
+                                                V3 t1) {
     const float an = fn * a.dt;
     const V3 af = mul(add(mul(t0, ft0), mul(t1, ft1)), a.dt);
     a.c_acc[c] = make_float4(an, af.x, af.y, af.z);
     a.c_rep[c] = make_float4(an, af.x, af.y, af.z);
-    if (!stick) {
-        PmhRigidBodyState pa, pb;
-        if (phase != 0) {
-            pa.position = pv(v3(a.tpos[p.x])); pa.orientation = pq(q4(a.tq[p.x]));
-            pb.position = pv(v3(a.tpos[p.y])); pb.orientation = pq(q4(a.tq[p.y]));
-        } else {
-            pa = avbd_pose(a, p.x);
-            pb = avbd_pose(a, p.y);
-        }
-        const V3 point = v3(a.c_pt[c]);
-        const V3 na = inv_rotate(sq(pa.orientation), sub(point, sv(pa.position)));
-        const V3 nb = inv_rotate(sq(pb.orientation), sub(point, sv(pb.position)));
-        a.c_aa[c] = f4(na, a.c_aa[c].w);
-        a.c_ab[c] = f4(nb, 0.0f);
-    }
+}
+// The re-anchoring of a sliding contact at the ends' poses.
+__device__ __forceinline__ void publish_anchors(const SolveArgs &a, uint32_t c, const PmhRigidBodyState &pa,
+                                                const PmhRigidBodyState &pb) {
+    const V3 point = v3(a.c_pt[c]);
+    const V3 na = inv_rotate(sq(pa.orientation), sub(point, sv(pa.position)));
+    const V3 nb = inv_rotate(sq(pb.orientation), sub(point, sv(pb.position)));
+    a.c_aa[c] = f4(na, a.c_aa[c].w);
+    a.c_ab[c] = f4(nb, 0.0f);
+}
+// The target pose, which the velocity phase anchors at.
+__device__ __forceinline__ PmhRigidBodyState target_pose(const SolveArgs &a, uint32_t i) {
+    PmhRigidBodyState s;
+    s.position = pv(v3(a.tpos[i]));
+    s.orientation = pq(q4(a.tq[i]));
+    return s;
+}
+__device__ void publish_point(const SolveArgs &a, uint32_t c, uint32_t phase, uint2 p, float fn, float ft0,
+                              float ft1, bool stick, V3 t0, V3 t1) {
+    publish_impulse(a, c, fn, ft0, ft1, t0, t1);
+    if (stick) return;
+    if (phase != 0) publish_anchors(a, c, target_pose(a, p.x), target_pose(a, p.y));
+    else publish_anchors(a, c, avbd_pose(a, p.x), avbd_pose(a, p.y));
+}
+// The same inside a dataflow sweep, with the ends' displacements in hand.
+__device__ void publish_flow(const SolveArgs &a, uint32_t c, uint32_t phase, uint32_t ia, uint32_t ib,
+                             const DualStep &s, const float *dA, float wA, const float *dB, float wB, V3 t0, V3 t1) {
+    publish_impulse(a, c, s.f.n, s.f.t0, s.f.t1, t0, t1);
+    if (s.stick) return;
+    if (phase != 0) publish_anchors(a, c, target_pose(a, ia), target_pose(a, ib));
+    else publish_anchors(a, c, pose_from(a, ia, dA, wA), pose_from(a, ib, dB, wB));
 }
 
 // Constraint residual of a contact point (no reference counterpart): an
@@ -1760,8 +1973,8 @@ __device__ __forceinline__ float contact_residual(const float *err, float fn, bo
     return r;
 }
 
-__device__ void dual_point(const SolveArgs &a, uint32_t c, uint32_t phase, const float *dA, const float *dB,
-                           const float4 *Jx, bool last, ResidualAcc &residual) {
+__device__ DualStep dual_point(const SolveArgs &a, uint32_t c, const float *dA, const float *dB, const float4 *Jx,
+                               ResidualAcc &residual) {
     float4 lam = a.c_lam[c], pen = a.c_pen[c];
     const float err[3] = {row_error(Jx[0].w, Jx[0], Jx[3], Jx[6], dA, dB),
                           row_error(Jx[1].w, Jx[1], Jx[4], Jx[7], dA, dB),
@@ -1782,8 +1995,7 @@ __device__ void dual_point(const SolveArgs &a, uint32_t c, uint32_t phase, const
     a.c_lam[c] = lam;
     a.c_pen[c] = pen;
     residual.add(contact_residual(err, f.n, stick));
-    if (last) publish_point(a, c, phase, a.ab[a.c_pair[c]], f.n, f.t0, f.t1, stick, v3(Jx[1]), v3(Jx[2]));
-    else if (a.tol > 0.0f) a.c_flags[c] = (a.c_flags[c] & ~kFlagSlipping) | (stick ? 0u : kFlagSlipping);
+    return {f, stick};
 }
 
 // advance_duals for contacts (solve.slang:492-566): one thread per point.
@@ -1801,7 +2013,9 @@ __device__ void advance_duals(const SolveArgs &a, uint32_t phase, uint32_t itera
         float4 Jx[9];
 #pragma unroll
         for (int q = 0; q < 9; ++q) Jx[q] = J[q];
-        dual_point(a, c, phase, dA, dB, Jx, last, residual);
+        const DualStep s = dual_point(a, c, dA, dB, Jx, residual);
+        if (last) publish_point(a, c, phase, p, s.f.n, s.f.t0, s.f.t1, s.stick, v3(Jx[1]), v3(Jx[2]));
+        else if (a.tol > 0.0f) a.c_flags[c] = (a.c_flags[c] & ~kFlagSlipping) | (s.stick ? 0u : kFlagSlipping);
     }
     if (iteration < kResidualSlots) residual_commit(a.log, phase * kResidualSlots + iteration, residual);
 }
@@ -2068,38 +2282,68 @@ __global__ void __launch_bounds__(256) k_stage_color(SolveArgs a, uint32_t begin
 // tickets of one block's worth of wavefront slots (each slot one
 // wavefront's worth of colour-ordered positions; a colour starts at a slot
 // boundary, so a wavefront holds one colour), in order, one atomic per
-// block.  A body waits only for lower-colour neighbours: their positions
-// were ticketed earlier, to blocks that are running, so every wait ends
+// block; the block's wavefronts draw the ticket's slots from LDS one by one,
+// so none waits for the slowest of the last ticket.  A body waits only for
+// lower-colour neighbours: their positions were ticketed earlier, and the
+// lowest slot not done is always in a running wavefront's hands (a block
+// takes a ticket only when its last one is given out), so every wait ends
 // (and each is bounded besides).  Colour c + 1 starts wherever colour c is
 // done, not after all of colour c.
+//
+// What bounds it is the chain over the colours: per colour one body's wait,
+// rows, reduction, solve, safeguard, pose and mailbox, about 6 us of which
+// 2 us are the store and the load through memory.  Measured on a heap of 1000
+// bodies (9 colours): 98 us per sweep with a flag per body behind the stored
+// displacement (a completed store, a flag store, a poll and a load per
+// colour), LDS shuffles and every lane solving the whole block; 62 us with
+// stamped mailboxes, DPP sums and the solve spread over the lanes.  32768
+// bodies: 144 -> 113 us (wavefronts' lifetimes, four per SIMD, count there).
 constexpr uint32_t kSweepWaves = 8;          // wavefronts per block without joints (512 threads)
 constexpr uint32_t kSweepJointWaves = 4;     // with joints (more registers per lane)
 // Without joints the sweep is held to 128 VGPRs (four wavefronts per SIMD,
-// two blocks per CU): at 137 only one block fit per CU, and twice the
-// bodies in flight cut the sweep from 175 to 149 µs on the settled pile
-// for 4 spilled registers.
+// two blocks per CU).
 template <int L, bool kJoints>
 __global__ void __launch_bounds__(64 * (kJoints ? kSweepJointWaves : kSweepWaves), kJoints ? 1 : 4)
 k_sweep(SolveArgs a, uint32_t phase, uint32_t it) {
-    __shared__ uint32_t s_ticket[2];
+    __shared__ unsigned long long s_draw;    // the block's ticket, slots of it given out
     uint32_t *tickets = a.ctr->sweep_ticket;
     // The other counter is the next sweep's: it starts at zero.
     if (blockIdx.x == 0 && threadIdx.x == 0) st_relaxed(&tickets[(a.flow_stamp + 1u) & 1u], 0u);
     if (a.tol > 0.0f && a.log->executed[phase] != 0u) return;   // converged earlier
     constexpr uint32_t groups = 64 / L;
     constexpr uint32_t waves = kJoints ? kSweepJointWaves : kSweepWaves;
-    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63;
     const uint32_t end = a.color_start[a.ctr->colors];
     const uint32_t wave_slots = (end + groups - 1) / groups;
     uint32_t *ticket = &tickets[a.flow_stamp & 1u];
-    for (uint32_t round = 0;; ++round) {
-        // Double-buffered: the slot written in round r + 1 was last read
-        // before every wavefront passed round r's barrier.
-        if (threadIdx.x == 0) s_ticket[round & 1u] = atomicAdd(ticket, 1u);
-        __syncthreads();
-        const uint32_t first = s_ticket[round & 1u] * waves;
-        if (first >= wave_slots) break;      // the same for the whole block
-        if (first + wave < wave_slots) solve_group<L, kJoints, true>(a, (first + wave) * groups, end, phase, it);
+    if (threadIdx.x == 0) s_draw = (unsigned long long)(atomicAdd(ticket, 1u)) << 32;
+    __syncthreads();
+    for (;;) {
+        uint32_t slot = 0;
+        if (lane == 0) {
+            for (;;) {
+                const unsigned long long d = atomicAdd(&s_draw, 1ull);
+                const uint32_t first = uint32_t(d >> 32) * waves, taken = uint32_t(d);
+                if (first >= wave_slots) {           // nothing left for any block
+                    slot = wave_slots;
+                    break;
+                }
+                if (taken < waves) {
+                    slot = first + taken;
+                    // The last slot's taker fetches the next ticket.
+                    if (taken + 1u == waves) atomicExch(&s_draw, (unsigned long long)(atomicAdd(ticket, 1u)) << 32);
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+        slot = __builtin_amdgcn_readfirstlane(slot);
+        if (slot >= wave_slots) {
+            // The tail of the last ticket, or no ticket left: later draws
+            // lie further on still.
+            break;
+        }
+        solve_group<L, kJoints, true>(a, slot * groups, end, phase, it);
     }
 }
 template <bool kJoints>
@@ -2180,7 +2424,7 @@ __global__ void k_stage_velocity_errors(SolveArgs a, const uint32_t *c_flags) {
         if (a.impact[j.dense_a] == 0u && a.impact[j.dense_b] == 0u) continue;
         Block scratch;
         block_zero(scratch);
-        visit_joint(a, j, scratch, true, kVisitImpact);
+        visit_joint(a, j, scratch, true, kVisitImpact, joint_ends(a, j.dense_a, j.dense_b));
     }
 }
 __global__ void k_stage_velocity_jacobians(SolveArgs a) {
@@ -2283,7 +2527,7 @@ __global__ void k_joint_init(SolveArgs a) {
     if (j.dense_a == kInvalid || j.dense_b == kInvalid) return;
     Block scratch;
     block_zero(scratch);
-    visit_joint(a, j, scratch, true, kVisitInitialize);
+    visit_joint(a, j, scratch, true, kVisitInitialize, joint_ends(a, j.dense_a, j.dense_b));
 }
 
 // The joints' iteration floor: the legacy profile without a requested
@@ -2626,7 +2870,7 @@ PmhResult Solver::each_buffer(uint32_t bodies, uint32_t pairs, uint32_t points, 
     R(color_bodies, positions); R(bp_start, positions + 1); R(anchored, bodies); R(mean, bodies);
     R(members, bodies); R(mean_list, bodies);
     R(jdeg, bodies + 1); R(jstart, bodies + 1); R(jcursor, bodies); R(joint_head, bodies);
-    R(prev_vel, bodies); R(done, bodies);
+    R(prev_vel, bodies); R(flow, kFlowWords * (size_t)bodies);
     R(code, pairs); R(ab, pairs); R(m_count, pairs + 1); R(m_start, pairs + 1); R(m_slot, pairs + 1);
     R(m_impact, pairs); R(m_face, pairs); R(m_init_rel, pairs); R(adj, 2 * (size_t)pairs);
     R(tri_list, pairs); R(face_list, pairs);
@@ -2641,14 +2885,14 @@ PmhResult Solver::each_buffer(uint32_t bodies, uint32_t pairs, uint32_t points, 
 }
 
 PmhResult Solver::reserve(uint32_t bodies, uint32_t pairs, uint32_t points) {
-    // Zeroed when first allocated: the velocity history, the published
-    // sweep stamps, the counters and the running totals.
-    const bool fresh_prev = prev_vel.n < bodies, fresh_done = done.n < bodies;
+    // Zeroed when first allocated: the velocity history, the sweep's
+    // mailboxes, the counters and the running totals.
+    const bool fresh_prev = prev_vel.n < bodies, fresh_flow = flow.n < kFlowWords * (size_t)bodies;
     const bool fresh_ctr = !counters.p, fresh_totals = !totals.p;
     PmhResult r = each_buffer(bodies, pairs, points, [](auto &buf, size_t count) { return buf.reserve(count); });
     if (r != PMH_SUCCESS) return r;
     if (fresh_prev) PMH_CHECK(hipMemset(prev_vel.p, 0, sizeof(float4) * bodies));
-    if (fresh_done) PMH_CHECK(hipMemset(done.p, 0, sizeof(uint32_t) * bodies));
+    if (fresh_flow) PMH_CHECK(hipMemset(flow.p, 0, sizeof(unsigned long long) * kFlowWords * bodies));
     if (fresh_ctr) PMH_CHECK(hipMemset(counters.p, 0, sizeof(StepCounters)));
     if (fresh_totals) PMH_CHECK(hipMemset(totals.p, 0, sizeof(SolveTotals)));
     ecap = 2 * (size_t)points;
@@ -2713,7 +2957,7 @@ void Solver::release() {
     tpos.release(); tq.release(); tv.release(); tw.release(); disp.release(); dq.release();
     inertia.release(); prev_vel.release(); color.release(); parent.release(); impact.release();
     deg.release(); adj_start.release(); adj_cursor.release(); color_bodies.release();
-    bp_start.release(); anchored.release(); mean.release(); members.release(); mean_list.release(); done.release();
+    bp_start.release(); anchored.release(); mean.release(); members.release(); mean_list.release(); flow.release();
     jdeg.release(); jstart.release(); jcursor.release(); joint_head.release(); jadj.release(); code.release(); ab.release();
     m_count.release(); m_start.release(); m_slot.release(); m_impact.release(); m_face.release();
     m_init_rel.release(); adj.release(); tri_list.release(); face_list.release(); c_np.release(); c_pt.release(); c_aa.release();
@@ -2800,7 +3044,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
     a.jadj = v.jadj.p;
     a.prev = previous;
     a.color = v.color.p;
-    a.done = v.done.p;
+    a.flow = v.flow.p;
     a.flow_stamp = 0;
     a.flow_limit = sp.sweep_wait_limit;
     a.log = v.residual.p;
@@ -3055,7 +3299,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
                 if (flow) {
                     SolveArgs af = a;
                     if (++v.sweep_stamp == 0u) {   // stamps wrapped: no stale stamp may match
-                        PMH_CHECK(hipMemsetAsync(v.done.p, 0, sizeof(uint32_t) * n, s));
+                        PMH_CHECK(hipMemsetAsync(v.flow.p, 0, sizeof(unsigned long long) * kFlowWords * n, s));
                         v.sweep_stamp = 1u;
                     }
                     af.flow_stamp = v.sweep_stamp;

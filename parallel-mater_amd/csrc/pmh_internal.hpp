@@ -116,6 +116,8 @@ struct SolveTotals {
     double algorithmic_bytes;
 };
 
+constexpr uint32_t kMaxBodies = 0x3fffffffu;   // body indices leave two bits of a word for flags
+constexpr uint32_t kFlowWords = 8;             // 64-bit mailbox words per body of the dataflow sweep
 constexpr uint32_t kMaxColors = 256;
 // A body the colouring gave up on (a wait ran out) holds this value: not a
 // colour, so no solve stage sees it, and published, so nobody waits on it.
@@ -279,10 +281,11 @@ struct Solver {
     DBuf<uint32_t> color_count, color_start;
     // Dataflow sweep: each colour's positions start at a multiple of the
     // bodies per wavefront (64 / lanes), the gaps holding kInvalid, so one
-    // wavefront never holds two colours; `done[i]` is the stamp of the last
-    // sweep that published body i's displacement.
+    // wavefront never holds two colours; `flow` holds each body's mailbox
+    // (kFlowWords words: the displacement it last published, each float with
+    // the stamp of its sweep).
     uint32_t slots = 0;                  // colour-ordered positions (bodies plus padding)
-    DBuf<uint32_t> done;
+    DBuf<unsigned long long> flow;
     uint32_t sweep_stamp = 0;
     DBuf<StepCounters> counters;
     DBuf<SolveTotals> totals;

@@ -394,9 +394,9 @@ extern "C" PmhResult pmhPrepareSolveGeometryConstraintsNoAlloc(
         PmhResult r = g.solver.carve(g.base, kStaticScratchBytes, kStaticBodies, kStaticPairs, kStaticPoints,
                                      &g.host_counters, g.host_starts);
         if (r != PMH_SUCCESS) return r;
-        // The published sweep stamps start below every stamp to come.
-        k_seam_clear<<<std::max<uint32_t>(1, (kStaticBodies + 255) / 256), 256, 0, s>>>(g.solver.done.p,
-                                                                                      kStaticBodies);
+        // The mailboxes' stamps start below every stamp to come.
+        k_seam_clear<<<kStaticBodies / 16, 256, 0, s>>>(reinterpret_cast<uint32_t *>(g.solver.flow.p),
+                                                        kStaticBodies * kFlowWords * 2u);
         g.ready = true;
     }
     uint32_t M = 0;

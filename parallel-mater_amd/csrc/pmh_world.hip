@@ -345,7 +345,7 @@ PmhResult World::ensure_device() {
     }
     if (bodies_dirty) {
         const uint32_t n = body_count;
-        if (n > 0x7fffffffu) return PMH_ERROR_CAPACITY_EXCEEDED;
+        if (n > kMaxBodies) return PMH_ERROR_CAPACITY_EXCEEDED;
         // Per-body candidate lists hold up to pairs_per_body entries; the
         // pair and point pools are sized by their realistic totals.
         const uint32_t pair_cap = std::max<uint32_t>(256, n * pairs_per_body);
