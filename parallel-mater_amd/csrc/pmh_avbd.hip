@@ -500,10 +500,14 @@ __global__ void k_uf_hook(const uint32_t *npairs, const PmhBodyParameters *P, co
     }
 }
 
+// Points every body at its root.  No hook runs meanwhile, so the walk's root
+// is final; the walk writes nothing on its way (a halving store could land
+// after the passed body's own, and leave it short of its root).
 __global__ void k_uf_compress(uint32_t n, uint32_t *parent) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    uint32_t r = uf_find(parent, i);
+    uint32_t r = i;
+    for (uint32_t p = ld_parent(&parent[r]); p != r; p = ld_parent(&parent[r])) r = p;
     st_relaxed(&parent[i], r);
 }
 
