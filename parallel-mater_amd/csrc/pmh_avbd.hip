@@ -19,6 +19,7 @@
 // then solved in registers by an unrolled LDL^T.  Per-point Jacobians are
 // computed once per phase (they only depend on the target poses).
 #include "pmh_internal.hpp"
+#include "pmh_lanes.hpp"
 #include "pmh_warmstart.hpp"
 
 #include <hip/hip_cooperative_groups.h>
@@ -56,20 +57,6 @@ __device__ __forceinline__ void st_relaxed(uint32_t *p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A lane exchange inside the wavefront as an operand modifier (DPP): the add
-// or multiply that uses it takes no extra instruction, where __shfl goes
-// through the LDS pipe (ds_bpermute).  Every lane must be active.
-enum : int { kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140, kDppRowShr = 0x110,
-             kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143, kDppNewBcast = 0x150 };
-template <int kCtrl>
-__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
-    return uint32_t(__builtin_amdgcn_update_dpp(0, int(x), kCtrl, 0xf, 0xf, true));
-}
-template <int kCtrl>
-__device__ __forceinline__ float dpp_f32(float x) { return __uint_as_float(dpp_u32<kCtrl>(__float_as_uint(x))); }
-// The value of lane kLane of each 16-lane row.
-template <int kLane>
-__device__ __forceinline__ float row_bcast(float x) { return dpp_f32<kDppNewBcast + kLane>(x); }
 // The value of the odd row of each pair of rows, in both.
 __device__ __forceinline__ float odd_row(float x) {
     return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);

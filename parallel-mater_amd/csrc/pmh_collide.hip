@@ -21,6 +21,7 @@
 // triangle-pair path (leaf-pair candidates or BVH traversal) in a second
 // kernel over a compact list of those pairs.
 #include "pmh_internal.hpp"
+#include "pmh_lanes.hpp"
 #include "pmh_world.hpp"
 
 #include <algorithm>
@@ -1612,13 +1613,12 @@ __device__ __forceinline__ uint32_t wave_reserve(uint32_t *counter, uint32_t cou
 // (:2855-2862).  Point flags: 2 persistent, 8 guided (the solver's rest
 // offset).
 constexpr uint32_t kPointGuided = 8u;
-__device__ void emit_manifold(const NarrowOut &o, uint32_t m, Manifold &man, const PmhRigidBodyState &A,
-                              const PmhRigidBodyState &B, bool persistent_shapes, const HingeFrame &ha,
-                              const HingeFrame &hb) {
+__device__ __forceinline__ void write_manifold(const NarrowOut &o, uint32_t m, Manifold &man, uint32_t start,
+                                               const PmhRigidBodyState &A, const PmhRigidBodyState &B,
+                                               bool persistent_shapes, const HingeFrame &ha, const HingeFrame &hb) {
     const bool guided = guided_pair(ha, hb);
     const bool persistent = guided || (persistent_shapes && ha.present == 0u && hb.present == 0u &&
                                        ha.fixed_member == 0u && hb.fixed_member == 0u);
-    uint32_t start = wave_reserve(&o.ctr->point_alloc, man.count);
     if (man.count) {
         if (start + man.count > o.point_cap) {
             atomicOr(&o.ctr->status, kStatusPointOverflow);
@@ -1648,9 +1648,346 @@ __device__ void emit_manifold(const NarrowOut &o, uint32_t m, Manifold &man, con
     }
 }
 
+__device__ void emit_manifold(const NarrowOut &o, uint32_t m, Manifold &man, const PmhRigidBodyState &A,
+                              const PmhRigidBodyState &B, bool persistent_shapes, const HingeFrame &ha,
+                              const HingeFrame &hb) {
+    const uint32_t start = wave_reserve(&o.ctr->point_alloc, man.count);
+    write_manifold(o, m, man, start, A, B, persistent_shapes, ha, hb);
+}
+
 __device__ __forceinline__ bool persistent_pair(const ShapeDev &a, const ShapeDev &b, const PmhBodyParameters &pb) {
     const auto sup = [](const ShapeDev &s) { return s.kind != kShapeMesh || (s.has_planes && s.idx_count <= 96u); };
     return sup(a) && (pb.motion != kDynamic || sup(b));
+}
+
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+    return v;
+}
+
+__device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t lane) {
+    uint32_t x = v;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(x, d, 64);
+        if (lane >= uint32_t(d)) x += y;
+    }
+    return x - v;
+}
+
+// ---- the convex face path on 16 lanes ------------------------------------
+// A row of 16 lanes works on one pair, so that a small world's few pairs do
+// not each wait for one lane's serial search: the separating axes run over
+// the lanes, a clipped polygon has one vertex per lane and a manifold one
+// contact per lane.  The results are those of the serial functions above
+// (the same operations on each value, ties decided by the serial order).
+constexpr uint32_t kFaceLanes = 16;
+struct FaceShared {
+    float v[kFaceLanes][3];     // polygon vertices on their way to the next plane; contact points
+};
+
+__device__ __forceinline__ uint32_t row_bits(bool p) {   // one bit per lane of the row
+    return uint32_t(__ballot(p) >> (threadIdx.x & 48u)) & 0xffffu;
+}
+__device__ __forceinline__ void row_sync() {   // orders the row's LDS accesses (one wavefront: in order already)
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// Largest value of the row and, among equals, the smallest index.
+__device__ __forceinline__ void row_first_max(float &v, uint32_t &i) {
+    auto take = [&](float ov, uint32_t oi) {
+        if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
+    };
+    take(dpp_f32<kDppRowRor + 8>(v), dpp_u32<kDppRowRor + 8>(i));
+    take(dpp_f32<kDppRowRor + 4>(v), dpp_u32<kDppRowRor + 4>(i));
+    take(dpp_f32<kDppRowRor + 2>(v), dpp_u32<kDppRowRor + 2>(i));
+    take(dpp_f32<kDppRowRor + 1>(v), dpp_u32<kDppRowRor + 1>(i));
+}
+__device__ __forceinline__ float row_min(float v) {
+    v = smin(v, dpp_f32<kDppRowRor + 8>(v));
+    v = smin(v, dpp_f32<kDppRowRor + 4>(v));
+    v = smin(v, dpp_f32<kDppRowRor + 2>(v));
+    return smin(v, dpp_f32<kDppRowRor + 1>(v));
+}
+__device__ __forceinline__ V3 row_get(V3 v, uint32_t lane) {
+    return {__shfl(v.x, int(lane), 16), __shfl(v.y, int(lane), 16), __shfl(v.z, int(lane), 16)};
+}
+
+// What the face path needs of one side of a pair, in registers: lanes of one
+// row look at different sides at once, so a side is chosen by value.
+struct FaceSide {
+    V3 pos;
+    Q rot;
+    uint32_t planes, verts, vert_count, indices, faces;
+};
+__device__ __forceinline__ FaceSide face_side(const PmhRigidBodyState &s, const ShapeDev &m) {
+    return {sv(s.position), sq(s.orientation), m.plane_off, m.vtx_off, m.vtx_count, m.idx_off, m.idx_count / 3};
+}
+__device__ __forceinline__ FaceSide pick(bool first, const FaceSide &a, const FaceSide &b) {
+    FaceSide r;
+    r.pos = {first ? a.pos.x : b.pos.x, first ? a.pos.y : b.pos.y, first ? a.pos.z : b.pos.z};
+    r.rot = {first ? a.rot.x : b.rot.x, first ? a.rot.y : b.rot.y, first ? a.rot.z : b.rot.z, first ? a.rot.w : b.rot.w};
+    r.planes = first ? a.planes : b.planes;
+    r.verts = first ? a.verts : b.verts;
+    r.vert_count = first ? a.vert_count : b.vert_count;
+    r.indices = first ? a.indices : b.indices;
+    r.faces = first ? a.faces : b.faces;
+    return r;
+}
+struct FaceGeometry {
+    const V3 *verts;
+    const uint32_t *idx;
+    const float4 *planes;
+};
+
+// The support of a shape along an axis of its own frame.
+__device__ __forceinline__ float face_support(const FaceGeometry &geo, const FaceSide &m, V3 axis) {
+    const V3 *v = geo.verts + m.verts;
+    float support = 3.402823466e+38f;
+    uint32_t k = 0;
+    for (; k + 4 <= m.vert_count; k += 4) {
+        const V3 a = v[k], b = v[k + 1], c = v[k + 2], d = v[k + 3];
+        support = smin(support, dot(axis, a));
+        support = smin(support, dot(axis, b));
+        support = smin(support, dot(axis, c));
+        support = smin(support, dot(axis, d));
+    }
+    for (; k < m.vert_count; ++k) support = smin(support, dot(axis, v[k]));
+    return support;
+}
+
+// A manifold held by a row: contact i in lane i; all share the normal.
+struct RowManifold {
+    uint32_t count;
+    V3 normal, point;
+    float pen, impact;
+};
+
+// add_contact for a row: the candidate is the same in all lanes.
+__device__ __forceinline__ void row_add_contact(RowManifold &m, uint32_t lane, V3 point, float pen, float spacing) {
+    const float sp2 = spacing * spacing;
+    const uint32_t near = row_bits(lane < m.count && len2(sub(m.point, point)) < sp2);
+    uint32_t at;
+    bool put;
+    if (near != 0u) {
+        at = __builtin_ctz(near);
+        put = lane == at && pen - m.pen > 0.0f;
+    } else if (m.count < 8u) {
+        put = lane == m.count;
+        ++m.count;
+    } else {
+        uint32_t sh = 0;
+        float low = __shfl(m.pen, 0, 16);
+        for (uint32_t i = 1; i < 8u; ++i) {
+            const float p = __shfl(m.pen, int(i), 16);
+            if (p < low) { low = p; sh = i; }
+        }
+        put = lane == sh && pen > m.pen;
+    }
+    if (put) {
+        m.point = point;
+        m.pen = pen;
+    }
+}
+
+// reduce_face_patch for a row: the 28 pairs (f, s) of at most 8 contacts are
+// shared out over the lanes.
+__device__ __forceinline__ void row_reduce_patch(RowManifold &m, uint32_t lane, FaceShared &S, float tol) {
+    const float t2 = tol * tol;
+    for (uint32_t cand = 0; cand < m.count;) {
+        row_sync();
+        if (lane < m.count) {
+            S.v[lane][0] = m.point.x; S.v[lane][1] = m.point.y; S.v[lane][2] = m.point.z;
+        }
+        row_sync();
+        auto at = [&](uint32_t i) { return V3{S.v[i][0], S.v[i][1], S.v[i][2]}; };
+        bool removed = false;
+        for (; cand < m.count && !removed;) {
+            const V3 p = at(cand);
+            bool on = false;
+            for (uint32_t q = lane; q < 28u; q += kFaceLanes) {
+                // pair q of the 28: f < s < 8
+                const uint32_t f = q < 7u ? 0u : q < 13u ? 1u : q < 18u ? 2u : q < 22u ? 3u : q < 25u ? 4u : q < 27u ? 5u : 6u;
+                const uint32_t s = q - f * (13u - f) / 2u + 1u;
+                if (s >= m.count || f == cand || s == cand) continue;
+                const V3 pf = at(f);
+                const V3 e = sub(at(s), pf);
+                const float e2 = len2(e);
+                if (e2 <= t2) continue;
+                const float t = dot(sub(p, pf), e) / e2;
+                if (t <= 1.0e-4f || t >= 0.9999f) continue;
+                const V3 cl = add(pf, mul(e, t));
+                if (len2(sub(p, cl)) > t2) continue;
+                on = true;
+            }
+            removed = row_bits(on) != 0u;
+            if (!removed) ++cand;
+        }
+        if (removed) {
+            const uint32_t from = lane >= cand && lane < 15u ? lane + 1u : lane;
+            m.point = row_get(m.point, from);
+            m.pen = __shfl(m.pen, int(from), 16);
+            --m.count;
+            cand = 0;
+        }
+    }
+}
+
+// The separating-axis search of convex_face_manifold for a row: the face of
+// the largest separation (the collider's faces first), kFaceApart past reach.
+constexpr uint32_t kFaceApart = 0xffffffffu;
+__device__ __forceinline__ uint32_t row_axis(const FaceGeometry &geo, const FaceSide &body, const FaceSide &collider,
+                                             float reach, uint32_t lane) {
+    const uint32_t nc = collider.faces, faces = nc + body.faces;
+    float best = -3.402823466e+38f;
+    uint32_t best_at = 0xffffu;
+    for (uint32_t j = lane; j < faces; j += kFaceLanes) {
+        const bool of_c = j < nc;
+        const FaceSide rm = pick(of_c, collider, body), im = pick(of_c, body, collider);
+        const float4 pl = geo.planes[rm.planes + (of_c ? j : j - nc)];
+        const V3 nrm = rotate(rm.rot, v3(pl));
+        const V3 inn = inv_rotate(im.rot, nrm);
+        const float sep = face_support(geo, im, inn) + dot(nrm, sub(im.pos, rm.pos)) - pl.w;
+        if (sep > best) { best = sep; best_at = j; }
+    }
+    row_first_max(best, best_at);
+    if (best > reach) return kFaceApart;
+    return best_at == 0xffffu ? 0u : best_at;
+}
+
+// The rest of convex_face_manifold for a row.  kFaceWide: a clipped polygon
+// grew past one vertex per lane.
+enum : uint32_t { kFaceDeclined = 0, kFaceSolved = 1, kFaceWide = 2 };
+__device__ __forceinline__ uint32_t row_clip(const FaceGeometry &geo, const FaceSide &body, const FaceSide &collider,
+                                             float margin, float reach, uint32_t best_at, uint32_t lane, FaceShared &S,
+                                             RowManifold &out) {
+    const float rest = smin(margin, 1.0e-3f);
+    const uint32_t nc = collider.faces;
+    const bool ref_is_body = best_at >= nc;
+    const uint32_t ref_face = ref_is_body ? best_at - nc : best_at;
+    const FaceSide rm = pick(ref_is_body, body, collider), im = pick(ref_is_body, collider, body);
+    const Q rq = rm.rot;
+    const float4 reference = geo.planes[rm.planes + ref_face];
+    const V3 rn = v3(reference);
+    const V3 outward = rotate(rq, rn);
+    const V3 iaxis = inv_rotate(im.rot, outward);
+    const uint32_t ni = im.faces, rfaces = rm.faces;
+    const float4 *ip = geo.planes + im.planes, *rp = geo.planes + rm.planes;
+    // The most opposed face: the smallest alignment below one, negated for
+    // the search (the first face when none is below).
+    float opposed = -1.0f;
+    uint32_t inc_face = 0xffffu;
+    for (uint32_t f = lane; f < ni; f += kFaceLanes) {
+        const float val = -dot(iaxis, v3(ip[f]));
+        if (val > opposed) { opposed = val; inc_face = f; }
+    }
+    row_first_max(opposed, inc_face);
+    if (inc_face == 0xffffu) inc_face = 0u;
+    out.normal = mul(outward, ref_is_body ? -1.0f : 1.0f);
+    const float4 incident = ip[inc_face];
+    for (uint32_t t0 = 0; t0 < ni; t0 += kFaceLanes) {
+        // The triangles of the incident face among these 16.
+        bool same = t0 + lane < ni;
+        if (same) {
+            const float4 face = ip[t0 + lane];
+            if (dot(v3(face), v3(incident)) < 0.99999f || fabsf(face.w - incident.w) > 1.0e-5f) same = false;
+        }
+        for (uint32_t todo = row_bits(same); todo != 0u; todo &= todo - 1u) {
+            const uint32_t t = t0 + __builtin_ctz(todo);
+            uint32_t count = 3;
+            V3 cur = {0.0f, 0.0f, 0.0f};
+            if (lane < 3u) {
+                const V3 local = geo.verts[im.verts + geo.idx[im.indices + t * 3 + lane]];
+                cur = inv_rotate(rq, sub(add(im.pos, rotate(im.rot, local)), rm.pos));
+            }
+            for (uint32_t pi = 0; pi < rfaces && count != 0u; ++pi) {
+                const float4 pl = rp[pi];
+                const V3 pn = v3(pl);
+                const float off = pl.w + (dot(pn, rn) > 0.99999f ? reach : 0.0f);
+                const float d = dot(pn, cur) - off;
+                const uint32_t all = (1u << count) - 1u;
+                const uint32_t in = row_bits(d <= 0.0f) & all;
+                if (in == all) continue;             // every vertex kept
+                if (in == 0u) { count = 0; break; }
+                // Vertex k follows vertex k - 1 (the first the last); where
+                // the two differ, their crossing comes before vertex k.
+                const uint32_t before = ((in << 1) | (in >> (count - 1u))) & all;
+                const uint32_t cut = in ^ before;
+                const uint32_t next = __builtin_popcount(in) + __builtin_popcount(cut);
+                if (next > kFaceLanes) return kFaceWide;
+                const uint32_t prev_lane = lane == 0u ? count - 1u : lane - 1u;
+                const V3 prev = row_get(cur, prev_lane);
+                const float pd = __shfl(d, int(prev_lane), 16);
+                const uint32_t below = (1u << lane) - 1u;
+                uint32_t at = __builtin_popcount(in & below) + __builtin_popcount(cut & below);
+                row_sync();
+                if (lane < count && ((cut >> lane) & 1u)) {
+                    const V3 x = add(prev, mul(sub(cur, prev), pd / (pd - d)));
+                    S.v[at][0] = x.x; S.v[at][1] = x.y; S.v[at][2] = x.z;
+                    ++at;
+                }
+                if (lane < count && ((in >> lane) & 1u)) {
+                    S.v[at][0] = cur.x; S.v[at][1] = cur.y; S.v[at][2] = cur.z;
+                }
+                row_sync();
+                count = next;
+                cur = {S.v[lane][0], S.v[lane][1], S.v[lane][2]};
+            }
+            const float d = dot(rn, cur) - reference.w;
+            const V3 point = add(rm.pos, rotate(rq, sub(cur, mul(rn, d * 0.5f))));
+            const float pen = rest - d + 1.0e-5f;
+            for (uint32_t keep = row_bits(lane < count && !(d > reach)); keep != 0u; keep &= keep - 1u) {
+                const uint32_t k = __builtin_ctz(keep);
+                row_add_contact(out, lane, row_get(point, k), __shfl(pen, int(k), 16), smax(margin * 2.0f, 1.0e-4f));
+            }
+        }
+    }
+    if (out.count == 0u) return kFaceDeclined;
+    row_reduce_patch(out, lane, S, smax(1.0e-6f, margin * 1.0e-3f));
+    return kFaceSolved;
+}
+
+// The separating-axis half of swept_convex_face_manifold for a row.
+enum : uint32_t { kSweptDecline = 0, kSweptEmpty = 1, kSweptTouching = 2, kSweptImpact = 3 };
+__device__ __forceinline__ uint32_t row_swept_entry(const FaceGeometry &geo, const FaceSide &pb, const FaceSide &b,
+                                                    const FaceSide &pc, const FaceSide &c, float margin, uint32_t lane,
+                                                    float &entry, V3 &entry_normal) {
+    const Q bd = relative_quaternion(pb.rot, b.rot, false);
+    const Q cd = relative_quaternion(pc.rot, c.rot, false);
+    if (bd.x != 0.0f || bd.y != 0.0f || bd.z != 0.0f || cd.x != 0.0f || cd.y != 0.0f || cd.z != 0.0f)
+        return kSweptDecline;
+    const V3 bmo = sub(b.pos, pb.pos), cmo = sub(c.pos, pc.pos);
+    const float rest = smin(margin, 1.0e-3f);
+    float exit_time = 1.0f;
+    entry = 0.0f;
+    uint32_t entry_at = 0xffffu;
+    bool apart = false;
+    const uint32_t nc = pc.faces, faces = nc + pb.faces;
+    for (uint32_t j = lane; j < faces; j += kFaceLanes) {
+        const bool of_c = j < nc;
+        const FaceSide rm = pick(of_c, pc, pb), im = pick(of_c, pb, pc);
+        const V3 rel = of_c ? sub(bmo, cmo) : sub(cmo, bmo);
+        const float4 pl = geo.planes[rm.planes + (of_c ? j : j - nc)];
+        const V3 nrm = rotate(rm.rot, v3(pl));
+        const V3 inn = inv_rotate(im.rot, nrm);
+        const float gap = face_support(geo, im, inn) + dot(nrm, sub(im.pos, rm.pos)) - pl.w;
+        const float speed = dot(nrm, rel);
+        if (speed == 0.0f) {
+            apart = apart || gap > rest;
+        } else {
+            const float crossing = (rest - gap) / speed;
+            if (speed < 0.0f && crossing > entry) { entry = crossing; entry_at = j; }
+            if (speed > 0.0f) exit_time = smin(exit_time, crossing);
+        }
+    }
+    if (row_bits(apart) != 0u) return kSweptEmpty;
+    row_first_max(entry, entry_at);
+    exit_time = row_min(exit_time);
+    if (entry > exit_time || entry > 1.0f || exit_time < 0.0f) return kSweptEmpty;
+    if (entry == 0.0f) return kSweptTouching;
+    const bool of_c = entry_at < nc;
+    const FaceSide rm = pick(of_c, pc, pb);
+    entry_normal = mul(rotate(rm.rot, v3(geo.planes[rm.planes + (of_c ? entry_at : entry_at - nc)])), of_c ? 1.0f : -1.0f);
+    return kSweptImpact;
 }
 
 // One thread per pair: the convex face path (and its swept variant) for
@@ -1662,47 +1999,379 @@ __device__ __forceinline__ bool persistent_pair(const ShapeDev &a, const ShapeDe
 // pairs of two meshes; k_face_pairs runs the face path over that queue and
 // passes what it declines on to the triangle-pair path.  Each pair's output
 // sits at its own index, so the queues' order changes nothing.
-__global__ void __launch_bounds__(128) k_narrowphase(const uint32_t *npairs, const PmhBodyParameters *P,
-                                                     const ShapeDev *shapes, const PmhRigidBodyState *prev,
-                                                     const PmhRigidBodyState *pred, const uint2 *ab, NarrowOut o,
-                                                     uint32_t *face_list, const HingeFrame *frames,
-                                                     const float4 *frame_ref) {
+//
+// A block reserves the points and list places of its 256 pairs with one
+// atomic each: atomics on one address queue (about 10 ns each), and one per
+// wavefront kept this kernel at 121 us on a heap of 32768 bodies (517k pairs),
+// now 43 us.
+constexpr uint32_t kNarrowBlock = 256;
+__global__ void __launch_bounds__(kNarrowBlock) k_narrowphase(const uint32_t *npairs, const PmhBodyParameters *P,
+                                                              const ShapeDev *shapes, const PmhRigidBodyState *prev,
+                                                              const PmhRigidBodyState *pred, const uint2 *ab,
+                                                              NarrowOut o, uint32_t *face_list,
+                                                              const HingeFrame *frames, const float4 *frame_ref) {
+    __shared__ uint32_t part[2][kNarrowBlock / 64], base[2];
     const uint32_t M = *npairs;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     uint32_t unsupported = 0;
-    for (uint32_t m = blockIdx.x * blockDim.x + threadIdx.x; m < M; m += gridDim.x * blockDim.x) {
-        const uint2 p = ab[m];
-        const PmhBodyParameters pa = P[p.x], pb = P[p.y];
-        const ShapeDev sa = shapes[pa.mesh_index], sb = shapes[pb.mesh_index];
-        if (sa.kind == kShapeMesh && sb.kind == kShapeMesh) {
-            face_list[wave_reserve(&o.ctr->face_pairs, 1u)] = m;
-            continue;
-        }
-        const PmhRigidBodyState A0 = prev[p.x], A = pred[p.x], B = pred[p.y];
-        const float margin = pa.collision_margin + pb.collision_margin;
-        const float cr = correction_reach(pa, sa) + correction_reach(pb, sb);
-        const PairFrames fr = pair_frames(frames, frame_ref, pa, pb, p, A0, A);
+    for (uint32_t first = blockIdx.x * kNarrowBlock; first < M; first += gridDim.x * kNarrowBlock) {
+        const uint32_t m = first + threadIdx.x;
         Manifold man;
         man.count = 0;
         man.face_patch = 0;
-        if (!analytic_manifold(A, sa, B, sb, margin, margin + cr, man)) {
-            man.count = 0;
-            man.face_patch = 0;
-            ++unsupported;
+        bool mesh = false, persistent = false;
+        uint2 p = make_uint2(0u, 0u);
+        PmhRigidBodyState A, B;
+        HingeFrame ha, hb;
+        if (m < M) {
+            p = ab[m];
+            const PmhBodyParameters pa = P[p.x], pb = P[p.y];
+            const ShapeDev sa = shapes[pa.mesh_index], sb = shapes[pb.mesh_index];
+            mesh = sa.kind == kShapeMesh && sb.kind == kShapeMesh;
+            if (!mesh) {
+                A = pred[p.x];
+                B = pred[p.y];
+                const float margin = pa.collision_margin + pb.collision_margin;
+                const float cr = correction_reach(pa, sa) + correction_reach(pb, sb);
+                const PairFrames fr = pair_frames(frames, frame_ref, pa, pb, p, prev[p.x], A);
+                ha = fr.ha;
+                hb = fr.hb;
+                persistent = persistent_pair(sa, sb, pb);
+                if (!analytic_manifold(A, sa, B, sb, margin, margin + cr, man)) {
+                    man.count = 0;
+                    man.face_patch = 0;
+                    ++unsupported;
+                }
+            }
         }
-        emit_manifold(o, m, man, A, B, persistent_pair(sa, sb, pb), fr.ha, fr.hb);
+        // Places: this thread's within its wavefront, the wavefronts' within
+        // the block, the block's from one atomic per counter.
+        const uint64_t meshes = __ballot(mesh);
+        const uint32_t points_before = wave_exclusive_scan(man.count, lane);
+        if (lane == 63u) {
+            part[0][wave] = points_before + man.count;
+            part[1][wave] = uint32_t(__popcll(meshes));
+        }
+        __syncthreads();
+        if (threadIdx.x < 2u) {
+            uint32_t total = 0;
+            for (uint32_t w = 0; w < kNarrowBlock / 64; ++w) {
+                const uint32_t v = part[threadIdx.x][w];
+                part[threadIdx.x][w] = total;
+                total += v;
+            }
+            base[threadIdx.x] =
+                total ? atomicAdd(threadIdx.x == 0u ? &o.ctr->point_alloc : &o.ctr->face_pairs, total) : 0u;
+        }
+        __syncthreads();
+        if (mesh) {
+            face_list[base[1] + part[1][wave] + uint32_t(__popcll(meshes & ((1ull << lane) - 1ull)))] = m;
+        } else if (m < M) {
+            write_manifold(o, m, man, base[0] + part[0][wave] + points_before, A, B, persistent, ha, hb);
+        }
+        __syncthreads();
     }
     if (unsupported) atomicAdd(&o.ctr->unsupported, unsupported);
 }
 
-__global__ void __launch_bounds__(128) k_face_pairs(const uint32_t *face_list, const PmhBodyParameters *P,
-                                                    const ShapeDev *shapes, const V3 *verts, const uint32_t *idx,
-                                                    const float4 *planes, const PmhRigidBodyState *prev,
-                                                    const PmhRigidBodyState *pred, const uint2 *ab, NarrowOut o,
-                                                    uint32_t *tri_list, const HingeFrame *frames,
-                                                    const float4 *frame_ref) {
+// The queued mesh pairs, one row of 16 lanes each.  The face path runs at
+// most twice on the swept side (at the predicted states, then at the previous
+// ones, or at the time of impact) and once without; the rows of a wavefront
+// may be at different ones of these.  Pairs whose polygon outgrows the row
+// are queued for k_face_wide.
+//
+// One lane per pair took 213 us on a 55-box pyramid and 716 us on a heap of
+// 32768 bodies (one lane's serial search and clipping in scratch memory, too
+// few wavefronts in flight to hide it), and 538 us on 1024 scenes; rows take 30,
+// 186 and 194 us.
+//
+// A block first reads its pairs one lane each (bodies, shapes, whether the
+// pair is swept) into records in LDS, then its rows take the records one by
+// one: read by every lane of a row, that set-up cost more than the search on
+// worlds with many pairs that turn out apart.
+constexpr uint32_t kFaceBlock = 256, kFaceRows = kFaceBlock / kFaceLanes;
+constexpr uint32_t kFaceChunk = 64;     // most pairs of a block's round
+struct FaceInput {
+    float pose[4][7];                   // body before, after; collider before, after
+    uint32_t shape[2][5];               // planes, vertices, vertex count, indices, faces
+    float margin, reach;                // reach: the bounded solver correction
+};
+struct FaceResult {                     // in the place of the input of a pair that is done
+    float contact[8][4];                // point and penetration
+    float normal[3], impact;
+    uint32_t count, face_patch, kind, start;
+};
+enum : uint32_t { kResultEmit = 0, kResultTriangles = 1, kResultWide = 2 };
+struct FaceRecord {
+    union {
+        FaceInput in;
+        FaceResult out;
+    };
+    uint32_t pair, flags;
+    float entry, normal[3];             // swept: time of impact and its axis
+    uint32_t at, axis;                  // where the search stands, and the reference face
+    uint32_t pad;                       // odd stride: the records of a wavefront's lanes hit different banks
+};
+static_assert(sizeof(FaceRecord) % 8 == 4, "odd number of words");
+enum : uint32_t { kFaceConvex = 1, kFaceSwept = 2, kFaceGuided = 4, kFacePersistent = 8 };
+
+__device__ __forceinline__ FaceSide record_side(const FaceRecord &r, uint32_t pose, uint32_t shape) {
+    const float *q = r.in.pose[pose];
+    const uint32_t *s = r.in.shape[shape];
+    return {{q[0], q[1], q[2]}, {q[3], q[4], q[5], q[6]}, s[0], s[1], s[2], s[3], s[4]};
+}
+
+__global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_list, const PmhBodyParameters *P,
+                                                           const ShapeDev *shapes, FaceGeometry geo,
+                                                           const PmhRigidBodyState *prev, const PmhRigidBodyState *pred,
+                                                           const uint2 *ab, NarrowOut o, uint32_t *tri_list,
+                                                           uint32_t *wide_list, const HingeFrame *frames) {
+    __shared__ FaceShared shared_rows[kFaceRows];
+    __shared__ FaceRecord records[kFaceChunk];
+    __shared__ uint8_t list[kFaceChunk];
+    __shared__ uint32_t listed;
+    const uint32_t row = threadIdx.x / kFaceLanes, lane = threadIdx.x % kFaceLanes;
+    FaceShared &S = shared_rows[row];
     const uint32_t F = o.ctr->face_pairs;
+    // One pair per row while blocks are left, then more per block.
+    const uint32_t share = (F + gridDim.x - 1) / gridDim.x;
+    const uint32_t chunk = min(max((share + kFaceRows - 1) / kFaceRows * kFaceRows, kFaceRows), kFaceChunk);
+    enum : uint32_t { kPlain, kAtEnd, kAtStart, kAtImpact, kDone, kWide, kListed };
+    for (uint32_t base = blockIdx.x * chunk; base < F; base += gridDim.x * chunk) {
+        const uint32_t pairs = min(chunk, F - base);
+        if (threadIdx.x < pairs) {
+            FaceRecord &r = records[threadIdx.x];
+            const uint32_t m = face_list[base + threadIdx.x];
+            const uint2 p = ab[m];
+            const PmhBodyParameters pa = P[p.x], pb = P[p.y];
+            const ShapeDev sa = shapes[pa.mesh_index], sb = shapes[pb.mesh_index];
+            const PmhRigidBodyState A0 = prev[p.x], A = pred[p.x], B0 = prev[p.y], B = pred[p.y];
+            const float margin = pa.collision_margin + pb.collision_margin;
+            // Of the bodies' hinge contact frames only flags matter here.
+            bool guided = false, persistent = persistent_pair(sa, sb, pb);
+            if (frames) {
+                const HingeFrame &ha = frames[p.x], &hb = frames[p.y];
+                guided = guided_pair(ha, hb);
+                persistent = guided || (persistent && ha.present == 0u && hb.present == 0u && ha.fixed_member == 0u &&
+                                        hb.fixed_member == 0u);
+            }
+            auto put = [&](uint32_t k, const PmhRigidBodyState &s) {
+                r.in.pose[k][0] = s.position.x; r.in.pose[k][1] = s.position.y; r.in.pose[k][2] = s.position.z;
+                r.in.pose[k][3] = s.orientation.x; r.in.pose[k][4] = s.orientation.y; r.in.pose[k][5] = s.orientation.z;
+                r.in.pose[k][6] = s.orientation.w;
+            };
+            put(0, A0);
+            put(1, A);
+            put(2, B0);
+            put(3, B);
+            auto shape = [&](uint32_t k, const ShapeDev &s) {
+                r.in.shape[k][0] = s.plane_off; r.in.shape[k][1] = s.vtx_off; r.in.shape[k][2] = s.vtx_count;
+                r.in.shape[k][3] = s.idx_off; r.in.shape[k][4] = s.idx_count / 3;
+            };
+            shape(0, sa);
+            shape(1, sb);
+            r.in.margin = margin;
+            r.in.reach = correction_reach(pa, sa) + correction_reach(pb, sb);
+            r.pair = m;
+            // A guided pair leaves the face path (geometry.slang:2779).
+            const bool convex = sa.convex_face && sb.convex_face && !guided;
+            r.flags = (convex ? kFaceConvex : 0u) | (guided ? kFaceGuided : 0u) | (persistent ? kFacePersistent : 0u) |
+                      (convex && requires_swept(A0, A, sa, B0, B, sb, margin) ? kFaceSwept : 0u);
+        }
+        if (threadIdx.x == 0) listed = 0;
+        __syncthreads();
+        // Stage 0 searches the axes; pairs that are apart end there, the
+        // others are listed for stage 1, which clips.  A wavefront's four
+        // rows run in step: without the list one pair to clip made three
+        // that were done wait.
+#pragma unroll 1
+        for (uint32_t stage = 0; stage < 2u; ++stage) {
+            const uint32_t todo = stage == 0u ? pairs : listed;
+            for (uint32_t k = row; k < todo; k += kFaceRows) {
+                FaceRecord &r = records[stage == 0u ? k : list[k]];
+                const uint32_t m = r.pair, flags = r.flags;
+                const float margin = r.in.margin, rest = smin(margin, 1.0e-3f);
+                const bool swept = (flags & kFaceSwept) != 0u;
+                RowManifold man;
+                man.count = 0;
+                man.normal = man.point = {0.0f, 0.0f, 0.0f};
+                man.pen = 0.0f;
+                man.impact = 1.0f;
+                bool face = false;
+                uint32_t face_patch = 0, at = (flags & kFaceConvex) != 0u ? kPlain : kDone, axis = 0;
+                float entry = 0.0f;
+                V3 entry_normal = {0.0f, 0.0f, 0.0f};
+                if (stage != 0u) {
+                    at = r.at;
+                    axis = r.axis;
+                    entry = r.entry;
+                    entry_normal = {r.normal[0], r.normal[1], r.normal[2]};
+                } else if (swept) {
+                    const uint32_t kind = row_swept_entry(geo, record_side(r, 0, 0), record_side(r, 1, 0),
+                                                          record_side(r, 2, 1), record_side(r, 3, 1), margin, lane, entry,
+                                                          entry_normal);
+                    if (kind == kSweptEmpty) { at = kDone; face = true; }
+                    else if (kind == kSweptTouching) at = kAtEnd;
+                    else if (kind == kSweptImpact) at = kAtImpact;
+                }
+                bool search = stage == 0u;
+                while (at < kDone) {
+                    const uint32_t end = at == kAtStart || at == kAtImpact ? 0u : 1u;
+                    FaceSide a = record_side(r, end, 0), b = record_side(r, 2u + end, 1);
+                    if (at == kAtImpact) {
+                        a.pos = add(a.pos, mul(sub(record_side(r, 1, 0).pos, a.pos), entry));
+                        b.pos = add(b.pos, mul(sub(record_side(r, 3, 1).pos, b.pos), entry));
+                    }
+                    const float mg = at == kAtImpact ? rest + 1.0e-5f : margin;
+                    const float reach = mg + (at == kPlain ? r.in.reach : 0.0f);
+                    if (search) axis = row_axis(geo, a, b, reach, lane);
+                    search = true;
+                    uint32_t got = kFaceSolved;
+                    man.count = 0;
+                    man.impact = 1.0f;
+                    if (axis != kFaceApart) {
+                        if (stage == 0u) {
+                            if (lane == 0u) {
+                                r.at = at;
+                                r.axis = axis;
+                                r.entry = entry;
+                                r.normal[0] = entry_normal.x;
+                                r.normal[1] = entry_normal.y;
+                                r.normal[2] = entry_normal.z;
+                                list[atomicAdd(&listed, 1u)] = uint8_t(k);
+                            }
+                            at = kListed;
+                            break;
+                        }
+                        got = row_clip(geo, a, b, mg, reach, axis, lane, S, man);
+                    }
+                    const bool ok = got == kFaceSolved;
+                    face_patch = ok && man.count != 0u ? 1u : 0u;
+                    if (got == kFaceWide) {
+                        at = kWide;
+                    } else if (at == kPlain) {
+                        face = ok && !(swept && man.count == 0u);
+                        at = kDone;
+                    } else if (!ok || man.count == 0u) {
+                        at = at == kAtEnd ? kAtStart : kPlain;
+                    } else if (at == kAtEnd) {
+                        face = true;
+                        at = kDone;
+                    } else {
+                        const V3 motion = sub(sub(record_side(r, 1, 0).pos, record_side(r, 0, 0).pos),
+                                              sub(record_side(r, 3, 1).pos, record_side(r, 2, 1).pos));
+                        const float closing = -dot(motion, man.normal);
+                        if (at == kAtStart) {
+                            face = !(closing <= 0.0f);
+                            man.pen += closing;
+                            man.impact = 0.0f;
+                        } else {
+                            face = !(dot(man.normal, entry_normal) < 0.99999f);
+                            const float remaining = closing * (1.0f - entry);
+                            man.pen = smax(0.0f, remaining + man.pen) + rest + 1.0e-5f;
+                            man.impact = entry;
+                        }
+                        at = face ? kDone : kPlain;
+                    }
+                }
+                if (at == kListed) continue;
+                row_sync();
+                if (lane < man.count) {
+                    r.out.contact[lane][0] = man.point.x; r.out.contact[lane][1] = man.point.y;
+                    r.out.contact[lane][2] = man.point.z; r.out.contact[lane][3] = man.pen;
+                }
+                if (lane == 0u) {
+                    r.out.normal[0] = man.normal.x; r.out.normal[1] = man.normal.y; r.out.normal[2] = man.normal.z;
+                    r.out.impact = man.impact;
+                    r.out.kind = at == kWide ? kResultWide : face ? kResultEmit : kResultTriangles;
+                    r.out.count = at != kWide && face ? man.count : 0u;
+                    r.out.face_patch = face_patch;
+                }
+            }
+            __syncthreads();
+        }
+        // The block's results go out together: one reservation of points and
+        // of list places for all its pairs (atomics on one address queue,
+        // about 10 ns each), then one thread per contact.
+        if (threadIdx.x < 64u) {
+            const bool live = threadIdx.x < pairs;
+            FaceRecord &r = records[live ? threadIdx.x : 0u];
+            const uint32_t kind = live ? r.out.kind : kResultEmit;
+            uint32_t count = live ? r.out.count : 0u;
+            const uint64_t tri = __ballot(kind == kResultTriangles), wide = __ballot(kind == kResultWide);
+            const uint32_t before = wave_exclusive_scan(count, threadIdx.x), total = wave_sum(count);
+            uint32_t at_point = 0, at_tri = 0, at_wide = 0;
+            if (threadIdx.x == 0u) {
+                if (total) at_point = atomicAdd(&o.ctr->point_alloc, total);
+                if (tri) at_tri = atomicAdd(&o.ctr->tri_pairs, uint32_t(__popcll(tri)));
+                if (wide) at_wide = atomicAdd(&o.ctr->wide_pairs, uint32_t(__popcll(wide)));
+            }
+            const uint64_t below = (1ull << threadIdx.x) - 1ull;
+            const uint32_t start = __shfl(at_point, 0, 64) + before;
+            at_tri = __shfl(at_tri, 0, 64) + uint32_t(__popcll(tri & below));
+            at_wide = __shfl(at_wide, 0, 64) + uint32_t(__popcll(wide & below));
+            if (live) {
+                const uint32_t m = r.pair;
+                if (kind == kResultTriangles) {
+                    tri_list[at_tri] = m;
+                } else if (kind == kResultWide) {
+                    wide_list[at_wide] = m;
+                } else {
+                    if (count && start + count > o.point_cap) {
+                        atomicOr(&o.ctr->status, kStatusPointOverflow);
+                        count = 0;
+                    }
+                    const uint2 p = ab[m];
+                    o.m_count[m] = count;
+                    o.m_start[m] = start;
+                    o.m_face[m] = r.out.face_patch;
+                    o.m_init_rel[m] = f4(sub(sv(pred[p.x].position), sv(pred[p.y].position)), 0.0f);
+                }
+                r.out.count = count;
+                r.out.start = start;
+            }
+        }
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < 8u * pairs; k += kFaceBlock) {
+            const FaceRecord &r = records[k / 8u];
+            const uint32_t q = k % 8u;
+            if (q >= r.out.count) continue;
+            const uint32_t i = r.out.start + q, m = r.pair;
+            const uint2 p = ab[m];
+            const PmhRigidBodyState A = pred[p.x], B = pred[p.y];
+            const float *c = r.out.contact[q];
+            const V3 normal = {r.out.normal[0], r.out.normal[1], r.out.normal[2]}, point = {c[0], c[1], c[2]};
+            const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            o.c_np[i] = f4(normal, c[3]);
+            o.c_pt[i] = f4(point, normal_speed(A, B, point, normal));
+            o.c_aa[i] = make_float4(0.0f, 0.0f, 0.0f, r.out.impact);   // w: impact fraction
+            o.c_ab[i] = z;
+            o.c_err[i] = z;
+            o.c_lam[i] = z;
+            o.c_pen[i] = z;
+            o.c_acc[i] = z;
+            o.c_rep[i] = z;
+            o.c_flags[i] = ((r.flags & kFacePersistent) ? 2u : 0u) | ((r.flags & kFaceGuided) ? kPointGuided : 0u);
+            o.c_pair[i] = m;
+        }
+        __syncthreads();
+    }
+}
+
+// Listed pairs one lane each, with the serial functions: a polygon clipped by
+// more planes than lanes can hold vertices for.  A plane adds at most one
+// vertex to a triangle's three, so only shapes of more than 13 triangles get
+// here.
+constexpr uint32_t kRowFaces = kFaceLanes - 3;
+__global__ void __launch_bounds__(128) k_face_wide(const uint32_t *wide_list, const PmhBodyParameters *P,
+                                                   const ShapeDev *shapes, const V3 *verts, const uint32_t *idx,
+                                                   const float4 *planes, const PmhRigidBodyState *prev,
+                                                   const PmhRigidBodyState *pred, const uint2 *ab, NarrowOut o,
+                                                   uint32_t *tri_list, const HingeFrame *frames,
+                                                   const float4 *frame_ref) {
+    const uint32_t F = o.ctr->wide_pairs;
     for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < F; f += gridDim.x * blockDim.x) {
-        const uint32_t m = face_list[f];
+        const uint32_t m = wide_list[f];
         const uint2 p = ab[m];
         const PmhBodyParameters pa = P[p.x], pb = P[p.y];
         ShapeView sa{shapes[pa.mesh_index], verts, idx, planes};
@@ -1775,20 +2444,6 @@ struct TriWaveShared {
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     __builtin_amdgcn_wave_barrier();
-}
-
-__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
-}
-
-__device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t lane) {
-    uint32_t x = v;
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d, 64);
-        if (lane >= uint32_t(d)) x += y;
-    }
-    return x - v;
 }
 
 __device__ __forceinline__ bool leaf_cell_overlaps(const TrianglePair &tp, bool swept, const BoundsFrame &fa,
@@ -2196,6 +2851,7 @@ __global__ void k_step_begin(StepCounters *ctr) {
     ctr->point_alloc = 0;
     ctr->tri_pairs = 0;
     ctr->face_pairs = 0;
+    ctr->wide_pairs = 0;
     ctr->fallback_pairs = 0;
     ctr->cell_size_bits = 0.0f;
 }
@@ -2299,11 +2955,16 @@ PmhResult World::step_once(uint32_t k_step, bool warm_infer) {
         jv.list = v.jlist;
         k_hinge_frames<<<bg, 256, 0, s>>>(n, params.p, prev, pred, jv, frames, frame_ref);
     }
-    k_narrowphase<<<blocks_for(v.pair_cap, 128, 4096), 128, 0, s>>>(&ctr->pairs, params.p, shapes_dev.p, prev, pred,
+    k_narrowphase<<<blocks_for(v.pair_cap, kNarrowBlock, 2048), kNarrowBlock, 0, s>>>(&ctr->pairs, params.p, shapes_dev.p, prev, pred,
                                                                     v.ab.p, out, v.face_list.p, frames, frame_ref);
-    k_face_pairs<<<blocks_for(v.pair_cap, 128, 4096), 128, 0, s>>>(
-        v.face_list.p, params.p, shapes_dev.p, verts_dev.p, idx_dev.p, planes_dev.p, prev, pred, v.ab.p, out,
-        v.tri_list.p, frames, frame_ref);
+    const FaceGeometry geo{verts_dev.p, idx_dev.p, planes_dev.p};
+    // The list of wide pairs lies in the impact flags, written later.
+    k_face_pairs<<<blocks_for(v.pair_cap, kFaceRows, 4096), kFaceBlock, 0, s>>>(
+        v.face_list.p, params.p, shapes_dev.p, geo, prev, pred, v.ab.p, out, v.tri_list.p, v.m_impact.p, frames);
+    if (face_triangles > kRowFaces)
+        k_face_wide<<<blocks_for(v.pair_cap, 128, 1024), 128, 0, s>>>(
+            v.m_impact.p, params.p, shapes_dev.p, verts_dev.p, idx_dev.p, planes_dev.p, prev, pred, v.ab.p, out,
+            v.tri_list.p, frames, frame_ref);
     k_triangle_pairs<<<2048, 256, 0, s>>>(
         v.tri_list.p, params.p, shapes_dev.p, verts_dev.p, idx_dev.p, planes_dev.p, nodes_dev.p, leaves_dev.p,
         shell_dev.p, prev, pred, v.ab.p, out, leaf_slots, leaf_limit, dt, rules, frames, frame_ref);

@@ -309,8 +309,10 @@ PmhResult World::ensure_device() {
         std::vector<float4> planes, shell;
         std::vector<BvhDev> nodes;
         std::vector<uint32_t> leaves;
+        face_triangles = 0;
         for (HostShape &s : shapes) {
             ShapeDev d = s.info;
+            if (d.convex_face) face_triangles = std::max(face_triangles, d.idx_count / 3);
             d.vtx_off = uint32_t(verts.size());
             d.idx_off = uint32_t(idx.size());
             d.plane_off = uint32_t(planes.size());
