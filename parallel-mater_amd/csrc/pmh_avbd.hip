@@ -625,9 +625,8 @@ __device__ __forceinline__ bool color_wait(const uint32_t *color, uint32_t j, ui
 
 __global__ void __launch_bounds__(256) k_color_lane(uint32_t n, const PmhBodyParameters *P, const uint2 *ab,
                                                const uint32_t *adj_start, const uint32_t *adj, uint32_t *color,
-                                               const uint32_t *jstart, const uint32_t *jadj,
-                                               const PmhRigidConstraint *joints, StepCounters *ctr,
-                                               uint32_t limit) {
+                                               const uint32_t *jstart, const uint2 *jent, bool joints,
+                                               StepCounters *ctr, uint32_t limit) {
     const uint32_t lane = threadIdx.x & 63;
     for (;;) {
         uint32_t base = 0;
@@ -658,9 +657,8 @@ __global__ void __launch_bounds__(256) k_color_lane(uint32_t n, const PmhBodyPar
                 }
                 if (!blocked)
                     for (; jk < je; ++jk) {
-                        const PmhRigidConstraint &jt = joints[jadj[jk]];
-                        const uint32_t j = jt.dense_a == i ? jt.dense_b : jt.dense_a;
-                        if (j >= i || P[j].motion != kDynamic) continue;
+                        const uint32_t other = jent[jk].y, j = other & kEntryBody;
+                        if (j >= i || (other & kEntryFixed) != 0u) continue;
                         if (!color_wait(color, j, u0, u1, u2, u3)) { blocked = true; break; }
                     }
                 if (!blocked) {
@@ -720,9 +718,9 @@ __device__ __forceinline__ uint32_t color_wait_bounded(const uint32_t *color, ui
 __global__ void __launch_bounds__(64 * kColorWaveBlock) k_color_wave(uint32_t n, const PmhBodyParameters *P,
                                                                    const uint2 *ab, const uint32_t *adj_start,
                                                                    const uint32_t *adj, uint32_t *color,
-                                                                   const uint32_t *jstart, const uint32_t *jadj,
-                                                                   const PmhRigidConstraint *joints,
-                                                                   StepCounters *ctr, uint32_t limit) {
+                                                                   const uint32_t *jstart, const uint2 *jent,
+                                                                   bool joints, StepCounters *ctr,
+                                                                   uint32_t limit) {
     __shared__ uint32_t s_ticket[2];
     __shared__ uint32_t s_top[kColorWaveBlock];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -752,9 +750,8 @@ __global__ void __launch_bounds__(64 * kColorWaveBlock) k_color_wave(uint32_t n,
         }
         if (joints && !gave_up) {
             for (uint32_t k = jstart[i] + lane; k < jstart[i + 1]; k += 64) {
-                const PmhRigidConstraint &jt = joints[jadj[k]];
-                const uint32_t j = jt.dense_a == i ? jt.dense_b : jt.dense_a;
-                if (j >= i || P[j].motion != kDynamic) continue;
+                const uint32_t other = jent[k].y, j = other & kEntryBody;
+                if (j >= i || (other & kEntryFixed) != 0u) continue;
                 const uint32_t c = color_wait_bounded(color, j, ctr, limit);
                 if (c == kInvalid) { gave_up = true; break; }
                 if (c < kMaxColors) used[c >> 6] |= 1ull << (c & 63);
@@ -981,6 +978,8 @@ struct SolveArgs {
     PmhRigidConstraint *joints;
     uint32_t nj;
     const uint32_t *jstart, *jadj;       // per-body incident joints, descending index
+    uint2 *jent;                         // the same list as entries (k_joint_entries)
+    JointStep *jstep;                    // what the step's visits of a joint share
     const PmhRigidBodyState *prev;
     // dataflow sweep: colours, the mailboxes, this sweep's stamp and the poll
     // limit of its waits
@@ -1009,9 +1008,8 @@ __global__ void k_uf_sample(SolveArgs a, const uint2 *ab, const uint32_t *adj_st
     }
     if (a.nj)
         for (uint32_t e = a.jstart[i]; e < a.jstart[i + 1]; ++e) {
-            const PmhRigidConstraint &jt = a.joints[a.jadj[e]];
-            const uint32_t j = jt.dense_a == i ? jt.dense_b : jt.dense_a;
-            if (a.P[j].motion == kDynamic) best = min(best, ld_parent(&parent[j]));
+            const uint32_t other = a.jent[e].y;
+            if ((other & kEntryFixed) == 0u) best = min(best, ld_parent(&parent[other & kEntryBody]));
         }
     if (best < r && ld_relaxed(&parent[r]) > best) atomicMin(&parent[r], best);
 }
@@ -1031,14 +1029,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t flow_box(const SolveArgs &a) {
 // instead of hanging.  The abort flag is read every 256th poll only:
 // thousands of waiting lanes reading one address on every poll would queue on
 // one memory channel, and the waits would slow down the bodies they wait for.
+// kW: the rotation delta's w with it, in d[6].
+template <bool kW = false>
 __device__ __forceinline__ void flow_take(const SolveArgs &a, __amdgpu_buffer_rsrc_t box, uint32_t j, float *d) {
-    flow_pair w0, w1, w2;
+    flow_pair w0, w1, w2, w3;
     for (uint32_t polls = 1;; ++polls) {
         w0 = flow_load(box, j, 0);
         w1 = flow_load(box, j, 1);
         w2 = flow_load(box, j, 2);
         const uint32_t s = a.flow_stamp;
-        if (((w0[1] ^ s) | (w0[3] ^ s) | (w1[1] ^ s) | (w1[3] ^ s) | (w2[1] ^ s) | (w2[3] ^ s)) == 0u) break;
+        if (kW) w3 = flow_load(box, j, 3);
+        else w3[1] = s;
+        if (((w0[1] ^ s) | (w0[3] ^ s) | (w1[1] ^ s) | (w1[3] ^ s) | (w2[1] ^ s) | (w2[3] ^ s) |
+             (w3[1] ^ s)) == 0u) break;
         if (polls > a.flow_limit) {
             st_relaxed(&a.ctr->color_abort, 1u);
             st_relaxed(&a.ctr->sweep_failed, 1u);
@@ -1051,6 +1054,7 @@ __device__ __forceinline__ void flow_take(const SolveArgs &a, __amdgpu_buffer_rs
     }
     d[0] = __uint_as_float(w0[0]); d[1] = __uint_as_float(w0[2]); d[2] = __uint_as_float(w1[0]);
     d[3] = __uint_as_float(w1[2]); d[4] = __uint_as_float(w2[0]); d[5] = __uint_as_float(w2[2]);
+    if (kW) d[6] = __uint_as_float(w3[0]);
 }
 // The rotation delta's w of a body whose displacement has been taken.
 __device__ __forceinline__ float flow_take_w(const SolveArgs &a, __amdgpu_buffer_rsrc_t box, uint32_t j) {
@@ -1072,9 +1076,9 @@ __device__ __forceinline__ float row_error(float e0, float4 axis, float4 angA, f
     return e0 + dot6(ja, dA) + dot6(jb, dB);
 }
 
-template <bool kFlow>
+template <bool kFlow, int L>
 __device__ __forceinline__ void body_joint_rows(const SolveArgs &a, uint32_t i, uint32_t phase, Block &blk,
-                                                uint32_t sub_lane, uint32_t L, const float *dI, float wI);
+                                                uint32_t lane, const float *dI, float wI);
 
 // A value the optimiser does not look through: a choice between such values
 // stays a choice between registers (a choice between elements of one array is
@@ -1363,7 +1367,7 @@ __device__ __forceinline__ void solve_group(const SolveArgs &a, uint32_t base, u
     if constexpr (kFlow && L >= 16) __builtin_amdgcn_s_setprio(3);
     // Joint rows follow the contact rows (solve.slang:401-430), each
     // joint in one lane's partial block.
-    if (kJoints && active) body_joint_rows<kFlow>(a, i, phase, blk, sub_lane, L, dI, dq.w);
+    if (kJoints && active) body_joint_rows<kFlow, L>(a, i, phase, blk, lane, dI, dq.w);
     group_reduce<L>(blk);
     float update[6];
     bool solved = false;
@@ -1510,13 +1514,16 @@ __device__ void solve_color(const SolveArgs &a, uint32_t begin, uint32_t end, ui
 }
 
 // The pose of body i with displacement d and rotation delta q.
-__device__ __forceinline__ PmhRigidBodyState pose_with(const SolveArgs &a, uint32_t i, V3 d, Q dq) {
+__device__ __forceinline__ PmhRigidBodyState pose_at(float4 target_pos, float4 target_q, V3 d, Q dq) {
     PmhRigidBodyState s;
-    s.position = pv(add(v3(a.tpos[i]), d));
-    Q o = q4(a.tq[i]);
+    s.position = pv(add(v3(target_pos), d));
+    Q o = q4(target_q);
     if (dq.x != 0.0f || dq.y != 0.0f || dq.z != 0.0f) o = qnormalize(qmul(dq, o));
     s.orientation = pq(o);
     return s;
+}
+__device__ __forceinline__ PmhRigidBodyState pose_with(const SolveArgs &a, uint32_t i, V3 d, Q dq) {
+    return pose_at(a.tpos[i], a.tq[i], d, dq);
 }
 __device__ __forceinline__ PmhRigidBodyState avbd_pose(const SolveArgs &a, uint32_t i) {
     return pose_with(a, i, v3(a.disp[2 * i]), q4(a.dq[i]));
@@ -1529,10 +1536,20 @@ __device__ __forceinline__ PmhRigidBodyState pose_from(const SolveArgs &a, uint3
 
 // ---------------------------------------------------------------------
 // Joints: rigid_avbd_visit_joint(_row), geometry_constraints.slang:
-// 289-445, 626-926.  One routine builds a joint's rows for the four visits
-// (initialise in prepare, accumulate in the colour sweep, advance in the
-// dual update, the velocity-phase rows).  Same operations and order as the
-// reference.
+// 289-445, 626-926.  The reference builds a joint's rows anew in each of four
+// visits (initialise in prepare, accumulate in the colour sweep, advance in
+// the dual update, the velocity-phase rows).  Here the first one
+// (initialize_joint) also lists the rows that the joint's type and options
+// give, with everything that only the step's start decides (JointStep), and
+// the others walk that list: one loop of one row's code.  Same operations and
+// order per row as the reference.
+//
+// What bounded the sweep over chains was this code: 23 KB, unrolled over
+// axes, kinds of row and types, run once per body from a cold instruction
+// cache, with loads in its branches and the other end's id, colour,
+// displacement and w each a dependent trip to memory.  A sweep over
+// 16 chains of 16 links (32 lanes) took 105 us, now 59; over 1024 chains of 64
+// (8 lanes) 256 us, now 145; their dual updates 13 and 29 us, now 9 and 22.
 // ---------------------------------------------------------------------
 // Both ends of a joint as a visit sees them: displacements and the rotation
 // deltas' w.
@@ -1548,7 +1565,6 @@ __device__ __forceinline__ JointEnds joint_ends(const SolveArgs &a, uint32_t ia,
     return e;
 }
 
-enum : uint32_t { kVisitInitialize = 0, kVisitAccumulate = 1, kVisitAdvance = 2, kVisitImpact = 3 };
 constexpr float kLimitStabilization = 0.8f;
 
 __device__ __forceinline__ float aabs_(float v) { return v < 0.0f ? -v : v; }
@@ -1580,8 +1596,8 @@ __device__ __forceinline__ V3 iiw(const PmhBodyParameters &p, Q o, V3 w) {
                       l.z * p.inverse_inertia_local.z});
 }
 
-// rigid_avbd_log_axis, :401-422.
-__device__ V3 log_axis(Q frame, V3 lg, uint32_t axis) {
+// rigid_avbd_log_axis, :401-422, and its coefficient, the same for every axis.
+__device__ __forceinline__ float log_coefficient(V3 lg) {
     const float sq2 = len2(lg);
     float coef = 1.0f / 12.0f + sq2 * (1.0f / 720.0f + sq2 * (1.0f / 30240.0f + sq2 * (1.0f / 1209600.0f +
                  sq2 / 47900160.0f)));
@@ -1590,7 +1606,9 @@ __device__ V3 log_axis(Q frame, V3 lg, uint32_t axis) {
         const float half = 0.5f * angle;
         coef = (1.0f - half * cosf(half) / sinf(half)) / sq2;
     }
-    const V3 unit = basis_axis(axis);
+    return coef;
+}
+__device__ __forceinline__ V3 log_axis(Q frame, V3 lg, float coef, V3 unit) {
     const V3 local = add(add(unit, mul(cross(lg, unit), 0.5f)), mul(cross(lg, cross(lg, unit)), coef));
     return rotate(frame, local);
 }
@@ -1599,117 +1617,220 @@ __device__ __forceinline__ V3 rel_rotation_vector(Q a, Q b) {
     return quaternion_rotation_vector(relative_quaternion(a, b, true));
 }
 
-struct JointRowArgs {
-    float ja[6], jb[6];
-    float current, previous, penalty;
-    bool angular;
-    float stiffness, damping, lower, upper;
-    bool motor;
-    float motor_speed;
-    V3 curv_a, curv_b;
-    float stabilization;
-};
-
 __device__ __forceinline__ void set6(float *d, V3 l, V3 r) {
     d[0] = l.x; d[1] = l.y; d[2] = l.z; d[3] = r.x; d[4] = r.y; d[5] = r.z;
 }
 
-// rigid_avbd_visit_joint_row, :626-713.
-__device__ void visit_joint_row(const SolveArgs &a, PmhRigidConstraint &j, Block &blk, uint32_t &index,
-                                float &impulse, bool first, const JointRowArgs &r, uint32_t visit,
-                                const JointEnds &ends) {
-    if (index >= 18u) return;
-    const uint32_t ri = index++;
-    PmhAvbdRow row = j.rows[ri];
-    const uint32_t ia = j.dense_a, ib = j.dense_b;
-    const float *da = ends.da, *db = ends.db;
-    const float linearized = dot6(r.ja, da) + dot6(r.jb, db);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) { row.a[k] = r.ja[k]; row.b[k] = r.jb[k]; }
-    row.stiffness = r.stiffness;
-    row.damping = r.damping;
-    if (visit == kVisitInitialize) {
-        if (!(row.penalty > kMinPenalty)) row.penalty = r.penalty;
-        warm_start(row.lambda, row.penalty, r.stiffness);
-        if (r.stiffness < kMaxPenalty) row.lambda = 0.0f;
-        row.beta = r.penalty * (r.angular ? 10.0f : 100.0f);
-        row.reference_force = 0.0f;
-    }
-    row.error = r.current - (r.stiffness < kMaxPenalty ? 0.0f : r.stabilization * r.previous) - linearized;
-    row.velocity = r.motor ? r.motor_speed : (r.current - r.previous - linearized) / a.dt;
-    row.lower = r.lower;
-    row.upper = r.upper;
-    if (visit == kVisitAccumulate) {
-        jrow_accumulate(blk, row, first, da, db, a.dt);
-        if (!r.angular) {
-            const V3 axis = {r.jb[0], r.jb[1], r.jb[2]};
-            const V3 arm = first ? r.curv_a : r.curv_b;
-            const float force = jrow_force(row, da, db, a.dt);
-            for (uint32_t c = 0; c < 3; ++c) {
-                const V3 value = sub(mul(add(mul(axis, comp(arm, c)), mul(arm, comp(axis, c))), 0.5f),
-                                     mul(basis_axis(c), dot(axis, arm)));
-                const uint32_t d = 3 + c;
-                blk.h[d * (d + 1) / 2 + d] += fabsf(force) * sqrtf(len2(value));
-            }
-        }
-        return;
-    }
-    if (visit == kVisitAdvance) {
-        impulse += fabsf(jrow_force(row, da, db, a.dt)) * a.dt;
-        jrow_advance(row, da, db);
-    } else if (visit == kVisitImpact) {
-        if (r.stiffness < kMaxPenalty) {
-            row.reference_force = jrow_force(row, da, db, a.dt);
-        } else {
-            const float gap = r.lower == 0.0f ? smin(0.0f, r.current) : (r.upper == 0.0f ? smax(0.0f, r.current) : 0.0f);
-            float va[6], vb[6];
-            set6(va, mul(v3(a.tv[ia]), a.dt), mul(v3(a.tw[ia]), a.dt));
-            set6(vb, mul(v3(a.tv[ib]), a.dt), mul(v3(a.tw[ib]), a.dt));
-            row.reference_force = row.lambda;
-            row.error = dot6(r.ja, va) + dot6(r.jb, vb) + gap - (r.motor ? r.motor_speed * a.dt : 0.0f);
-        }
-    }
-    j.rows[ri] = row;
+// A joint's two frames in their bodies' poses and what its rows measure.
+struct JointFrames {
+    V3 armA, armB, error;
+    Q fA, fB;
+};
+__device__ __forceinline__ JointFrames joint_frames(const JointHead &o, const PmhRigidBodyState &sa,
+                                                    const PmhRigidBodyState &sb) {
+    JointFrames f;
+    const Q qa = sq(sa.orientation), qb = sq(sb.orientation);
+    f.armA = rotate(qa, sv(o.anchor_a));
+    f.armB = rotate(qb, sv(o.anchor_b));
+    f.error = sub(add(sv(sb.position), f.armB), add(sv(sa.position), f.armA));
+    f.fA = qnormalize(qmul(qa, sq(o.orientation_a)));
+    f.fB = qnormalize(qmul(qb, sq(o.orientation_b)));
+    return f;
+}
+__device__ __forceinline__ V3 joint_free_axis(uint32_t flags) {
+    return (flags & kJointAxisZ) != 0u ? V3{0.0f, 0.0f, 1.0f} : V3{1.0f, 0.0f, 0.0f};
 }
 
-// rigid_avbd_visit_joint, :715-926.
-__device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstraint &j, Block &blk, bool first,
-                                          uint32_t visit, const JointEnds &ends) {
-    uint32_t index = 0;
+// What a walk reads of a row besides its own geometry.
+struct JointRowIn {
+    JointRowStep s;
+    float lambda, penalty, velocity, lower, upper, stiffness, damping, beta, reference_force;
+};
+__device__ __forceinline__ JointRowIn joint_row_in(const JointRowStep *rows, const PmhRigidConstraint &j,
+                                                   uint32_t r) {
+    JointRowIn in;
+    in.s = rows[r];
+    const PmhAvbdRow &row = j.rows[r];
+    in.lambda = row.lambda; in.penalty = row.penalty; in.velocity = row.velocity;
+    in.lower = row.lower; in.upper = row.upper; in.stiffness = row.stiffness; in.damping = row.damping;
+    in.beta = row.beta; in.reference_force = row.reference_force;
+    return in;
+}
+
+// Whether a row is a hard equality, whose violation the residual counts.
+__device__ __forceinline__ bool hard_equality(float stiffness, float lower, float upper) {
+    return !(stiffness < kMaxPenalty || lower != -kMaxPenalty || upper != kMaxPenalty);
+}
+
+// A later visit: the listed rows at the ends' poses.  Accumulate adds them to
+// the block of one end; the others write the rows.  Advance returns the
+// applied impulse, and in `residual` the largest violation of a hard equality.
+enum : uint32_t { kVisitWrite = 0, kVisitAccumulate = 1, kVisitAdvance = 2, kVisitImpact = 3 };
+template <uint32_t kVisit>
+__device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstraint &j, const JointHead &st,
+                                             const JointRowStep *rows, const PmhRigidBodyState &sa, const PmhRigidBodyState &sb, JointRowIn in,
+                                             const JointEnds &ends, Block &blk, bool first, float &residual) {
+    const JointFrames f = joint_frames(st, sa, sb);
+    const uint32_t flags = st.flags, count = st.count;
+    const V3 free_axis = joint_free_axis(flags);
+    const V3 zero = {0.0f, 0.0f, 0.0f};
+    V3 twist = zero, swing_axis = zero, turn = zero;
+    float twist_coef = 0.0f, turn_coef = 0.0f;
+    if ((flags & kJointTwist) != 0u) {
+        twist = rel_rotation_vector(f.fA, f.fB);
+        twist_coef = log_coefficient(twist);
+    }
+    const bool swing = (flags & kJointSwing) != 0u;
+    if (swing) swing_axis = inv_rotate(f.fA, rotate(f.fB, free_axis));
+    if ((flags & kJointMotorTurn) != 0u) {
+        turn = rel_rotation_vector({0.0f, 0.0f, 0.0f, 1.0f},
+                                   relative_quaternion(sq(st.old_relative), relative_quaternion(f.fA, f.fB, true), false));
+        turn_coef = log_coefficient(turn);
+    }
+    const V3 swing_rotation = cross(free_axis, swing_axis);
+    const V3 arm = first ? add(f.error, f.armA) : f.armB;   // of a linear row's curvature
+    const float *da = ends.da, *db = ends.db;
     float impulse = 0.0f;
+#pragma unroll 1
+    for (uint32_t ri = 0; ri < count; ++ri) {
+        const JointRowIn next = joint_row_in(rows, j, ri + 1u < count ? ri + 1u : ri);
+        const uint32_t axis = in.s.code & 3u;
+        const bool angular = (in.s.code & kRowAngular) != 0u, motor = (in.s.code & kRowMotor) != 0u;
+        const bool by_twist = (in.s.code & kRowTwist) != 0u || !swing;
+        const V3 unit = basis_axis(axis);
+        PmhAvbdRow row;
+        float current;
+        if (angular) {
+            V3 at;
+            if (motor) {
+                at = log_axis(f.fA, turn, turn_coef, unit);
+                current = comp(turn, axis);
+            } else if (by_twist) {
+                at = log_axis(f.fA, twist, twist_coef, unit);
+                current = comp(twist, axis);
+            } else {
+                at = rotate(f.fA, sub(mul(unit, dot(free_axis, swing_axis)), mul(free_axis, comp(swing_axis, axis))));
+                current = comp(swing_rotation, axis);
+            }
+            set6(row.a, zero, mul(at, -1.0f));
+            set6(row.b, zero, at);
+        } else {
+            const V3 direction = rotate(f.fA, unit);
+            set6(row.a, mul(direction, -1.0f),
+                 add(mul(cross(f.armA, direction), -1.0f), cross(direction, f.error)));
+            set6(row.b, direction, cross(f.armB, direction));
+            current = dot(f.error, direction);
+            if (motor) current = current - in.s.previous;
+        }
+        current = current - in.s.offset;
+        const float linearized = dot6(row.a, da) + dot6(row.b, db);
+        row.lambda = in.lambda; row.penalty = in.penalty; row.stiffness = in.stiffness; row.damping = in.damping;
+        row.lower = in.lower; row.upper = in.upper; row.reference_force = in.reference_force; row.beta = in.beta;
+        row.error = current - in.s.weighted - linearized;
+        row.velocity = motor ? in.velocity : (current - in.s.previous - linearized) / a.dt;
+        if (kVisit == kVisitAccumulate) {
+            jrow_accumulate(blk, row, first, da, db, a.dt);
+            if (!angular) {
+                const V3 dir = {row.b[0], row.b[1], row.b[2]};
+                const float force = jrow_force(row, da, db, a.dt);
+#pragma unroll
+                for (uint32_t c = 0; c < 3; ++c) {
+                    const V3 value = sub(mul(add(mul(dir, comp(arm, c)), mul(arm, comp(dir, c))), 0.5f),
+                                         mul(basis_axis(c), dot(dir, arm)));
+                    const uint32_t d = 3 + c;
+                    blk.h[d * (d + 1) / 2 + d] += fabsf(force) * sqrtf(len2(value));
+                }
+            }
+        } else {
+            if (kVisit == kVisitAdvance) {
+                impulse += fabsf(jrow_force(row, da, db, a.dt)) * a.dt;
+                if (hard_equality(row.stiffness, row.lower, row.upper))
+                    residual = smax(residual, fabsf(row.error + dot6(row.a, da) + dot6(row.b, db)));
+                jrow_advance(row, da, db);
+            } else if (kVisit == kVisitWrite) {
+            } else if (row.stiffness < kMaxPenalty) {
+                row.reference_force = jrow_force(row, da, db, a.dt);
+            } else {
+                const float gap = row.lower == 0.0f ? smin(0.0f, current)
+                                                    : (row.upper == 0.0f ? smax(0.0f, current) : 0.0f);
+                float va[6], vb[6];
+                set6(va, mul(v3(a.tv[st.dense_a]), a.dt), mul(v3(a.tw[st.dense_a]), a.dt));
+                set6(vb, mul(v3(a.tv[st.dense_b]), a.dt), mul(v3(a.tw[st.dense_b]), a.dt));
+                row.reference_force = row.lambda;
+                row.error = dot6(row.a, va) + dot6(row.b, vb) + gap - (motor ? in.velocity * a.dt : 0.0f);
+            }
+            j.rows[ri] = row;
+        }
+        in = next;
+    }
+    return impulse;
+}
+
+// Initialises the rows of an enabled joint (rigid_avbd_visit_joint, :715-926,
+// first visit) and lists them in its step record.
+__device__ __forceinline__ void initialize_joint(const SolveArgs &a, PmhRigidConstraint &j, JointStep &step,
+                                                 const JointEnds &ends) {
     const PmhRigidConstraintOptions &o = j.options;
-    const uint32_t ia = j.dense_a, ib = j.dense_b;
+    const uint32_t ia = j.dense_a, ib = j.dense_b, type = o.type;
+    const bool motor_type = type == kJointMotor;
+    const bool swing = type == kJointHinge || type == kJointPiston || (motor_type && o.motor.angular_enabled != 0u);
+    const bool generic = type == kJointGeneric || type == kJointGenericSpring;
+    JointHead st;
+    st.dense_a = ia;
+    st.dense_b = ib;
+    st.anchor_a = o.local_anchor_a;
+    st.anchor_b = o.local_anchor_b;
+    st.orientation_a = o.local_orientation_a;
+    st.orientation_b = o.local_orientation_b;
+    uint32_t flags = (swing ? kJointSwing : 0u) | (type == kJointHinge ? kJointAxisZ : 0u);
     const PmhRigidBodyState sa = pose_from(a, ia, ends.da, ends.wa), sb = pose_from(a, ib, ends.db, ends.wb);
     const PmhRigidBodyState pa = a.prev[ia], pb = a.prev[ib];
+    const JointFrames now = joint_frames(st, sa, sb), old = joint_frames(st, pa, pb);
     const Q qa = sq(sa.orientation), qb = sq(sb.orientation);
-    const V3 armA = rotate(qa, sv(o.local_anchor_a)), armB = rotate(qb, sv(o.local_anchor_b));
-    const V3 error = sub(add(sv(sb.position), armB), add(sv(sa.position), armA));
-    const V3 old_error = sub(add(sv(pb.position), rotate(sq(pb.orientation), sv(o.local_anchor_b))),
-                             add(sv(pa.position), rotate(sq(pa.orientation), sv(o.local_anchor_a))));
-    const Q fA = qnormalize(qmul(qa, sq(o.local_orientation_a)));
-    const Q fB = qnormalize(qmul(qb, sq(o.local_orientation_b)));
-    const Q ofA = qnormalize(qmul(sq(pa.orientation), sq(o.local_orientation_a)));
-    const Q ofB = qnormalize(qmul(sq(pb.orientation), sq(o.local_orientation_b)));
-    const V3 twist = rel_rotation_vector(fA, fB);
-    const V3 old_twist = rel_rotation_vector(ofA, ofB);
-    const uint32_t type = o.type;
-    const bool swing = type == kJointHinge || type == kJointPiston ||
-                       (type == kJointMotor && o.motor.angular_enabled != 0u);
-    const V3 free_axis = type == kJointHinge ? V3{0.0f, 0.0f, 1.0f} : V3{1.0f, 0.0f, 0.0f};
-    const V3 swing_axis = inv_rotate(fA, rotate(fB, free_axis));
-    const V3 old_swing_axis = inv_rotate(ofA, rotate(ofB, free_axis));
-    const V3 rotation = swing ? cross(free_axis, swing_axis) : twist;
-    const V3 old_rotation = swing ? cross(free_axis, old_swing_axis) : old_twist;
+    const V3 old_twist = rel_rotation_vector(old.fA, old.fB);
+    const V3 free_axis = joint_free_axis(flags);
+    const V3 old_rotation = swing ? cross(free_axis, inv_rotate(old.fA, rotate(old.fB, free_axis))) : old_twist;
+    st.old_relative = pq(relative_quaternion(old.fA, old.fB, true));
     const PmhBodyParameters Pa = a.P[ia], Pb = a.P[ib];
     const float linear_penalty = pair_stiffness(Pa, Pb, a.dt);
-    const bool generic = type == kJointGeneric || type == kJointGenericSpring;
-    const bool motor_type = type == kJointMotor;
-    const V3 zero = {0.0f, 0.0f, 0.0f};
+    uint32_t count = 0;
+    // `current` is measured against `offset`; `previous` is its value at the
+    // step's start (for a linear motor the measure itself, which its travel
+    // counts from).
+    auto row = [&](uint32_t code, float offset, float previous, float penalty, float stiffness, float damping,
+                   float lower, float upper, float stabilization) {
+        if (count >= 18u) return;
+        const uint32_t ri = count++;
+        JointRowStep s;
+        s.code = code;
+        s.offset = offset;
+        s.previous = previous;
+        s.weighted = stiffness < kMaxPenalty || (code & kRowMotor) != 0u ? 0.0f : stabilization * previous;
+        step.rows[ri] = s;
+        PmhAvbdRow r = j.rows[ri];
+        if (!(r.penalty > kMinPenalty)) r.penalty = penalty;
+        warm_start(r.lambda, r.penalty, stiffness);
+        if (stiffness < kMaxPenalty) r.lambda = 0.0f;
+        r.beta = penalty * ((code & kRowAngular) != 0u ? 10.0f : 100.0f);
+        r.reference_force = 0.0f;
+        r.stiffness = stiffness;
+        r.damping = damping;
+        r.lower = lower;
+        r.upper = upper;
+        j.rows[ri] = r;
+    };
+    // An angular equality starts from at least this penalty.
+    auto floor_penalty = [&](float penalty) {
+        if (count < 18u) j.rows[count].penalty = smax(j.rows[count].penalty, penalty / kGamma);
+    };
+#pragma unroll 1
     for (uint32_t axis = 0; axis < 3; ++axis) {
-        const V3 direction = rotate(fA, basis_axis(axis));
-        const V3 old_direction = rotate(ofA, basis_axis(axis));
+        const V3 direction = rotate(now.fA, basis_axis(axis));
+        const V3 old_direction = rotate(old.fA, basis_axis(axis));
+#pragma unroll 1
         for (uint32_t av = 0; av < 2; ++av) {
             const bool angular = av != 0;
+            const uint32_t code = axis | (angular ? kRowAngular : 0u);
             const bool lock = angular
                 ? type == kJointFixed || type == kJointSlider || (type == kJointHinge && axis != 2u) ||
                       (type == kJointPiston && axis != 0u) ||
@@ -1719,102 +1840,62 @@ __device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstra
                       (motor_type && (axis != 0u || o.motor.linear_enabled == 0u));
             const PmhJointLimits &limits = angular ? o.angular_limits : o.linear_limits;
             const PmhJointSprings &springs = angular ? o.angular_springs : o.linear_springs;
-            const float current = angular ? comp(rotation, axis) : dot(error, direction);
-            const float old_current = angular ? comp(old_rotation, axis) : dot(old_error, old_direction);
-            const V3 angular_axis = swing
-                ? rotate(fA, sub(mul(basis_axis(axis), dot(free_axis, swing_axis)),
-                                 mul(free_axis, comp(swing_axis, axis))))
-                : log_axis(fA, twist, axis);
-            JointRowArgs r;
-            if (angular) {
-                set6(r.ja, zero, mul(angular_axis, -1.0f));
-                set6(r.jb, zero, angular_axis);
-            } else {
-                set6(r.ja, mul(direction, -1.0f), add(mul(cross(armA, direction), -1.0f), cross(direction, error)));
-                set6(r.jb, direction, cross(armB, direction));
-            }
+            const float old_current = angular ? comp(old_rotation, axis) : dot(old.error, old_direction);
             const float penalty = angular
                 ? 1.0f / (smax(dot(direction, add(iiw(Pa, qa, direction), iiw(Pb, qb, direction))), 1.0e-6f) *
                           a.dt * a.dt)
                 : linear_penalty;
             const float lock_penalty = angular
-                ? smax(penalty, 2.0f * linear_penalty * smax(len2(cross(direction, armA)), len2(cross(direction, armB))))
+                ? smax(penalty, 2.0f * linear_penalty * smax(len2(cross(direction, now.armA)),
+                                                             len2(cross(direction, now.armB))))
                 : penalty;
-            r.angular = angular;
-            r.motor = false;
-            r.motor_speed = 0.0f;
-            r.curv_a = add(error, armA);
-            r.curv_b = armB;
             if (lock) {
-                if (visit == kVisitInitialize && angular && index < 18u)
-                    j.rows[index].penalty = smax(j.rows[index].penalty, lock_penalty / kGamma);
-                r.current = current; r.previous = old_current; r.penalty = lock_penalty;
-                r.stiffness = kMaxPenalty; r.damping = 0.0f; r.lower = -kMaxPenalty; r.upper = kMaxPenalty;
-                r.stabilization = kAlpha;
-                visit_joint_row(a, j, blk, index, impulse, first, r, visit, ends);
+                if (angular) floor_penalty(lock_penalty);
+                if (angular && !swing) flags |= kJointTwist;
+                row(code, 0.0f, old_current, lock_penalty, kMaxPenalty, 0.0f, -kMaxPenalty, kMaxPenalty, kAlpha);
             }
             const bool free_limit = angular ? (type == kJointHinge && axis == 2u) || (type == kJointPiston && axis == 0u)
                                             : (type == kJointSlider || type == kJointPiston) && axis == 0u;
             if ((generic || free_limit) && (limits.axes & (1u << axis)) != 0u) {
-                JointRowArgs l = r;
-                const float limit_current = angular ? comp(twist, axis) : current;
-                const float old_limit_current = angular ? comp(old_twist, axis) : old_current;
-                if (angular) {
-                    const V3 limit_axis = log_axis(fA, twist, axis);
-                    set6(l.ja, zero, mul(limit_axis, -1.0f));
-                    set6(l.jb, zero, limit_axis);
-                }
+                const uint32_t limit = code | kRowTwist;
+                const float at = angular ? comp(old_twist, axis) : old_current;
                 const float lower = comp(sv(limits.lower), axis), upper = comp(sv(limits.upper), axis);
-                l.stiffness = kMaxPenalty;
-                l.damping = 0.0f;
+                if (angular) flags |= kJointTwist;
                 if (lower == upper) {
                     const float equal_penalty = angular && generic ? lock_penalty : penalty;
-                    if (visit == kVisitInitialize && angular && generic && index < 18u)
-                        j.rows[index].penalty = smax(j.rows[index].penalty, equal_penalty / kGamma);
-                    l.current = limit_current - lower; l.previous = old_limit_current - lower;
-                    l.penalty = equal_penalty; l.lower = -kMaxPenalty; l.upper = kMaxPenalty;
-                    l.stabilization = kAlpha;
-                    visit_joint_row(a, j, blk, index, impulse, first, l, visit, ends);
+                    if (angular && generic) floor_penalty(equal_penalty);
+                    row(limit, lower, at - lower, equal_penalty, kMaxPenalty, 0.0f, -kMaxPenalty, kMaxPenalty, kAlpha);
                 } else if (lower < upper) {
-                    l.current = limit_current - upper; l.previous = smax(old_limit_current - upper, 0.0f);
-                    l.penalty = penalty; l.lower = 0.0f; l.upper = kMaxPenalty;
-                    l.stabilization = kLimitStabilization;
-                    visit_joint_row(a, j, blk, index, impulse, first, l, visit, ends);
-                    l.current = limit_current - lower; l.previous = smin(old_limit_current - lower, 0.0f);
-                    l.lower = -kMaxPenalty; l.upper = 0.0f;
-                    visit_joint_row(a, j, blk, index, impulse, first, l, visit, ends);
+                    row(limit, upper, smax(at - upper, 0.0f), penalty, kMaxPenalty, 0.0f, 0.0f, kMaxPenalty,
+                        kLimitStabilization);
+                    row(limit, lower, smin(at - lower, 0.0f), penalty, kMaxPenalty, 0.0f, -kMaxPenalty, 0.0f,
+                        kLimitStabilization);
                 }
             }
             if (type == kJointGenericSpring && (springs.axes & (1u << axis)) != 0u) {
-                JointRowArgs sr = r;
-                sr.current = current; sr.previous = old_current; sr.penalty = penalty;
-                sr.stiffness = comp(sv(springs.stiffness), axis); sr.damping = comp(sv(springs.damping), axis);
-                sr.lower = -kMaxPenalty; sr.upper = kMaxPenalty; sr.stabilization = kAlpha;
-                visit_joint_row(a, j, blk, index, impulse, first, sr, visit, ends);
+                if (angular) flags |= kJointTwist;
+                row(code, 0.0f, old_current, penalty, comp(sv(springs.stiffness), axis),
+                    comp(sv(springs.damping), axis), -kMaxPenalty, kMaxPenalty, kAlpha);
             }
             if (motor_type && axis == 0u && (angular ? o.motor.angular_enabled != 0u : o.motor.linear_enabled != 0u)) {
                 const float speed = angular ? o.motor.angular_target_velocity : o.motor.linear_target_velocity;
                 const float bound = (angular ? o.motor.angular_maximum_impulse : o.motor.linear_maximum_impulse) / a.dt;
-                const Q rel = relative_quaternion(fA, fB, true);
-                const Q old_rel = relative_quaternion(ofA, ofB, true);
-                const V3 motor_rotation = rel_rotation_vector({0.0f, 0.0f, 0.0f, 1.0f},
-                                                              relative_quaternion(old_rel, rel, false));
-                JointRowArgs mr = r;
-                if (angular) {
-                    const V3 motor_axis = log_axis(fA, motor_rotation, axis);
-                    set6(mr.ja, zero, mul(motor_axis, -1.0f));
-                    set6(mr.jb, zero, motor_axis);
-                }
-                const float travel = angular ? comp(motor_rotation, axis) : current - old_current;
-                mr.current = travel - speed * a.dt; mr.previous = 0.0f; mr.penalty = penalty;
-                mr.stiffness = kMaxPenalty; mr.damping = 0.0f; mr.lower = -bound; mr.upper = bound;
-                mr.motor = true; mr.motor_speed = speed; mr.stabilization = kAlpha;
-                visit_joint_row(a, j, blk, index, impulse, first, mr, visit, ends);
+                if (angular) flags |= kJointMotorTurn;
+                if (count < 18u) j.rows[count].velocity = speed;
+                row(code | kRowMotor, speed * a.dt, old_current, penalty, kMaxPenalty, 0.0f, -bound, bound, kAlpha);
             }
         }
     }
-    if (visit == kVisitInitialize) j.avbd_count = index;
-    return impulse;
+    st.flags = flags;
+    st.count = count;
+    st.pad[0] = st.pad[1] = 0u;
+    step.head = st;
+    j.avbd_count = count;
+    if (count == 0u) return;
+    // The rows as the reference leaves them here.
+    Block scratch;
+    float unused = 0.0f;
+    visit_joint<kVisitWrite>(a, j, st, step.rows, sa, sb, joint_row_in(step.rows, j, 0), ends, scratch, true, unused);
 }
 
 // The joint rows of body i in its list order, added to its block: the
@@ -1824,92 +1905,124 @@ __device__ __forceinline__ float visit_joint(const SolveArgs &a, PmhRigidConstra
 // group (the k-th enabled joint of the list to lane k mod L) and added to
 // that lane's partial block before the group reduction.
 // The body's own displacement and rotation delta come in registers, the
-// other end's from its mailbox where this sweep has moved it already.
-template <bool kFlow>
+// other end's from its mailbox where this sweep has moved it already; the
+// rest of a joint is loaded before that wait.
+template <bool kFlow, int L>
 __device__ __forceinline__ void body_joint_rows(const SolveArgs &a, uint32_t i, uint32_t phase, Block &blk,
-                                                uint32_t sub_lane, uint32_t L, const float *dI, float wI) {
-    uint32_t pos = 0;
-    for (uint32_t e = a.jstart[i]; e < a.jstart[i + 1]; ++e) {
-        PmhRigidConstraint &j = a.joints[a.jadj[e]];
-        if (j.state_enabled == 0u) continue;
-        if (pos++ % L != sub_lane) continue;
-        const bool first = i == j.dense_a;
-        const uint32_t other = first ? j.dense_b : j.dense_a;
-        float dO[6], wO = 1.0f;
-        // Bodies without a colour hold kInvalid: never lower.
-        if (kFlow && a.color[other] < a.color[i]) {
-            const __amdgpu_buffer_rsrc_t box = flow_box(a);
-            flow_take(a, box, other, dO);
-            if (phase == 0u) wO = flow_take_w(a, box, other);
-        } else {
-            load_disp(a.disp, other, dO);
-            if (phase == 0u) wO = a.dq[other].w;
+                                                uint32_t lane, const float *dI, float wI) {
+    const uint32_t b = a.jstart[i], e = a.jstart[i + 1];
+    const uint32_t sub_lane = lane % L, lane0 = lane - sub_lane;
+    const uint64_t group = (L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull) << lane0;
+    const float4 tp = a.tpos[i], tq = a.tq[i];
+    uint32_t done = 0;
+    for (uint32_t base = b; base < e; base += L) {
+        const uint32_t p = base + sub_lane;
+        uint2 ent = make_uint2(0u, 0u);
+        bool on = false;
+        if (p < e) {
+            ent = a.jent[p];
+            on = a.joints[ent.x & ~kSideFirst].state_enabled != 0u;
         }
+        uint64_t mask = (__ballot(on) & group) >> lane0;
+        const uint32_t enabled = uint32_t(__popcll(mask)), skip = (sub_lane - done) % L;
+        done += enabled;
+        // This lane's joint: the skip-th enabled one of the chunk.
+        for (uint32_t s = 0; s < skip; ++s) mask &= mask - 1ull;
+        const int from = int(lane0) + (mask ? __builtin_ctzll(mask) : 0);
+        ent.x = uint32_t(__shfl(int(ent.x), from, 64));
+        ent.y = uint32_t(__shfl(int(ent.y), from, 64));
+        if (mask == 0ull) continue;
+        const bool first = (ent.x & kSideFirst) != 0u;
+        const uint32_t k = ent.x & ~kSideFirst, other = ent.y & kEntryBody;
+        PmhRigidConstraint &j = a.joints[k];
+        const bool wait = kFlow && (ent.y & kEntryLower) != 0u;
+        float dO[7];
         JointEnds ends;
+        auto pair_ends = [&]() {
 #pragma unroll
-        for (int q = 0; q < 6; ++q) {
-            ends.da[q] = first ? dI[q] : dO[q];
-            ends.db[q] = first ? dO[q] : dI[q];
-        }
-        ends.wa = first ? wI : wO;
-        ends.wb = first ? wO : wI;
+            for (int q = 0; q < 6; ++q) {
+                ends.da[q] = first ? dI[q] : dO[q];
+                ends.db[q] = first ? dO[q] : dI[q];
+            }
+            ends.wa = first ? wI : dO[6];
+            ends.wb = first ? dO[6] : wI;
+        };
         if (phase == 0u) {
-            visit_joint(a, j, blk, first, kVisitAccumulate, ends);
+            const JointRowStep *rows = a.jstep[k].rows;
+            const JointHead head = a.jstep[k].head;
+            const JointRowIn in = joint_row_in(rows, j, 0);
+            const float4 op = a.tpos[other], oq = a.tq[other];
+            if (wait) {
+                flow_take<true>(a, flow_box(a), other, dO);
+            } else {
+                load_disp(a.disp, other, dO);
+                dO[6] = a.dq[other].w;
+            }
+            pair_ends();
+            float unused = 0.0f;
+            const PmhRigidBodyState sI = pose_at(tp, tq, {dI[0], dI[1], dI[2]},
+                                                 {0.5f * dI[3], 0.5f * dI[4], 0.5f * dI[5], wI});
+            const PmhRigidBodyState sO = pose_at(op, oq, {dO[0], dO[1], dO[2]},
+                                                 {0.5f * dO[3], 0.5f * dO[4], 0.5f * dO[5], dO[6]});
+            visit_joint<kVisitAccumulate>(a, j, head, rows, first ? sI : sO, first ? sO : sI, in, ends, blk, first,
+                                          unused);
             continue;
         }
-        for (uint32_t r = 0; r < j.avbd_count; ++r) {
-            const PmhAvbdRow row = j.rows[r];
+        const uint32_t count = j.avbd_count;
+        PmhAvbdRow row = j.rows[0];
+        if (wait) flow_take(a, flow_box(a), other, dO);
+        else load_disp(a.disp, other, dO);
+        dO[6] = 1.0f;
+        pair_ends();
+#pragma unroll 1
+        for (uint32_t r = 0; r < count; ++r) {
+            const PmhAvbdRow next = j.rows[r + 1u < count ? r + 1u : r];
             if (row.stiffness >= kMaxPenalty) jrow_accumulate(blk, row, first, ends.da, ends.db, a.dt);
+            row = next;
         }
     }
 }
 
 // Joint part of advance_duals (solve.slang:566-614): dual updates, the
-// applied impulse and breaking, one thread per joint.
-__device__ void advance_joint(const SolveArgs &a, uint32_t k, uint32_t phase) {
+// applied impulse and breaking, one thread per joint.  Returns the residual
+// of the joint's hard equality rows: |C| at the current displacements.
+__device__ float advance_joint(const SolveArgs &a, uint32_t k, uint32_t phase) {
     PmhRigidConstraint &j = a.joints[k];
-    if (j.avbd_count == 0u || j.state_enabled == 0u) return;
-    const uint32_t ia = j.dense_a, ib = j.dense_b;
-    if (phase != 0u && a.impact[ia] == 0u && a.impact[ib] == 0u) return;
-    float impulse = 0.0f;
+    const JointHead head = a.jstep[k].head;
+    const JointRowStep *rows = a.jstep[k].rows;
+    const uint32_t ia = head.dense_a, ib = head.dense_b;
+    const JointEnds ends = joint_ends(a, ia, ib);
+    float impulse = 0.0f, residual = 0.0f;
     if (phase == 0u) {
         Block scratch;
-        block_zero(scratch);
-        impulse = visit_joint(a, j, scratch, true, kVisitAdvance, joint_ends(a, ia, ib));
+        impulse = visit_joint<kVisitAdvance>(a, j, head, rows, pose_from(a, ia, ends.da, ends.wa),
+                                             pose_from(a, ib, ends.db, ends.wb), joint_row_in(rows, j, 0), ends,
+                                             scratch, true, residual);
     } else {
-        float da[6], db[6];
-        load_disp(a.disp, ia, da);
-        load_disp(a.disp, ib, db);
-        for (uint32_t r = 0; r < j.avbd_count; ++r) {
-            PmhAvbdRow row = j.rows[r];
+        const float *da = ends.da, *db = ends.db;
+        const uint32_t count = j.avbd_count;
+        PmhAvbdRow row = j.rows[0];
+#pragma unroll 1
+        for (uint32_t r = 0; r < count; ++r) {
+            const PmhAvbdRow next = j.rows[r + 1u < count ? r + 1u : r];
             impulse += fabsf(row.stiffness < kMaxPenalty ? row.reference_force : jrow_force(row, da, db, a.dt)) * a.dt;
+            if (hard_equality(row.stiffness, row.lower, row.upper))
+                residual = smax(residual, fabsf(row.error + dot6(row.a, da) + dot6(row.b, db)));
             if (row.stiffness >= kMaxPenalty) {
                 jrow_advance(row, da, db);
-                j.rows[r] = row;
+                j.rows[r].lambda = row.lambda;
+                j.rows[r].penalty = row.penalty;
             }
+            row = next;
         }
     }
     j.applied_impulse = impulse;
     if (j.options.breaking_impulse_threshold > 0.0f && impulse > j.options.breaking_impulse_threshold) {
         j.state_broken = 1u;
         j.state_enabled = 0u;
+        return 0.0f;
     }
-}
-
-// Residual of a joint's hard equality rows: |C| at the current
-// displacements.
-__device__ float joint_residual(const SolveArgs &a, const PmhRigidConstraint &j) {
-    if (j.avbd_count == 0u || j.state_enabled == 0u) return 0.0f;
-    float da[6], db[6];
-    load_disp(a.disp, j.dense_a, da);
-    load_disp(a.disp, j.dense_b, db);
-    float r = 0.0f;
-    for (uint32_t k = 0; k < j.avbd_count; ++k) {
-        const PmhAvbdRow &row = j.rows[k];
-        if (row.stiffness < kMaxPenalty || row.lower != -kMaxPenalty || row.upper != kMaxPenalty) continue;
-        r = smax(r, fabsf(row.error + dot6(row.a, da) + dot6(row.b, db)));
-    }
-    return r;
+    return residual;
 }
 
 // kFlagSlipping: the point slid at the last dual update (to-residual mode,
@@ -2347,8 +2460,7 @@ __global__ void __launch_bounds__(256) k_stage_duals(SolveArgs a, uint32_t phase
             const PmhRigidConstraint &j = a.joints[k];
             if (j.avbd_count == 0u || j.state_enabled == 0u) continue;
             if (phase != 0u && a.impact[j.dense_a] == 0u && a.impact[j.dense_b] == 0u) continue;
-            advance_joint(a, k, phase);
-            r.add(joint_residual(a, j));
+            r.add(advance_joint(a, k, phase));
         }
         if (it < kResidualSlots) residual_commit(a.log, phase * kResidualSlots + it, r);
     }
@@ -2363,8 +2475,7 @@ __global__ void __launch_bounds__(256) k_stage_joint_duals(SolveArgs a, uint32_t
         const PmhRigidConstraint &j = a.joints[k];
         if (j.avbd_count == 0u || j.state_enabled == 0u) continue;
         if (phase != 0u && a.impact[j.dense_a] == 0u && a.impact[j.dense_b] == 0u) continue;
-        advance_joint(a, k, phase);
-        r.add(joint_residual(a, j));
+        r.add(advance_joint(a, k, phase));
     }
     if (it < kResidualSlots) residual_commit(a.log, phase * kResidualSlots + it, r);
 }
@@ -2413,9 +2524,14 @@ __global__ void k_stage_velocity_errors(SolveArgs a, const uint32_t *c_flags) {
         PmhRigidConstraint &j = a.joints[k];
         if (j.avbd_count == 0u || j.state_enabled == 0u) continue;
         if (a.impact[j.dense_a] == 0u && a.impact[j.dense_b] == 0u) continue;
+        const JointHead head = a.jstep[k].head;
+        const JointRowStep *rows = a.jstep[k].rows;
+        const JointEnds ends = joint_ends(a, j.dense_a, j.dense_b);
         Block scratch;
-        block_zero(scratch);
-        visit_joint(a, j, scratch, true, kVisitImpact, joint_ends(a, j.dense_a, j.dense_b));
+        float unused = 0.0f;
+        visit_joint<kVisitImpact>(a, j, head, rows, pose_from(a, j.dense_a, ends.da, ends.wa),
+                                  pose_from(a, j.dense_b, ends.db, ends.wb), joint_row_in(rows, j, 0), ends, scratch,
+                                  true, unused);
     }
 }
 __global__ void k_stage_velocity_jacobians(SolveArgs a) {
@@ -2516,9 +2632,7 @@ __global__ void k_joint_init(SolveArgs a) {
     j.dense_a = ia.index < a.n && ia.generation == 1u ? ia.index : kInvalid;
     j.dense_b = ib.index < a.n && ib.generation == 1u ? ib.index : kInvalid;
     if (j.dense_a == kInvalid || j.dense_b == kInvalid) return;
-    Block scratch;
-    block_zero(scratch);
-    visit_joint(a, j, scratch, true, kVisitInitialize, joint_ends(a, j.dense_a, j.dense_b));
+    initialize_joint(a, j, a.jstep[k], joint_ends(a, j.dense_a, j.dense_b));
 }
 
 // The joints' iteration floor: the legacy profile without a requested
@@ -2543,54 +2657,75 @@ __global__ void k_joint_budget(SolveArgs a, StepCounters *ctr) {
 // wavefront kernel below.
 template <int kPass>
 __global__ void k_joint_lists(SolveArgs a, const uint32_t *jlist_start, const uint32_t *jlist, uint32_t *jdeg,
-                              uint32_t *jadj) {
+                              uint32_t *jadj, uint32_t *joint_head) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.n) return;
     const uint32_t b = jlist_start[i], e = jlist_start[i + 1];
     if (e - b > 64u) return;
-    uint32_t o = kPass == 1 ? a.jstart[i] : 0u;
+    uint32_t o = kPass == 1 ? a.jstart[i] : 0u, head = kInvalid;
     for (uint32_t p = b; p < e; ++p) {
         const uint32_t k = jlist[p];
         if (a.joints[k].avbd_count == 0u) continue;
+        if (head == kInvalid) head = k;
         if (kPass == 1) jadj[o] = k;
         ++o;
     }
+    if (kPass == 1) joint_head[i] = head;
     if (kPass == 0) jdeg[i] = o;
 }
 
 template <int kPass>
 __global__ void __launch_bounds__(64) k_joint_lists_heavy(SolveArgs a, const uint32_t *heavy, uint32_t nheavy,
                                                           const uint32_t *jlist_start, const uint32_t *jlist,
-                                                          uint32_t *jdeg, uint32_t *jadj) {
+                                                          uint32_t *jdeg, uint32_t *jadj, uint32_t *joint_head) {
     const uint32_t lane = threadIdx.x;
     for (uint32_t h = blockIdx.x; h < nheavy; h += gridDim.x) {
         const uint32_t i = heavy[h];
         const uint32_t b = jlist_start[i], e = jlist_start[i + 1];
-        uint32_t o = kPass == 1 ? a.jstart[i] : 0u;
+        uint32_t o = kPass == 1 ? a.jstart[i] : 0u, head = kInvalid;
         for (uint32_t base = b; base < e; base += 64) {
             const uint32_t p = base + lane;
             const bool keep = p < e && a.joints[jlist[p]].avbd_count != 0u;
             const uint64_t mask = __ballot(keep);
+            if (kPass == 1 && head == kInvalid && mask) head = jlist[base + uint32_t(__builtin_ctzll(mask))];
             if (kPass == 1 && keep) jadj[o + __popcll(mask & ((1ull << lane) - 1ull))] = jlist[p];
             o += uint32_t(__popcll(mask));
         }
         if (kPass == 0 && lane == 0) jdeg[i] = o;
+        if (kPass == 1 && lane == 0) joint_head[i] = head;
     }
 }
 
-// List links of the reference layout (push-front in joint order, so each
-// body's list runs in descending joint index) from the sorted segments.
-__global__ void k_joint_links(SolveArgs a, uint32_t *joint_head) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.n) return;
-    const uint32_t b = a.jstart[i], e = a.jstart[i + 1];
-    joint_head[i] = b < e ? a.jadj[b] : kInvalid;
-    for (uint32_t p = b; p < e; ++p) {
-        PmhRigidConstraint &j = a.joints[a.jadj[p]];
-        const uint32_t next = p + 1 < e ? a.jadj[p + 1] : kInvalid;
-        if (j.dense_a == i) j.avbd_next_a = next;
-        else j.avbd_next_b = next;
-    }
+// Joint ends in list order, one thread per end: the joint with the end's
+// side, and the other body with a flag where it is not dynamic.  And the list
+// links of the reference layout (push-front in joint order, so each body's
+// list runs in descending joint index).  By bodies, the thread of an anchor
+// with 1024 joints alone walked all of them: 235 us of chains of 65536 links,
+// now 6 us.
+__global__ void k_joint_entries(SolveArgs a) {
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= a.jstart[a.n]) return;
+    const uint32_t k = a.jadj[p];
+    PmhRigidConstraint &j = a.joints[k];
+    const uint32_t ia = j.dense_a, ib = j.dense_b;
+    const bool first = p >= a.jstart[ia] && p < a.jstart[ia + 1];
+    const uint32_t i = first ? ia : ib, other = first ? ib : ia;
+    a.jent[p] = make_uint2(k | (first ? kSideFirst : 0u), other | (a.P[other].motion == kDynamic ? 0u : kEntryFixed));
+    const uint32_t next = p + 1 < a.jstart[i + 1] ? a.jadj[p + 1] : kInvalid;
+    if (next == k) return;   // both ends on one body: the second entry's link stands
+    if (first) j.avbd_next_a = next;
+    else j.avbd_next_b = next;
+}
+
+// Once the colours stand: marks the ends whose other body has a lower one.
+// Bodies without a colour hold kInvalid: never lower.
+__global__ void k_joint_lower(SolveArgs a) {
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= a.jstart[a.n]) return;
+    const uint2 ent = a.jent[p];
+    const uint32_t k = ent.x & ~kSideFirst, other = ent.y & kEntryBody;
+    const uint32_t i = (ent.x & kSideFirst) != 0u ? a.joints[k].dense_a : a.joints[k].dense_b;
+    if (a.color[other] < a.color[i]) a.jent[p].y = ent.y | kEntryLower;
 }
 
 __global__ void k_joint_hook(SolveArgs a, uint32_t *parent) {
@@ -2842,7 +2977,10 @@ void KernelTimer::release() {
 
 PmhResult Solver::reserve_joints(uint32_t count) {
     PmhResult r = PMH_SUCCESS;
-    if ((r = jadj.reserve(2 * size_t(std::max<uint32_t>(1, count)))) != PMH_SUCCESS) return r;
+    const size_t ends = 2 * size_t(std::max<uint32_t>(1, count));
+    if ((r = jadj.reserve(ends)) != PMH_SUCCESS || (r = jent.reserve(ends)) != PMH_SUCCESS ||
+        (r = jstep.reserve(std::max<uint32_t>(1, count))) != PMH_SUCCESS)
+        return r;
     return PMH_SUCCESS;
 }
 
@@ -2949,7 +3087,8 @@ void Solver::release() {
     inertia.release(); prev_vel.release(); color.release(); parent.release(); impact.release();
     deg.release(); adj_start.release(); adj_cursor.release(); color_bodies.release();
     bp_start.release(); anchored.release(); mean.release(); members.release(); mean_list.release(); flow.release();
-    jdeg.release(); jstart.release(); jcursor.release(); joint_head.release(); jadj.release(); code.release(); ab.release();
+    jdeg.release(); jstart.release(); jcursor.release(); joint_head.release(); jadj.release();
+    jent.release(); jstep.release(); code.release(); ab.release();
     m_count.release(); m_start.release(); m_slot.release(); m_impact.release(); m_face.release();
     m_init_rel.release(); adj.release(); tri_list.release(); face_list.release(); c_np.release(); c_pt.release(); c_aa.release();
     c_ab.release(); c_err.release(); c_lam.release(); c_pen.release(); c_acc.release();
@@ -3033,6 +3172,8 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
     a.nj = v.nj;
     a.jstart = v.jstart.p;
     a.jadj = v.jadj.p;
+    a.jent = v.jent.p;
+    a.jstep = v.jstep.p;
     a.prev = previous;
     a.color = v.color.p;
     a.flow = v.flow.p;
@@ -3042,6 +3183,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
     a.tol = sp.tolerance;
     a.c_flags = v.c_flags.p;
     const uint32_t jg = grid_for(std::max<uint32_t>(1, v.nj), 256, 0xffffffffu);
+    const uint32_t eg = grid_for(std::max<uint32_t>(1, 2 * v.nj), 256, 0xffffffffu);   // one thread per joint end
     k_schedule_init<<<1, 64, 0, s>>>(v.schedule.p, ctr, budget, sp.profile, sp.base_iterations,
                                      sp.reset_status ? 1u : 0u);
     k_residual_reset<<<32, 256, 0, s>>>(v.residual.p);
@@ -3077,17 +3219,17 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
         // Joint lists, geometry_constraints.slang:1462-1475.
         if (!realtime && sp.requested_iterations == 0u) k_joint_budget<<<jg, 256, 0, s>>>(a, ctr);
         const uint32_t hg = std::max<uint32_t>(1, std::min<uint32_t>(v.nheavy, 4096));
-        k_joint_lists<0><<<bg, 256, 0, s>>>(a, v.jlist_start, v.jlist, v.jdeg.p, v.jadj.p);
+        k_joint_lists<0><<<bg, 256, 0, s>>>(a, v.jlist_start, v.jlist, v.jdeg.p, v.jadj.p, v.joint_head.p);
         if (v.nheavy)
             k_joint_lists_heavy<0><<<hg, 64, 0, s>>>(a, v.jheavy, v.nheavy, v.jlist_start, v.jlist, v.jdeg.p,
-                                                     v.jadj.p);
+                                                     v.jadj.p, v.joint_head.p);
         r = exclusive_scan(s, v.jdeg.p, v.jstart.p, n, nullptr, nullptr, v.scan_tmp);
         if (r != PMH_SUCCESS) return r;
-        k_joint_lists<1><<<bg, 256, 0, s>>>(a, v.jlist_start, v.jlist, v.jdeg.p, v.jadj.p);
+        k_joint_lists<1><<<bg, 256, 0, s>>>(a, v.jlist_start, v.jlist, v.jdeg.p, v.jadj.p, v.joint_head.p);
         if (v.nheavy)
             k_joint_lists_heavy<1><<<hg, 64, 0, s>>>(a, v.jheavy, v.nheavy, v.jlist_start, v.jlist, v.jdeg.p,
-                                                     v.jadj.p);
-        k_joint_links<<<bg, 256, 0, s>>>(a, v.joint_head.p);
+                                                     v.jadj.p, v.joint_head.p);
+        k_joint_entries<<<eg, 256, 0, s>>>(a);
     }
     // Labelling rounds before the pass over all edges, each worth its two
     // launches while many roots are left (heap of 32768 bodies: the edge pass
@@ -3112,18 +3254,19 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
     // contact and joint ends per body), one wavefront per body otherwise.
     if (v.neighbour_hint < kLaneColorNeighbours) {
         const uint32_t blocks = std::max<uint32_t>(1, std::min<uint32_t>((n + 255) / 256, 4 * device_compute_units()));
-        k_color_lane<<<blocks, 256, 0, s>>>(n, P, v.ab.p, v.adj_start.p, v.adj.p, v.color.p, v.jstart.p, v.jadj.p,
-                                            v.nj ? v.joints : nullptr, ctr, sp.color_wait_limit);
+        k_color_lane<<<blocks, 256, 0, s>>>(n, P, v.ab.p, v.adj_start.p, v.adj.p, v.color.p, v.jstart.p, v.jent.p,
+                                            v.nj != 0, ctr, sp.color_wait_limit);
     } else {
         const uint32_t blocks = std::max<uint32_t>(
             1, std::min<uint32_t>((n + kColorWaveBlock - 1) / kColorWaveBlock, 2 * device_compute_units()));
-        k_color_wave<<<blocks, 64 * kColorWaveBlock, 0, s>>>(n, P, v.ab.p, v.adj_start.p, v.adj.p, v.color.p, v.jstart.p, v.jadj.p,
-                                            v.nj ? v.joints : nullptr, ctr, sp.color_wait_limit);
+        k_color_wave<<<blocks, 64 * kColorWaveBlock, 0, s>>>(n, P, v.ab.p, v.adj_start.p, v.adj.p, v.color.p, v.jstart.p, v.jent.p,
+                                            v.nj != 0, ctr, sp.color_wait_limit);
     }
     PMH_CHECK(hipMemsetAsync(v.color_count.p, 0, sizeof(uint32_t) * (kMaxColors + 1), s));
     k_color_count<<<bg, 256, 0, s>>>(n, v.color.p, v.color_count.p);
     k_color_scan<<<1, 64, 0, s>>>(v.color_count.p, v.color_start.p, ctr, v.color_bodies.p, 64u / sp.lanes);
     k_color_place<<<bg, 256, 0, s>>>(n, v.color.p, v.color_start.p, v.color_count.p, v.color_bodies.p);
+    if (v.nj) k_joint_lower<<<eg, 256, 0, s>>>(a);
     // colour-ordered point lists (deg array reused as the per-position count)
     // The degree array is free again once the adjacency is built (the
     // fill cursor keeps each body's degree): it holds the point counts.

@@ -214,6 +214,35 @@ __host__ __device__ inline float residual_rms(unsigned long long sum, uint32_t c
     return count ? float(sqrt(double(sum) / 1099511627776.0 / double(count))) : 0.0f;
 }
 
+// What a joint's visits within one step share: its frames, and the rows that
+// its type and options give with what the step's start decides of each.
+enum : uint32_t {
+    kRowAngular = 4u,                    // with the axis in the low two bits
+    kRowTwist = 8u,                      // a limit: measured on the twist, also where the joint swings
+    kRowMotor = 16u,
+};
+enum : uint32_t {
+    kJointSwing = 1u,                    // the angular rows keep the free axis
+    kJointAxisZ = 2u,                    // the free axis is z (else x)
+    kJointTwist = 4u,                    // some row needs the rotation between the frames
+    kJointMotorTurn = 8u,                // some row needs the rotation since the step's start
+};
+struct alignas(16) JointRowStep {
+    uint32_t code;
+    float offset, previous;
+    float weighted;                      // the stabilised part of `previous`; 0 for soft rows
+};
+struct alignas(16) JointHead {
+    uint32_t dense_a, dense_b, flags, count;
+    PmhQuat orientation_a, orientation_b, old_relative;
+    PmhVec3 anchor_a, anchor_b;
+    uint32_t pad[2];
+};
+struct alignas(16) JointStep {
+    JointHead head;
+    JointRowStep rows[18];
+};
+
 // Everything AVBD needs after the narrowphase: per-body, per-pair and
 // per-point solver state.  Shared by the world step and the kernel seam.
 struct Solver {
@@ -233,6 +262,8 @@ struct Solver {
     uint32_t nj = 0;
     bool hinges = false;                 // some joint is a hinge (anchor projection)
     DBuf<uint32_t> jdeg, jstart, jcursor, jadj, joint_head;
+    DBuf<uint2> jent;                    // jadj's ends: joint and side, other body and flags
+    DBuf<JointStep> jstep;               // one per joint
     // Every body's candidate joints (alive, both ids valid) in descending
     // joint index, built by the owner at upload; each step keeps the joints
     // that initialised rows.  Bodies with more than 64 are listed apart

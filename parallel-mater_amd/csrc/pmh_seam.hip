@@ -230,7 +230,7 @@ static PmhResult seam_joints_in(Solver &v, SeamJoints &sj, hipStream_t s, const 
         (r = sj.list.reserve(jl.list.size())) || (r = sj.heavy.reserve(std::max<size_t>(1, jl.heavy.size()))) ||
         (r = sj.hinges.reserve(std::max<size_t>(1, jl.hinges.size()))) ||
         (r = sj.levels.reserve(std::max<size_t>(1, jl.level_start.size()))) ||
-        (r = v.jadj.reserve(std::max<size_t>(1, jl.list.size()))))
+        (r = v.reserve_joints(capacity)))
         return r;
     PMH_CHECK(hipMemcpyAsync(sj.copy.p, sj.host.data(), sizeof(PmhRigidConstraint) * capacity, hipMemcpyHostToDevice, s));
     PMH_CHECK(hipMemcpyAsync(sj.list_start.p, jl.start.data(), sizeof(uint32_t) * (n + 1), hipMemcpyHostToDevice, s));

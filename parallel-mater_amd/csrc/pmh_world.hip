@@ -488,7 +488,6 @@ PmhResult World::upload_joints() {
     solver.jlist = jlist.p;
     solver.jheavy = jheavy.p;
     solver.nheavy = uint32_t(jl.heavy.size());
-    if ((r = solver.jadj.reserve(std::max<size_t>(1, jl.list.size())))) return r;
     excl_count = total;
     if ((r = excl_list.reserve(list.size()))) return r;
     PMH_CHECK(hipMemcpy(excl_start.p, start.data(), sizeof(uint32_t) * (n + 1), hipMemcpyHostToDevice));
