@@ -99,6 +99,7 @@ struct StepCounters {
     uint32_t m1, m2, p1, p2, m1i, m2i, p1i, p2i;
     uint32_t point_alloc;      // narrowphase point-range allocator
     uint32_t tri_pairs;        // mesh pairs on the triangle-pair path
+    uint32_t tri_hits;         // those of them with overlapping leaves
     uint32_t fallback_pairs;   // of those, solved by BVH traversal
     uint32_t mean_roots;       // unanchored islands with contacts (free-motion mean)
     uint32_t joint_budget;     // largest joint iteration count (legacy budget floor)
