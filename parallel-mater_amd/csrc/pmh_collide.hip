@@ -1056,11 +1056,6 @@ __device__ bool segment_hits_triangle(V3 p, V3 q, V3 a, V3 b, V3 c, V3 &hit) {
            dot(cross(sub(a, c), sub(hit, c)), n) >= tol;
 }
 
-__device__ __forceinline__ void keep_closer(V3 a, V3 b, float &best, V3 &best_a, V3 &best_b) {
-    const float d = len2(sub(a, b));
-    if (d < best) { best = d; best_a = a; best_b = b; }
-}
-
 // A triangle in registers.  Every loop over corners or edges turns it instead
 // of indexing it: an index that is not a constant would put it in memory.
 struct Triangle {
@@ -1074,53 +1069,75 @@ __device__ __forceinline__ void turn(Triangle &t) {
 }
 __device__ __forceinline__ V3 triangle_cross(const Triangle &t) { return cross(sub(t.p1, t.p0), sub(t.p2, t.p0)); }
 
-// Closest points of two triangles.  The calls of the swept pass (up to 32 per
-// triangle pair) take their triangles in registers and loop over one body of
-// each of the three tests: the corners and edges in arrays were stored and
-// loaded through memory and the tests laid out 21 times, 20 KB of code (the
-// triangle kernel over 8000 flying boxes and spheres: 1.29 ms, then 1.14).
+// Closest points of two triangles, on four lanes that hold the same two: lane
+// e takes edge and corner e of both through the crossing tests, the corners
+// against the other face and its edge of A against B's three, and the first of
+// the nearest in the serial order wins.  The swept pass calls it up to 32 times
+// in a row, and each test is one chain of operations: 21 of them on one lane
+// took 10.6 us a round of the swept pass where 8000 bodies fly (1400 pairs, the
+// longest 0.39 ms), these 7 and the exchange 6 us (0.25 ms).
 struct ClosestPair {
     V3 a, b;
 };
+constexpr int kQuadFirst = 0x00, kQuadSecond = 0x55, kQuadThird = 0xaa;   // broadcasts within four lanes
+
+template <int kFrom>
+__device__ __forceinline__ V3 quad_v3(V3 v) {
+    return {dpp_f32<kFrom>(v.x), dpp_f32<kFrom>(v.y), dpp_f32<kFrom>(v.z)};
+}
+__device__ __forceinline__ Triangle turned(const Triangle &t, uint32_t e) {
+    const V3 p0 = e == 0u ? t.p0 : e == 1u ? t.p1 : t.p2, p1 = e == 0u ? t.p1 : e == 1u ? t.p2 : t.p0;
+    return {p0, p1, e == 0u ? t.p2 : e == 1u ? t.p0 : t.p1};
+}
+// The first hit of the lanes in order.
+__device__ __forceinline__ bool quad_first_hit(bool hit, V3 at, V3 &first) {
+    const uint32_t h = hit ? 1u : 0u;
+    const bool h0 = dpp_u32<kQuadFirst>(h) != 0u, h1 = dpp_u32<kQuadSecond>(h) != 0u, h2 = dpp_u32<kQuadThird>(h) != 0u;
+    const V3 a0 = quad_v3<kQuadFirst>(at), a1 = quad_v3<kQuadSecond>(at), a2 = quad_v3<kQuadThird>(at);
+    first = h0 ? a0 : h1 ? a1 : a2;
+    return h0 || h1 || h2;
+}
+struct NearestPair {
+    float d;
+    uint32_t order;                       // in the serial search
+    ClosestPair at;
+};
+__device__ __forceinline__ void keep_nearer(NearestPair &best, V3 a, V3 b, uint32_t order) {
+    const float d = len2(sub(a, b));
+    if (d < best.d) best = {d, order, {a, b}};
+}
+template <int kFrom>
+__device__ __forceinline__ void quad_nearer(NearestPair &best) {
+    const NearestPair o{dpp_f32<kFrom>(best.d), dpp_u32<kFrom>(best.order),
+                        {quad_v3<kFrom>(best.at.a), quad_v3<kFrom>(best.at.b)}};
+    if (o.d < best.d || (o.d == best.d && o.order < best.order)) best = o;
+}
 __device__ __noinline__ ClosestPair closest_points(float a0, float a1, float a2, float a3, float a4, float a5, float a6,
                                                    float a7, float a8, float b0, float b1, float b2, float b3, float b4,
                                                    float b5, float b6, float b7, float b8) {
-    Triangle A{{a0, a1, a2}, {a3, a4, a5}, {a6, a7, a8}}, B{{b0, b1, b2}, {b3, b4, b5}, {b6, b7, b8}};
-    V3 hit;
+    const Triangle A{{a0, a1, a2}, {a3, a4, a5}, {a6, a7, a8}}, B{{b0, b1, b2}, {b3, b4, b5}, {b6, b7, b8}};
+    const uint32_t e = min(threadIdx.x & 3u, 2u);       // the fourth lane repeats the third
+    const Triangle Ae = turned(A, e);
+    Triangle Be = turned(B, e);
+    V3 hit, first;
+    bool crosses = segment_hits_triangle(Ae.p0, Ae.p1, B.p0, B.p1, B.p2, hit);
+    if (quad_first_hit(crosses, hit, first)) return {first, first};
+    crosses = segment_hits_triangle(Be.p0, Be.p1, A.p0, A.p1, A.p2, hit);
+    if (quad_first_hit(crosses, hit, first)) return {first, first};
+    NearestPair best{3.402823466e+38f, ~0u, {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}}};
+    keep_nearer(best, Ae.p0, closest_on_triangle(Ae.p0, B.p0, B.p1, B.p2), e);
+    keep_nearer(best, closest_on_triangle(Be.p0, A.p0, A.p1, A.p2), Be.p0, 3u + e);
+    Be = B;
 #pragma unroll 1
-    for (uint32_t e = 0; e < 3; ++e) {
-        if (segment_hits_triangle(A.p0, A.p1, B.p0, B.p1, B.p2, hit)) return {hit, hit};
-        turn(A);
+    for (uint32_t j = 0; j < 3; ++j) {
+        V3 u, w;
+        closest_segments(Ae.p0, Ae.p1, Be.p0, Be.p1, u, w);
+        keep_nearer(best, u, w, 6u + 3u * e + j);
+        turn(Be);
     }
-#pragma unroll 1
-    for (uint32_t e = 0; e < 3; ++e) {
-        if (segment_hits_triangle(B.p0, B.p1, A.p0, A.p1, A.p2, hit)) return {hit, hit};
-        turn(B);
-    }
-    float best = 3.402823466e+38f;
-    ClosestPair c{{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
-#pragma unroll 1
-    for (uint32_t i = 0; i < 3; ++i) {
-        keep_closer(A.p0, closest_on_triangle(A.p0, B.p0, B.p1, B.p2), best, c.a, c.b);
-        turn(A);
-    }
-#pragma unroll 1
-    for (uint32_t i = 0; i < 3; ++i) {
-        keep_closer(closest_on_triangle(B.p0, A.p0, A.p1, A.p2), B.p0, best, c.a, c.b);
-        turn(B);
-    }
-#pragma unroll 1
-    for (uint32_t i = 0; i < 3; ++i) {
-#pragma unroll 1
-        for (uint32_t j = 0; j < 3; ++j) {
-            V3 u, w;
-            closest_segments(A.p0, A.p1, B.p0, B.p1, u, w);
-            keep_closer(u, w, best, c.a, c.b);
-            turn(B);
-        }
-        turn(A);
-    }
-    return c;
+    quad_nearer<kDppXor1>(best);
+    quad_nearer<kDppXor2>(best);
+    return best.at;
 }
 __device__ __forceinline__ void closest_triangle_pair(const Triangle &A, const Triangle &B, V3 &pa, V3 &pb) {
     const ClosestPair c = closest_points(A.p0.x, A.p0.y, A.p0.z, A.p1.x, A.p1.y, A.p1.z, A.p2.x, A.p2.y, A.p2.z, B.p0.x,
@@ -2479,11 +2496,16 @@ __global__ void k_scene_pairs(const uint32_t *npairs, const uint2 *ab, const uin
 constexpr uint32_t kTriWaves = 4;          // wavefronts per block
 constexpr uint32_t kLeafListCap = 512;     // ordered leaf pairs held in LDS per wavefront
 constexpr uint32_t kListOverflow = 0xffffffffu;
+constexpr uint32_t kTraversalStack = 64;   // the reference's
+constexpr uint32_t kTriBatch = 16;         // triangle pairs of a wavefront's batch, four lanes each
 
 struct TriWaveShared {
     uint2 list[kLeafListCap];              // (body leaf node, collider leaf node) in evaluation order
-    uint32_t cand[64];                     // triangle pairs to evaluate: leaf pair << 4 | slot in it
-    float4 disc[64][2], swept[64][2];      // their contacts: normal+pen, point+impact fraction
+    uint2 stack[kTraversalStack];          // of the BVH traversal
+    uint32_t cand[kTriBatch];              // triangle pairs to evaluate: leaf pair << 4 | slot in it
+    uint32_t found[2];                     // which of them gave a contact, discrete and swept
+    uint32_t held;                         // how many there are
+    float4 disc[kTriBatch][2], swept[kTriBatch][2];   // their contacts: normal+pen, point+impact fraction
     Manifold man, local;
     uint32_t count;
     // The wavefront's triangle pair (one per wavefront, read by every lane):
@@ -2510,7 +2532,7 @@ __device__ __forceinline__ bool leaf_cell_overlaps(const TrianglePair &tp, bool 
 // The leaf pairs rigid_collide_meshes visits, in visiting order, or
 // kListOverflow when its stack would overflow (the reference then runs
 // every triangle pair) or the list does not fit.
-__device__ uint32_t traversal_list(const TrianglePair &P, bool swept, uint2 *list) {
+__device__ uint32_t traversal_list(const TrianglePair &P, bool swept, uint2 *list, uint2 *stack) {
     const BoundsFrame fa = bounds_frame(P.a), fb = bounds_frame(P.b);
     const BoundsFrame pfa = swept ? bounds_frame(P.ap) : BoundsFrame{};
     const BoundsFrame pfb = swept ? bounds_frame(P.bp) : BoundsFrame{};
@@ -2519,14 +2541,11 @@ __device__ uint32_t traversal_list(const TrianglePair &P, bool swept, uint2 *lis
     motion_bounds(sarr(P.bm.s.mn), sarr(P.bm.s.mx), pfb, fb, swept, 0.0f, bmn, bmx);
     if (!boxes_touch(amn, amx, bmn, bmx)) return 0;
     if (P.am.s.node_count == 0u || P.bm.s.node_count == 0u) return kListOverflow;
-    constexpr uint32_t kStack = 64;
-    uint32_t sa[kStack], sb[kStack];
-    sa[0] = 0;
-    sb[0] = 0;
+    stack[0] = make_uint2(0u, 0u);
     uint32_t top = 1, count = 0;
     while (top > 0u) {
         --top;
-        const uint32_t ia = sa[top], ib = sb[top];
+        const uint32_t ia = stack[top].x, ib = stack[top].y;
         const BvhDev na = P.am.node(ia), nb = P.bm.node(ib);
         node_bounds(na, pfa, fa, swept, P.margin, amn, amx);
         node_bounds(nb, pfb, fb, swept, 0.0f, bmn, bmx);
@@ -2538,25 +2557,26 @@ __device__ uint32_t traversal_list(const TrianglePair &P, bool swept, uint2 *lis
             continue;
         }
         const uint32_t need = la || lb ? 2u : 4u;
-        if (top + need > kStack) return kListOverflow;
+        if (top + need > kTraversalStack) return kListOverflow;
         if (la) {
-            sa[top] = ia; sb[top++] = nb.right;
-            sa[top] = ia; sb[top++] = nb.left;
+            stack[top++] = make_uint2(ia, nb.right);
+            stack[top++] = make_uint2(ia, nb.left);
         } else if (lb) {
-            sa[top] = na.right; sb[top++] = ib;
-            sa[top] = na.left; sb[top++] = ib;
+            stack[top++] = make_uint2(na.right, ib);
+            stack[top++] = make_uint2(na.left, ib);
         } else {
-            sa[top] = na.right; sb[top++] = nb.right;
-            sa[top] = na.right; sb[top++] = nb.left;
-            sa[top] = na.left; sb[top++] = nb.right;
-            sa[top] = na.left; sb[top++] = nb.left;
+            stack[top++] = make_uint2(na.right, nb.right);
+            stack[top++] = make_uint2(na.right, nb.left);
+            stack[top++] = make_uint2(na.left, nb.right);
+            stack[top++] = make_uint2(na.left, nb.left);
         }
     }
     return count;
 }
 
 // Serial evaluation for the rare pairs whose leaf list does not fit in
-// LDS: the same candidate order and merge rule on one lane.  Leaf
+// LDS: the same candidate order and merge rule on one lane (four lanes of
+// the same data, which the closest-point search is laid out for).  Leaf
 // candidates come from the motion test alone (`swept`); the ranges of a
 // guided pair always take the swept pass (`swept_eval`).
 __device__ void triangle_pair_serial(const TrianglePair &tp, bool swept, bool swept_eval, bool leaf_mode,
@@ -2689,9 +2709,9 @@ __global__ void __launch_bounds__(kScreenBlock) k_triangle_screen(
 // any other pair takes the leaf pairs of the BVH traversal in visiting
 // order and merges contacts directly.  Of 4 leaf pairs x 16 triangle pairs at
 // a time (leaves hold at most 4 triangles) those whose boxes touch are
-// gathered until 64 are there, whole leaf pairs at a time, and evaluated at
-// once: the swept pass costs what its longest lane costs, and by fours of
-// leaf pairs most lanes held pairs that the box test ended.  One lane then
+// gathered until 16 are there, whole leaf pairs at a time, and evaluated on
+// four lanes each: by fours of leaf pairs most lanes held pairs that the box
+// test ended (8 or 9 of a mesh pair's are left in the mean).  One lane then
 // replays the contacts through the merge rule in order: per leaf pair the
 // discrete contacts body-triangle-major, then the swept ones.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_triangle_pairs(const uint32_t *hit_list,
@@ -2708,9 +2728,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     TriWaveShared &S = shared_waves[wv];
     const uint32_t T = o.ctr->tri_hits;
-    const uint32_t nwaves = gridDim.x * kTriWaves;
+    // A list with no more pairs than blocks gives each pair a whole block: its
+    // wavefronts gather the same candidates, each evaluates its turn of the
+    // batches, and the first merges.  A pair that needs all 32 advances of the
+    // swept pass in several batches otherwise outlasts all others (8000 flying
+    // bodies, 1400 pairs: 0.31 ms, so 0.25).  A longer list keeps every
+    // wavefront busy by itself (7200 pairs of meshes at rest: 0.21 ms, 0.51 by
+    // blocks).
+    const bool wide = T <= gridDim.x;
+    const uint32_t stride = wide ? gridDim.x : gridDim.x * kTriWaves;
     uint32_t fallback = 0;
-    for (uint32_t t = blockIdx.x * kTriWaves + wv; t < T; t += nwaves) {
+    for (uint32_t t = wide ? blockIdx.x : blockIdx.x * kTriWaves + wv; t < T; t += stride) {
         const uint32_t m = hit_list[t];
         const uint64_t mask = hit_mask[t];
         const uint2 p = ab[m];
@@ -2772,8 +2800,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
             }
         } else {
             if (lane == 0) {
-                ++fallback;
-                S.count = traversal_list(tp, swept_eval, S.list);
+                fallback += wide && wv != 0 ? 0u : 1u;
+                S.count = traversal_list(tp, swept_eval, S.list, S.stack);
             }
             wave_sync();
             nlist = S.count;
@@ -2781,68 +2809,85 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         wave_sync();
         // 2. Contacts.
         if (nlist == kListOverflow) {
-            if (lane == 0) triangle_pair_serial(tp, swept, swept_eval, leaf_mode, S.man, S.local);
+            if (lane < 4u && !(wide && wv != 0)) triangle_pair_serial(tp, swept, swept_eval, leaf_mode, S.man, S.local);
         } else {
             if (lane == 0) {
                 S.man.count = 0;
                 S.man.face_patch = 0;
             }
             const float spacing = smax(tp.margin * 2.0f, 1.0e-4f);
-            uint32_t held = 0;
-            // Evaluates and merges the candidates held.
-            auto flush = [&]() {
-                wave_sync();
-                bool hd = false, hs = false;
-                Contact cd, cs;
-                if (lane < held) {
-                    const uint32_t cand = S.cand[lane];
-                    const uint2 e = S.list[cand >> 4];
-                    const uint32_t at = tp.am.node(e.x).first + (cand >> 2 & 3u);
-                    const uint32_t bt = tp.bm.node(e.y).first + (cand & 3u);
-                    hd = !guided && triangle_pair_contact(tp, at, bt, inside_a, inside_b, cd);
-                    if (swept_eval) hs = triangle_pair_swept_contact(tp, at, bt, inside_a, inside_b, cs);
-                }
-                if (hd) {
-                    S.disc[lane][0] = f4(cd.normal, cd.pen);
-                    S.disc[lane][1] = f4(cd.point, cd.impact_fraction);
-                }
-                if (hs) {
-                    S.swept[lane][0] = f4(cs.normal, cs.pen);
-                    S.swept[lane][1] = f4(cs.point, cs.impact_fraction);
-                }
-                const uint64_t md = __ballot(hd), ms = __ballot(hs);
-                wave_sync();
-                if (lane == 0) {
+            uint32_t held = 0, batch = 0;
+            // Merges the batches evaluated since the last merge.
+            auto merge = [&](uint32_t batches) {
+                if (wide) __syncthreads();
+                else wave_sync();
+                for (uint32_t w = 0; w < batches; ++w) {
+                    if (lane != 0 || (wide && wv != 0)) continue;
+                    TriWaveShared &R = wide ? shared_waves[w] : S;
+                    const uint32_t md = R.found[0], ms = R.found[1];
                     Manifold &dst = leaf_mode ? S.local : S.man;
-                    for (uint64_t left = md | ms; left;) {
+                    for (uint32_t left = md | ms; left;) {
                         // the candidates of the next leaf pair with contacts
-                        const uint32_t k0 = uint32_t(__builtin_ctzll(left)), leaf = S.cand[k0] >> 4;
+                        const uint32_t k0 = uint32_t(__builtin_ctz(left)), leaf = R.cand[k0] >> 4;
                         uint32_t k1 = k0 + 1;
-                        while (k1 < held && S.cand[k1] >> 4 == leaf) ++k1;
-                        const uint64_t group = (k1 == 64u ? ~0ull : (1ull << k1) - 1ull) & ~((1ull << k0) - 1ull);
+                        while (k1 < R.held && R.cand[k1] >> 4 == leaf) ++k1;
+                        const uint32_t group = (1u << k1) - (1u << k0);
                         left &= ~group;
                         if (leaf_mode) {
                             S.local.count = 0;
                             S.local.face_patch = 0;
                         }
-                        for (uint64_t b = md & group; b; b &= b - 1ull) {
-                            const uint32_t k = uint32_t(__builtin_ctzll(b));
-                            const Contact c{v3(S.disc[k][0]), v3(S.disc[k][1]), S.disc[k][0].w, S.disc[k][1].w};
+                        for (uint32_t b = md & group; b; b &= b - 1u) {
+                            const uint32_t k = uint32_t(__builtin_ctz(b));
+                            const Contact c{v3(R.disc[k][0]), v3(R.disc[k][1]), R.disc[k][0].w, R.disc[k][1].w};
                             merge_contact(tp, dst, c, spacing);
                         }
-                        for (uint64_t b = ms & group; b; b &= b - 1ull) {
-                            const uint32_t k = uint32_t(__builtin_ctzll(b));
-                            const Contact c{v3(S.swept[k][0]), v3(S.swept[k][1]), S.swept[k][0].w, S.swept[k][1].w};
+                        for (uint32_t b = ms & group; b; b &= b - 1u) {
+                            const uint32_t k = uint32_t(__builtin_ctz(b));
+                            const Contact c{v3(R.swept[k][0]), v3(R.swept[k][1]), R.swept[k][0].w, R.swept[k][1].w};
                             merge_contact(tp, dst, c, spacing);
                         }
                         if (leaf_mode)
                             for (uint32_t k = 0; k < S.local.count; ++k) merge_contact(tp, S.man, S.local.c[k], spacing);
                     }
                 }
-                wave_sync();
-                held = 0;
+                if (wide) __syncthreads();
+                else wave_sync();
+                batch = 0;
             };
-            for (uint32_t first = 0; first < nlist; first += 4u) {
+            // Evaluates the candidates held, as this wavefront's batch or
+            // another's.
+            auto evaluate = [&]() {
+                wave_sync();
+                bool hd = false, hs = false;
+                Contact cd, cs;
+                const bool mine = !wide || batch == wv;
+                const uint32_t k = lane / 4u;
+                if (mine && k < held) {
+                    const uint32_t cand = S.cand[k];
+                    const uint2 e = S.list[cand >> 4];
+                    const uint32_t at = tp.am.node(e.x).first + (cand >> 2 & 3u);
+                    const uint32_t bt = tp.bm.node(e.y).first + (cand & 3u);
+                    hd = !guided && triangle_pair_contact(tp, at, bt, inside_a, inside_b, cd);
+                    if (swept_eval) hs = triangle_pair_swept_contact(tp, at, bt, inside_a, inside_b, cs);
+                }
+                if (hd && lane % 4u == 0u) {
+                    S.disc[k][0] = f4(cd.normal, cd.pen);
+                    S.disc[k][1] = f4(cd.point, cd.impact_fraction);
+                }
+                if (hs && lane % 4u == 0u) {
+                    S.swept[k][0] = f4(cs.normal, cs.pen);
+                    S.swept[k][1] = f4(cs.point, cs.impact_fraction);
+                }
+                if (mine && lane == 0) S.found[0] = S.found[1] = 0u;
+                if (hd && lane % 4u == 0u) atomicOr(&S.found[0], 1u << k);
+                if (hs && lane % 4u == 0u) atomicOr(&S.found[1], 1u << k);
+                if (mine && lane == 0) S.held = held;
+                held = 0;
+                ++batch;
+            };
+            for (uint32_t first = 0;; first += 4u) {
+                const bool end = first >= nlist;
                 const uint32_t j = first + lane / 16u, ai = lane / 4u % 4u, bi = lane % 4u;
                 bool near = false;
                 if (j < nlist) {
@@ -2856,16 +2901,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 #pragma unroll 1
                 for (uint32_t g = 0; g < 4u; ++g) {
                     const uint32_t bits = uint32_t(found >> (16u * g)) & 0xffffu, count = uint32_t(__popc(bits));
-                    if (held + count > 64u) flush();
-                    if (lane / 16u == g && near) S.cand[held + __popc(bits & ((1u << (lane % 16u)) - 1u))] = j << 4 | lane % 16u;
+                    if (held + count > kTriBatch || (end && held)) evaluate();
+                    if (batch == (wide ? kTriWaves : 1u) || (end && batch)) merge(batch);
+                    if (lane / 16u == g && near && (!wide || batch == wv))
+                        S.cand[held + __popc(bits & ((1u << (lane % 16u)) - 1u))] = j << 4 | lane % 16u;
                     held += count;
                 }
+                if (end) break;
             }
-            if (held) flush();
         }
         wave_sync();
         // 3. Emit.
-        if (lane == 0) {
+        if (lane == 0 && !(wide && wv != 0)) {
             Manifold man = S.man;
             emit_manifold(o, m, man, tp.a, tp.b, persistent_pair(tp.am.s, tp.bm.s, pb), tp.f.ha, tp.f.hb);
         }
