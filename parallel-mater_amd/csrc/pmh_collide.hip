@@ -280,25 +280,36 @@ __global__ void k_scene_large(const StepCounters *ctr, const uint32_t *large, co
     }
 }
 
-// Kept candidates of dynamic body a, found by a group of 32 lanes: lane
-// q < 27 walks neighbour cell q of the 3x3x3 block around the body's cell,
-// and every lane takes every 32nd entry of the large-body list.  Pass 0
-// counts them; pass 1 writes each lane's candidates at the body's offset
-// (from an exclusive scan of the counts) plus the lane's prefix within the
-// group, then one lane sorts the segment ascending (identity order =
-// index), so a body may own any number of pairs.
-constexpr uint32_t kQueryLanes = 32;
+// Grid query, a group of 32 lanes per body: the entries of the body's 27
+// cells' buckets as one list dealt over the lanes (a bucket has none, a few
+// or, in a crowd, dozens, and a lane per cell waited for the longest chain),
+// two at a time so that their loads overlap.  Pass 0 gathers what it finds in
+// LDS, counts it, and leaves it sorted ascending (identity order = index) in
+// the body's segment of `pool`, `segment` candidates for every body; pass 1
+// copies it to the body's offset (an exclusive scan of the counts).  A body
+// with more candidates walks again in pass 1 and sorts where it writes, so a
+// body may own any number of pairs.  Bounded by the latency of bucket, entry
+// and box loads.  Counting in pass 0 and walking twice more in pass 1 took
+// 217 + 416 us of a step of 32768 bodies (0.52M pairs), now 60 + 9;
+// segments reserved from one counter instead of laid out took 330 us, and 405
+// over 65538 chain links (by segments 52).
+constexpr uint32_t kQueryLanes = 32, kQueryBlock = 256;
+constexpr uint32_t kQueryHeld = 128;       // candidates of a body held in LDS
 
 template <int kPass>
-__global__ void __launch_bounds__(256) k_bp_query(uint32_t n, const PmhBodyParameters *P, const float4 *pmn,
+__global__ void __launch_bounds__(kQueryBlock) k_bp_query(uint32_t n, const PmhBodyParameters *P, const float4 *pmn,
                                                   const float4 *pmx, const int4 *cell_of, const uint32_t *bucket_start,
                                                   const int4 *entry_cell, const float4 *entry_mn,
                                                   const float4 *entry_mx, uint32_t table_mask, const uint32_t *large,
-                                                  uint32_t *cand_count, const uint32_t *offset, uint32_t *code,
-                                                  uint2 *ab, const StepCounters *ctr, JointFilter jf) {
-    const uint64_t t = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const uint32_t a = uint32_t(t / kQueryLanes), q = uint32_t(t % kQueryLanes);
-    // Every exit above the shuffles is uniform over the body's group.
+                                                  uint32_t *cand_count, uint32_t *pool, uint32_t segment,
+                                                  const uint32_t *offset, uint32_t *code, uint2 *ab,
+                                                  const StepCounters *ctr, JointFilter jf) {
+    constexpr uint32_t groups = kQueryBlock / kQueryLanes;
+    __shared__ uint32_t s_held[kPass == 0 ? groups : 1][kQueryHeld];
+    // Every exit is uniform over the body's group.
+    const uint32_t g = threadIdx.x / kQueryLanes, q = threadIdx.x % kQueryLanes;
+    const uint32_t a = blockIdx.x * groups + g;
+    const uint32_t below = (1u << q) - 1u;
     if (a >= n) return;
     if (P[a].motion != kDynamic) {
         if (kPass == 0 && q == 0) cand_count[a] = 0;
@@ -307,69 +318,113 @@ __global__ void __launch_bounds__(256) k_bp_query(uint32_t n, const PmhBodyParam
     if (kPass == 1 && ctr->pairs == 0) return;   // pair pool overflow: nothing is emitted
     const int4 c = cell_of[a];
     if (c.x == kLargeCell) return;   // k_bp_large owns this body
-    const float4 amn = pmn[a], amx = pmx[a];
-    uint32_t count = 0;
-    auto walk = [&](auto &&emit) {
-        if (q < 27u) {
-            const int x = c.x + int(q % 3u) - 1, y = c.y + int((q / 3u) % 3u) - 1, z = c.z + int(q / 9u) - 1;
-            const uint32_t bk = cell_hash(x, y, z) & table_mask;
-            for (uint32_t e = bucket_start[bk]; e < bucket_start[bk + 1]; ++e) {
-                const int4 cb = entry_cell[e];
-                if (cb.x != x || cb.y != y || cb.z != z) continue;
-                const float4 bmn = entry_mn[e];
-                const uint32_t b = __float_as_uint(bmn.w);
-                if (b == a || (cb.w != 0 && !(a < b))) continue;
-                if (!overlap(amn, amx, bmn, entry_mx[e])) continue;
-                if (joint_excluded(jf, a, b)) continue;
-                emit(b);
+    uint32_t *mine = pool + size_t(a) * segment;
+    uint32_t base = 0;
+    if (kPass == 1) {
+        const uint32_t total = cand_count[a];
+        base = offset[a];
+        if (total <= segment) {
+            for (uint32_t k = q; k < total; k += kQueryLanes) {
+                const uint32_t b = mine[k];
+                code[base + k] = a * n + b;
+                ab[base + k] = make_uint2(a, b);
             }
+            return;
         }
-        auto consider = [&](uint32_t b) {
-            if (b == a) return;
-            if (P[b].motion == kDynamic && !(a < b)) return;
-            if (!overlap(amn, amx, pmn[b], pmx[b])) return;
-            if (joint_excluded(jf, a, b)) return;
-            emit(b);
-        };
-        if (jf.scene_large) {
-            const uint32_t sc = jf.scene[a];
-            for (uint32_t k = jf.scene_large_start[sc] + q; k < jf.scene_large_start[sc + 1]; k += kQueryLanes)
-                consider(jf.scene_large[k]);
-        } else {
-            const uint32_t nl = ctr->large_count;
-            for (uint32_t k = q; k < nl; k += kQueryLanes) consider(large[k]);
-        }
-    };
-    walk([&](uint32_t) { ++count; });   // pass 1 counts again: its lanes need their own prefixes
-    // Inclusive scan of the lane counts within the group.
-    uint32_t incl = count;
+    }
+    const float4 amn = pmn[a], amx = pmx[a];
+    uint32_t first = 0, len = 0;
+    if (q < 27u) {
+        const uint32_t bk = cell_hash(c.x + int(q % 3u) - 1, c.y + int((q / 3u) % 3u) - 1, c.z + int(q / 9u) - 1) &
+                            table_mask;
+        first = bucket_start[bk];
+        len = bucket_start[bk + 1] - first;
+    }
+    uint32_t incl = len;
     for (uint32_t d = 1; d < kQueryLanes; d <<= 1) {
         const uint32_t y = __shfl_up(incl, d, kQueryLanes);
         if (q >= d) incl += y;
     }
-    const uint32_t total = __shfl(incl, kQueryLanes - 1, kQueryLanes);
+    const uint32_t entries = __shfl(incl, kQueryLanes - 1, kQueryLanes);
+    first -= incl - len;                             // entry f of the list is first + f
+    // Calls emit(slot, body) for every candidate, slots in the order found.
+    auto walk = [&](auto &&emit) -> uint32_t {
+        uint32_t found = 0;
+        auto gather = [&](bool hit, uint32_t b) {
+            const uint32_t mask = uint32_t(__ballot(hit) >> (threadIdx.x & 32u));
+            if (hit) emit(found + uint32_t(__popc(mask & below)), b);
+            found += uint32_t(__popc(mask));
+        };
+        for (uint32_t f0 = 0; f0 < entries; f0 += 2 * kQueryLanes) {
+            int4 at[2], cb[2];
+            float4 bmn[2], bmx[2];
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) {
+                const uint32_t f = min(f0 + u * kQueryLanes + q, entries - 1u);
+                uint32_t k = 0;                          // its cell: as many lists end at or before f
+#pragma unroll
+                for (uint32_t step = kQueryLanes / 2; step >= 1u; step /= 2)
+                    if (__shfl(incl, k + step - 1u, kQueryLanes) <= f) k += step;
+                const uint32_t e = f + __shfl(first, k, kQueryLanes);
+                at[u] = make_int4(c.x + int(k % 3u) - 1, c.y + int((k / 3u) % 3u) - 1, c.z + int(k / 9u) - 1, 0);
+                cb[u] = entry_cell[e];
+                bmn[u] = entry_mn[e];
+                bmx[u] = entry_mx[e];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) {
+                const uint32_t b = __float_as_uint(bmn[u].w);
+                const bool hit = f0 + u * kQueryLanes + q < entries && cb[u].x == at[u].x && cb[u].y == at[u].y &&
+                                 cb[u].z == at[u].z && b != a && (cb[u].w == 0 || a < b) &&
+                                 overlap(amn, amx, bmn[u], bmx[u]) && !joint_excluded(jf, a, b);
+                gather(hit, b);
+            }
+        }
+        const uint32_t *list = large;
+        uint32_t lb = 0, le = ctr->large_count;
+        if (jf.scene_large) {
+            const uint32_t sc = jf.scene[a];
+            list = jf.scene_large;
+            lb = jf.scene_large_start[sc];
+            le = jf.scene_large_start[sc + 1];
+        }
+        for (; lb < le; lb += kQueryLanes) {
+            const uint32_t b = lb + q < le ? list[lb + q] : a;
+            const bool hit = b != a && (P[b].motion != kDynamic || a < b) && overlap(amn, amx, pmn[b], pmx[b]) &&
+                             !joint_excluded(jf, a, b);
+            gather(hit, b);
+        }
+        return found;
+    };
     if (kPass == 0) {
+        const uint32_t total = walk([&](uint32_t slot, uint32_t b) {
+            if (slot < kQueryHeld) s_held[g][slot] = b;
+        });
         if (q == 0) cand_count[a] = total;
+        if (total > segment) return;
+        __threadfence_block();
+        __builtin_amdgcn_wave_barrier();
+        // Rank sort: element k goes to the count of elements below it (a body
+        // is found once).
+        for (uint32_t k = q; k < total; k += kQueryLanes) {
+            const uint32_t v = s_held[g][k];
+            uint32_t rank = 0;
+            for (uint32_t i = 0; i < total; ++i) rank += s_held[g][i] < v ? 1u : 0u;
+            mine[rank] = v;
+        }
         return;
     }
-    const uint32_t base = offset[a];
     uint32_t *out = code + base;
-    uint32_t at = incl - count;
-    walk([&](uint32_t b) { out[at++] = b; });
+    const uint32_t total = walk([&](uint32_t slot, uint32_t b) { out[slot] = b; });
     // The segment's writes of every lane are visible to the whole group.
     __threadfence_block();
     __builtin_amdgcn_wave_barrier();
-    // Rank sort of the segment over the group's lanes: element k goes to
-    // the count of elements below it, ties in segment order (the order a
-    // stable insertion sort leaves).  The pairs are written first, then the
-    // codes from them, since the codes' slots hold the unsorted segment.
+    // The pairs are written first, then the codes from them, since the codes'
+    // slots hold the unsorted segment.
     for (uint32_t k = q; k < total; k += kQueryLanes) {
         const uint32_t v = out[k];
         uint32_t rank = 0;
-        for (uint32_t i = 0; i < total; ++i) {
-            const uint32_t w = out[i];
-            rank += (w < v || (w == v && i < k)) ? 1u : 0u;
-        }
+        for (uint32_t i = 0; i < total; ++i) rank += out[i] < v ? 1u : 0u;
         ab[base + rank] = make_uint2(a, v);
     }
     __threadfence_block();
@@ -391,13 +446,16 @@ __global__ void k_set_pairs(StepCounters *ctr, const uint32_t *offset, uint32_t 
 // Large bodies: one block scans every body in index order; a block-wide
 // prefix sum places the hits, so the segment comes out ascending.  Blocks
 // beyond the number of large bodies return at once.
-constexpr uint32_t kLargeBlocks = 1024;
+// Four chunks of 256 at a time, their boxes loaded together: one chunk took
+// 0.36 us for its two loads and barriers (65538 bodies, 93 us a pass, now
+// 36).
+constexpr uint32_t kLargeBlocks = 1024, kLargeChunks = 4;
 template <int kPass>
 __global__ void __launch_bounds__(256) k_bp_large(uint32_t n, const PmhBodyParameters *P, const float4 *pmn,
                                                   const float4 *pmx, const uint32_t *large, uint32_t *cand_count,
                                                   const uint32_t *offset, uint32_t *code, uint2 *ab,
                                                   const StepCounters *ctr, JointFilter jf) {
-    __shared__ uint32_t warp_tot[4];
+    __shared__ uint32_t warp_tot[kLargeChunks][4];
     const uint32_t nl = ctr->large_count;
     const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     for (uint32_t k = blockIdx.x; k < nl; k += gridDim.x) {
@@ -412,25 +470,39 @@ __global__ void __launch_bounds__(256) k_bp_large(uint32_t n, const PmhBodyParam
         // In a batch only the body's own scene can pair with it.
         const uint32_t first = jf.scene_first ? jf.scene_first[jf.scene[a]] : 0u;
         const uint32_t last = jf.scene_first ? first + jf.scene_count[jf.scene[a]] : n;
-        for (uint32_t base = first; base < last; base += 256) {
-            const uint32_t b = base + threadIdx.x;
-            bool hit = false;
-            if (b < last && b != a && !(P[b].motion == kDynamic && !(a < b)))
-                hit = overlap(amn, amx, pmn[b], pmx[b]) && !joint_excluded(jf, a, b);
-            const uint64_t bal = __ballot(hit);
-            if (lane == 0) warp_tot[wid] = __popcll(bal);
+        for (uint32_t base = first; base < last; base += 256 * kLargeChunks) {
+            float4 bmn[kLargeChunks], bmx[kLargeChunks];
+            uint64_t bal[kLargeChunks];
+#pragma unroll
+            for (uint32_t u = 0; u < kLargeChunks; ++u) {
+                const uint32_t b = min(base + u * 256 + threadIdx.x, last - 1u);
+                bmn[u] = pmn[b];
+                bmx[u] = pmx[b];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kLargeChunks; ++u) {
+                const uint32_t b = base + u * 256 + threadIdx.x;
+                const bool hit = b < last && b != a && overlap(amn, amx, bmn[u], bmx[u]) &&
+                                 !(P[b].motion == kDynamic && !(a < b)) && !joint_excluded(jf, a, b);
+                bal[u] = __ballot(hit);
+                if (lane == 0) warp_tot[u][wid] = __popcll(bal[u]);
+            }
             __syncthreads();
-            uint32_t before = 0, total = 0;
-            for (uint32_t w = 0; w < 4; ++w) {
-                if (w < wid) before += warp_tot[w];
-                total += warp_tot[w];
+#pragma unroll
+            for (uint32_t u = 0; u < kLargeChunks; ++u) {
+                uint32_t before = 0, total = 0;
+                for (uint32_t w = 0; w < 4; ++w) {
+                    if (w < wid) before += warp_tot[u][w];
+                    total += warp_tot[u][w];
+                }
+                if (kPass == 1 && ((bal[u] >> lane) & 1ull) != 0ull) {
+                    const uint32_t b = base + u * 256 + threadIdx.x;
+                    const uint32_t pos = running + before + __popcll(bal[u] & ((1ull << lane) - 1ull));
+                    code[pos] = a * n + b;
+                    ab[pos] = make_uint2(a, b);
+                }
+                running += total;
             }
-            if (kPass == 1 && hit) {
-                const uint32_t pos = running + before + __popcll(bal & ((1ull << lane) - 1ull));
-                code[pos] = a * n + b;
-                ab[pos] = make_uint2(a, b);
-            }
-            running += total;
             __syncthreads();
         }
         if (kPass == 0 && threadIdx.x == 0) cand_count[a] = running;
@@ -3144,10 +3216,12 @@ PmhResult World::step_once(uint32_t k_step, bool warm_infer) {
         jf.scene_first = scene_first_dev.p;
         jf.scene_count = scene_count.p;
     }
-    const uint32_t query_blocks = uint32_t((uint64_t(n) * kQueryLanes + 255) / 256);
-    k_bp_query<0><<<query_blocks, 256, 0, s>>>(n, params.p, proxy_mn.p, proxy_mx.p, cell_of.p,
-                                                  bucket_start.p, entry_cell.p, entry_mn.p, entry_mx.p, table_size - 1, large.p,
-                                                  cand_count.p, nullptr, nullptr, nullptr, ctr, jf);
+    const uint32_t query_blocks = uint32_t((uint64_t(n) * kQueryLanes + kQueryBlock - 1) / kQueryBlock);
+    // The triangle list is not in use yet: the pool of the candidates.
+    const uint32_t segment = std::min(v.pair_cap / std::max<uint32_t>(1, n), kQueryHeld);
+    k_bp_query<0><<<query_blocks, kQueryBlock, 0, s>>>(
+        n, params.p, proxy_mn.p, proxy_mx.p, cell_of.p, bucket_start.p, entry_cell.p, entry_mn.p, entry_mx.p,
+        table_size - 1, large.p, cand_count.p, v.tri_list.p, segment, nullptr, nullptr, nullptr, ctr, jf);
     k_bp_large<0><<<kLargeBlocks, 256, 0, s>>>(n, params.p, proxy_mn.p, proxy_mx.p, large.p, cand_count.p, nullptr, nullptr,
                                      nullptr, ctr, jf);
     r = exclusive_scan(s, cand_count.p, cand_offset.p, n, nullptr, nullptr, v.scan_tmp);
@@ -3155,9 +3229,9 @@ PmhResult World::step_once(uint32_t k_step, bool warm_infer) {
     k_set_pairs<<<1, 64, 0, s>>>(ctr, cand_offset.p, n, v.pair_cap);
     k_bp_large<1><<<kLargeBlocks, 256, 0, s>>>(n, params.p, proxy_mn.p, proxy_mx.p, large.p, cand_count.p, cand_offset.p,
                                      v.code.p, v.ab.p, ctr, jf);
-    k_bp_query<1><<<query_blocks, 256, 0, s>>>(n, params.p, proxy_mn.p, proxy_mx.p, cell_of.p,
-                                                  bucket_start.p, entry_cell.p, entry_mn.p, entry_mx.p, table_size - 1, large.p,
-                                                  cand_count.p, cand_offset.p, v.code.p, v.ab.p, ctr, jf);
+    k_bp_query<1><<<query_blocks, kQueryBlock, 0, s>>>(
+        n, params.p, proxy_mn.p, proxy_mx.p, cell_of.p, bucket_start.p, entry_cell.p, entry_mn.p, entry_mx.p,
+        table_size - 1, large.p, cand_count.p, v.tri_list.p, segment, cand_offset.p, v.code.p, v.ab.p, ctr, jf);
     mark(2);
     if (rules.scene) k_scene_pairs<<<pg, 256, 0, s>>>(&ctr->pairs, v.ab.p, scene_of.p, scene_pair_start.p);
     // Narrowphase + point compaction.
