@@ -156,7 +156,12 @@ __device__ __forceinline__ float contact_skin(const PmhBodyParameters &a, const 
 }
 
 // ---------------------------------------------------------------------
-// Device-wide exclusive scan (three passes, 1024 elements per block).
+// Device-wide exclusive scan, 1024 elements per block.  out[count] is the
+// total.  Bounded by its launches: one block takes short inputs whole, and in
+// two launches each block of the second sums the blocks' totals before it
+// itself; only where those would be more than a few thousand per block does a
+// third launch scan them.  As four launches (totals, their scan, application,
+// total) 5400 elements took 9 us and the gaps between them, now 3.1.
 // ---------------------------------------------------------------------
 constexpr uint32_t kScanBlock = 256, kScanItems = 4, kScanTile = kScanBlock * kScanItems;
 
@@ -184,6 +189,7 @@ __device__ uint32_t block_exclusive(uint32_t v, uint32_t *total) {
 __global__ void k_scan_reduce(const uint32_t *in, uint32_t count, const uint32_t *count_ptr, uint32_t *sums) {
     const uint32_t n = count_ptr ? *count_ptr : count;
     const uint32_t base = blockIdx.x * kScanTile;
+    if (base > n) return;
     uint32_t s = 0;
     for (uint32_t k = 0; k < kScanItems; ++k) {
         uint32_t i = base + k * kScanBlock + threadIdx.x;
@@ -194,7 +200,7 @@ __global__ void k_scan_reduce(const uint32_t *in, uint32_t count, const uint32_t
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-__global__ void k_scan_sums(uint32_t *sums, uint32_t blocks, uint32_t *total_out) {
+__global__ void k_scan_sums(uint32_t *sums, uint32_t blocks) {
     // One block scans up to blocks <= 1024*? sums sequentially in tiles.
     __shared__ uint32_t carry;
     if (threadIdx.x == 0) carry = 0;
@@ -209,13 +215,25 @@ __global__ void k_scan_sums(uint32_t *sums, uint32_t blocks, uint32_t *total_out
         if (threadIdx.x == 0) carry += total;
         __syncthreads();
     }
-    if (threadIdx.x == 0 && total_out) *total_out = carry;
 }
 
-__global__ void k_scan_apply(const uint32_t *in, uint32_t *out, uint32_t count, const uint32_t *count_ptr,
-                             const uint32_t *sums) {
+// kScanned: the totals are scanned already.
+template <bool kScanned>
+__global__ void __launch_bounds__(kScanBlock) k_scan_apply(const uint32_t *in, uint32_t *out, uint32_t count,
+                                                           const uint32_t *count_ptr, const uint32_t *sums,
+                                                           uint32_t *total_out) {
     const uint32_t n = count_ptr ? *count_ptr : count;
-    const uint32_t base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+    const uint32_t first = blockIdx.x * kScanTile;
+    if (first > n) return;
+    uint32_t before = 0;
+    if (kScanned) {
+        before = sums[blockIdx.x];
+    } else {
+        uint32_t part = 0;
+        for (uint32_t k = threadIdx.x; k < blockIdx.x; k += kScanBlock) part += sums[k];
+        block_exclusive(part, &before);
+    }
+    const uint32_t base = first + threadIdx.x * kScanItems;
     uint32_t v[kScanItems], s = 0;
     for (uint32_t k = 0; k < kScanItems; ++k) {
         uint32_t i = base + k;
@@ -223,28 +241,73 @@ __global__ void k_scan_apply(const uint32_t *in, uint32_t *out, uint32_t count, 
         s += v[k];
     }
     uint32_t total;
-    uint32_t ex = block_exclusive(s, &total) + sums[blockIdx.x];
+    uint32_t ex = block_exclusive(s, &total) + before;
     for (uint32_t k = 0; k < kScanItems; ++k) {
         uint32_t i = base + k;
-        if (i < n) out[i] = ex;
+        if (i <= n) out[i] = ex;
+        if (i == n && total_out) *total_out = ex;
         ex += v[k];
     }
 }
 
-__global__ void k_scan_tail(const uint32_t *in, uint32_t *out, uint32_t count, const uint32_t *count_ptr) {
+// The whole input in one block, tile by tile: two tiles take what the second
+// launch of the long form would (4 us).
+constexpr uint32_t kScanShort = 8192;
+__global__ void __launch_bounds__(1024) k_scan_short(const uint32_t *in, uint32_t *out, uint32_t count,
+                                                     const uint32_t *count_ptr, uint32_t *total_out) {
+    __shared__ uint32_t s_sums[2][16];
     const uint32_t n = count_ptr ? *count_ptr : count;
-    out[n] = n ? out[n - 1] + in[n - 1] : 0;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t carry = 0;
+    for (uint32_t tile = 0; tile <= n; tile += 1024 * kScanItems) {
+        const uint32_t base = tile + threadIdx.x * kScanItems;
+        uint32_t v[kScanItems], s = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kScanItems; ++k) {
+            v[k] = base + k < n ? in[base + k] : 0u;
+            s += v[k];
+        }
+        uint32_t x = s;
+#pragma unroll
+        for (uint32_t d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d, 64);
+            if (lane >= d) x += y;
+        }
+        uint32_t *sums = s_sums[(tile / (1024 * kScanItems)) & 1u];
+        if (lane == 63) sums[wave] = x;
+        __syncthreads();
+        uint32_t ex = carry + x - s;
+#pragma unroll
+        for (uint32_t w = 0; w < 16; ++w) {
+            if (w < wave) ex += sums[w];
+            carry += sums[w];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kScanItems; ++k) {
+            if (base + k <= n) out[base + k] = ex;
+            if (base + k == n && total_out) *total_out = ex;
+            ex += v[k];
+        }
+    }
 }
 
 PmhResult exclusive_scan(hipStream_t s, const uint32_t *in, uint32_t *out, uint32_t count,
                          const uint32_t *count_ptr, uint32_t *total, DBuf<uint32_t> &tmp) {
     // `count` is the capacity bound when count_ptr is given.
-    const uint32_t blocks = std::max<uint32_t>(1, (count + kScanTile - 1) / kScanTile);
+    if (count <= kScanShort) {
+        k_scan_short<<<1, 1024, 0, s>>>(in, out, count, count_ptr, total);
+        PMH_CHECK(hipGetLastError());
+        return PMH_SUCCESS;
+    }
+    const uint32_t blocks = count / kScanTile + 1;   // out[count] has its thread too
     if (tmp.reserve(blocks) != PMH_SUCCESS) return PMH_ERROR_OUT_OF_DEVICE_MEMORY;
     k_scan_reduce<<<blocks, kScanBlock, 0, s>>>(in, count, count_ptr, tmp.p);
-    k_scan_sums<<<1, kScanBlock, 0, s>>>(tmp.p, blocks, total);
-    k_scan_apply<<<blocks, kScanBlock, 0, s>>>(in, out, count, count_ptr, tmp.p);
-    k_scan_tail<<<1, 1, 0, s>>>(in, out, count, count_ptr);
+    if (blocks <= 4096u) {
+        k_scan_apply<false><<<blocks, kScanBlock, 0, s>>>(in, out, count, count_ptr, tmp.p, total);
+    } else {
+        k_scan_sums<<<1, kScanBlock, 0, s>>>(tmp.p, blocks);
+        k_scan_apply<true><<<blocks, kScanBlock, 0, s>>>(in, out, count, count_ptr, tmp.p, total);
+    }
     PMH_CHECK(hipGetLastError());
     return PMH_SUCCESS;
 }
@@ -844,17 +907,27 @@ __global__ void k_color_place(uint32_t n, const uint32_t *color, const uint32_t 
 }
 
 // Per colour position: the body's contact points in list order.
+// Eight lanes per position take its manifolds: each manifold is a chain of
+// loads (list, manifold, its points and bodies, the other's colour), and one
+// thread after the other's chain bounded these (1000 bodies of a heap: 8 and 43
+// us, now 4 and 5; 32768: 64 us for the second, now 14).
+constexpr uint32_t kFillLanes = 8;
 __global__ void k_bp_count(uint32_t n, const StepCounters *ctr, const uint32_t *start, const uint32_t *bodies,
                            const uint32_t *adj_start, const uint32_t *adj, const uint32_t *m_count,
                            uint32_t *bp_count) {
     const uint32_t D = start[ctr->colors];
-    uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t t = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const uint32_t k = uint32_t(t / kFillLanes), q = uint32_t(t % kFillLanes);
     if (k >= n) return;
     const uint32_t i = k < D ? bodies[k] : kInvalid;
-    if (i == kInvalid) { bp_count[k] = 0; return; }
     uint32_t s = 0;
-    for (uint32_t e = adj_start[i]; e < adj_start[i + 1]; ++e) s += m_count[adj[e]];
-    bp_count[k] = s;
+    if (i != kInvalid) {
+        const uint32_t last = adj_start[i + 1];
+        for (uint32_t e = adj_start[i] + q; e < last; e += kFillLanes) s += m_count[adj[e]];
+    }
+#pragma unroll
+    for (uint32_t d = 1; d < kFillLanes; d <<= 1) s += __shfl_xor(s, d, kFillLanes);
+    if (q == 0) bp_count[k] = s;
 }
 
 __global__ void k_bp_fill(const StepCounters *ctr, const uint32_t *start, const uint32_t *bodies,
@@ -862,24 +935,39 @@ __global__ void k_bp_fill(const StepCounters *ctr, const uint32_t *start, const 
                           const uint32_t *m_start, const uint2 *ab, const uint32_t *bp_start, uint2 *entries,
                           uint32_t *c_entry, const uint32_t *color) {
     const uint32_t D = start[ctr->colors];
-    uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t t = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const uint32_t k = uint32_t(t / kFillLanes), q = uint32_t(t % kFillLanes);
     if (k >= D) return;
     const uint32_t i = bodies[k];
     if (i == kInvalid) return;
-    const uint32_t ci = color[i];
-    uint32_t o = bp_start[k];
-    for (uint32_t e = adj_start[i]; e < adj_start[i + 1]; ++e) {
-        const uint32_t m = adj[e];
-        const uint2 p = ab[m];
-        const bool first = p.x == i;
-        const uint32_t other = first ? p.y : p.x;
-        // Only dynamic bodies hold a colour.
-        const uint32_t co = color[other];
-        const uint32_t tag = other | (co == kInvalid ? kEntryFixed : co < ci ? kEntryLower : 0u);
-        for (uint32_t q = 0; q < m_count[m]; ++q) {
-            c_entry[2 * (m_start[m] + q) + (first ? 0u : 1u)] = o;
-            entries[o++] = make_uint2((m_start[m] + q) | (first ? kSideFirst : 0u), tag);
+    const uint32_t ci = color[i], last = adj_start[i + 1];
+    uint32_t at = bp_start[k];
+    for (uint32_t base = adj_start[i]; base < last; base += kFillLanes) {
+        uint32_t count = 0, point = 0, tag = 0;
+        bool first = false;
+        if (base + q < last) {
+            const uint32_t m = adj[base + q];
+            count = m_count[m];
+            point = m_start[m];
+            const uint2 p = ab[m];
+            first = p.x == i;
+            const uint32_t other = first ? p.y : p.x;
+            // Only dynamic bodies hold a colour.
+            const uint32_t co = color[other];
+            tag = other | (co == kInvalid ? kEntryFixed : co < ci ? kEntryLower : 0u);
         }
+        uint32_t incl = count;
+#pragma unroll
+        for (uint32_t d = 1; d < kFillLanes; d <<= 1) {
+            const uint32_t y = __shfl_up(incl, d, kFillLanes);
+            if (q >= d) incl += y;
+        }
+        const uint32_t o = at + incl - count;
+        for (uint32_t c = 0; c < count; ++c) {
+            c_entry[2 * (point + c) + (first ? 0u : 1u)] = o + c;
+            entries[o + c] = make_uint2((point + c) | (first ? kSideFirst : 0u), tag);
+        }
+        at += __shfl(incl, kFillLanes - 1, kFillLanes);
     }
 }
 
@@ -1545,9 +1633,9 @@ __device__ __forceinline__ PmhRigidBodyState pose_from(const SolveArgs &a, uint3
 // order per row as the reference.
 //
 // What bounded the sweep over chains was this code: 23 KB, unrolled over
-// axes, kinds of row and types, run once per body from a cold instruction
-// cache, with loads in its branches and the other end's id, colour,
-// displacement and w each a dependent trip to memory.  A sweep over
+// axes, kinds of row and types, with half of it for the pose at the step's
+// start, loads in its branches, and the other end's id, colour, displacement
+// and w each a dependent trip to memory.  A sweep over
 // 16 chains of 16 links (32 lanes) took 105 us, now 59; over 1024 chains of 64
 // (8 lanes) 256 us, now 145; their dual updates 13 and 29 us, now 9 and 22.
 // ---------------------------------------------------------------------
@@ -2805,7 +2893,8 @@ __global__ void k_residual_reset(ResidualLog *log) {
 }
 
 __global__ void k_schedule_init(PmhContactSchedule *s, StepCounters *ctr, uint32_t budget, uint32_t profile,
-                                uint32_t base_iterations, uint32_t reset_status) {
+                                uint32_t base_iterations, uint32_t reset_status, uint32_t *color_count) {
+    for (uint32_t k = threadIdx.x; k <= kMaxColors; k += blockDim.x) color_count[k] = 0u;
     if (threadIdx.x != 0) return;
     if (reset_status) ctr->status = 0;
     ctr->color_abort = 0;
@@ -3185,7 +3274,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
     const uint32_t jg = grid_for(std::max<uint32_t>(1, v.nj), 256, 0xffffffffu);
     const uint32_t eg = grid_for(std::max<uint32_t>(1, 2 * v.nj), 256, 0xffffffffu);   // one thread per joint end
     k_schedule_init<<<1, 64, 0, s>>>(v.schedule.p, ctr, budget, sp.profile, sp.base_iterations,
-                                     sp.reset_status ? 1u : 0u);
+                                     sp.reset_status ? 1u : 0u, v.color_count.p);
     k_residual_reset<<<32, 256, 0, s>>>(v.residual.p);
     k_body_init<<<bg, 256, 0, s>>>(n, P, previous, states, dt, sp.gravity, v.tpos.p, v.tq.p, v.tv.p, v.tw.p,
                                    v.disp.p, v.dq.p, v.inertia.p, v.prev_vel.p, v.color.p, v.parent.p,
@@ -3262,7 +3351,6 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
         k_color_wave<<<blocks, 64 * kColorWaveBlock, 0, s>>>(n, P, v.ab.p, v.adj_start.p, v.adj.p, v.color.p, v.jstart.p, v.jent.p,
                                             v.nj != 0, ctr, sp.color_wait_limit);
     }
-    PMH_CHECK(hipMemsetAsync(v.color_count.p, 0, sizeof(uint32_t) * (kMaxColors + 1), s));
     k_color_count<<<bg, 256, 0, s>>>(n, v.color.p, v.color_count.p);
     k_color_scan<<<1, 64, 0, s>>>(v.color_count.p, v.color_start.p, ctr, v.color_bodies.p, 64u / sp.lanes);
     k_color_place<<<bg, 256, 0, s>>>(n, v.color.p, v.color_start.p, v.color_count.p, v.color_bodies.p);
@@ -3270,7 +3358,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
     // colour-ordered point lists (deg array reused as the per-position count)
     // The degree array is free again once the adjacency is built (the
     // fill cursor keeps each body's degree): it holds the point counts.
-    const uint32_t sg = grid_for(v.slots, 256, 0xffffffffu);
+    const uint32_t sg = uint32_t((uint64_t(v.slots) * kFillLanes + 255) / 256);
     k_bp_count<<<sg, 256, 0, s>>>(v.slots, ctr, v.color_start.p, v.color_bodies.p, v.adj_start.p, v.adj.p,
                                   v.m_count.p, v.deg.p);
     r = exclusive_scan(s, v.deg.p, v.bp_start.p, v.slots, nullptr, nullptr, v.scan_tmp);

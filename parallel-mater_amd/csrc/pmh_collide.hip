@@ -59,8 +59,10 @@ __global__ void k_integrate_proxy(uint32_t n, const PmhBodyParameters *P, const 
                                   PmhRigidBodyState *pred, float4 *pmn, float4 *pmx, V3 g, float dt,
                                   float4 *inputs, const PmhRigidBodyState *targets, uint32_t *target_flags,
                                   uint32_t remaining, uint32_t first_substep, uint32_t last_substep,
-                                  StepCounters *ctr) {
+                                  uint32_t *bucket_count, uint32_t buckets) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    // The hash table's counts, which the next kernel adds to.
+    for (uint32_t k = i; k < buckets; k += gridDim.x * blockDim.x) bucket_count[k] = 0u;
     if (i >= n) return;
     const PmhBodyParameters b = P[i];
     const PmhRigidBodyState s0 = cur[i];
@@ -137,7 +139,6 @@ __global__ void k_integrate_proxy(uint32_t n, const PmhBodyParameters *P, const 
     const V3 mx = add(cmax(sv(s0.position), sv(s.position)), e);
     pmn[i] = f4(mn, 0.0f);
     pmx[i] = f4(mx, 0.0f);
-    (void)ctr;
 }
 
 // ---------------------------------------------------------------------
@@ -177,13 +178,13 @@ __global__ void k_bp_cells(uint32_t n, const float4 *pmn, const float4 *pmx, int
 // tests of a candidate (cell, dynamic flag, box), so the query reads those
 // records by entry index instead of gathering them by body index.
 __global__ void k_bp_scatter(uint32_t n, const PmhBodyParameters *P, const float4 *pmn, const float4 *pmx,
-                             const int4 *cell_of, const uint32_t *bucket_start, uint32_t *cursor, int4 *entry_cell,
+                             const int4 *cell_of, const uint32_t *bucket_start, uint32_t *count, int4 *entry_cell,
                              float4 *entry_mn, float4 *entry_mx) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int4 c = cell_of[i];
     if (c.x == kLargeCell) return;
-    const uint32_t e = bucket_start[c.w] + atomicAdd(&cursor[c.w], 1u);
+    const uint32_t e = bucket_start[c.w] + atomicSub(&count[c.w], 1u) - 1u;
     const float4 mn = pmn[i];
     entry_cell[e] = make_int4(c.x, c.y, c.z, P[i].motion == kDynamic ? 1 : 0);
     entry_mn[e] = make_float4(mn.x, mn.y, mn.z, __uint_as_float(i));
@@ -3172,7 +3173,7 @@ PmhResult World::step_once(uint32_t k_step, bool warm_infer) {
     k_integrate_proxy<<<bg, 256, 0, s>>>(n, params.p, shapes_dev.p, cur, prev, pred, proxy_mn.p, proxy_mx.p,
                                          gravity, dt, inputs_dev.p, targets_dev.p, target_flags_dev.p,
                                          substeps - substep, substep == 0 ? 1u : 0u,
-                                         substep + 1 == substeps ? 1u : 0u, ctr);
+                                         substep + 1 == substeps ? 1u : 0u, bucket_count.p, table_size + 1);
     mark(1);
     JointFilter jf;
     SceneRules rules;
@@ -3194,12 +3195,10 @@ PmhResult World::step_once(uint32_t k_step, bool warm_infer) {
         jf.joints = joints_dev.p;
     }
     // Broadphase.
-    PMH_CHECK(hipMemsetAsync(bucket_count.p, 0, sizeof(uint32_t) * (table_size + 1), s));
     k_bp_cells<<<bg, 256, 0, s>>>(n, proxy_mn.p, proxy_mx.p, cell_of.p, bucket_count.p, table_size - 1,
                                   large.p, ctr, grid_cell);
     PmhResult r = exclusive_scan(s, bucket_count.p, bucket_start.p, table_size, nullptr, nullptr, v.scan_tmp);
     if (r != PMH_SUCCESS) return r;
-    PMH_CHECK(hipMemsetAsync(bucket_count.p, 0, sizeof(uint32_t) * table_size, s));
     k_bp_scatter<<<bg, 256, 0, s>>>(n, params.p, proxy_mn.p, proxy_mx.p, cell_of.p, bucket_start.p, bucket_count.p,
                                     entry_cell.p, entry_mn.p, entry_mx.p);
     if (jf.scene) {
