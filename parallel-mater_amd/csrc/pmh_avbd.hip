@@ -10,14 +10,14 @@
 // body takes the smallest colour its lower-index neighbours do not use,
 // exactly the reference's serial greedy result.
 //
-// Solve (solve_avbd_kernel, geometry_constraints_solve.slang:771-865) is
-// one cooperative launch: budget x (colours + dual pass) separated by grid
-// barriers.  Each body of the active colour is owned by a group of L lanes
-// of a wavefront; the lanes gather the body's contact rows from a
-// colour-ordered CSR list, each accumulating a partial 6x6 block, and the
-// partial blocks meet in an xor-butterfly over the group.  The block is
-// then solved in registers by an unrolled LDL^T.  Per-point Jacobians are
-// computed once per phase (they only depend on the target poses).
+// Solve (solve_avbd_kernel, geometry_constraints_solve.slang:771-865): one
+// dataflow sweep per iteration over all colours (k_sweep; one launch per
+// colour or one cooperative launch on request).  Each body is owned by a
+// group of L lanes of a wavefront; the lanes gather the body's contact rows
+// from a colour-ordered CSR list, each accumulating a partial 6x6 block, and
+// the partial blocks meet in a butterfly over the group.  The block's LDL^T
+// is spread over a row of lanes.  Per-point Jacobians are computed once per
+// phase (they only depend on the target poses).
 #include "pmh_internal.hpp"
 #include "pmh_lanes.hpp"
 #include "pmh_warmstart.hpp"

@@ -14,12 +14,13 @@
 // code a*n+b.  The overlap test is the same comparison on the same floats,
 // so the pair set and order equal the reference's bit for bit.
 //
-// Narrowphase: one thread per pair; convex meshes with <= 96 indices take
-// the reference's SAT + face clipping path (rigid_convex_face_manifold and
-// its swept variant, geometry.slang:1606-1853); analytic spheres/capsules
-// use closed forms.  Mesh pairs the face path declines take the
-// triangle-pair path (leaf-pair candidates or BVH traversal) in a second
-// kernel over a compact list of those pairs.
+// Narrowphase: analytic spheres/capsules use closed forms, one thread per
+// pair; convex meshes with <= 96 indices take the reference's SAT + face
+// clipping path (rigid_convex_face_manifold and its swept variant,
+// geometry.slang:1606-1853) on 16 lanes per pair.  Mesh pairs the face path
+// declines take the triangle-pair path (leaf-pair candidates or BVH
+// traversal): a screen of the leaf bounds, one thread per pair, then a
+// wavefront or a block per pair that is left.
 #include "pmh_internal.hpp"
 #include "pmh_lanes.hpp"
 #include "pmh_world.hpp"
