@@ -8,8 +8,11 @@
 // point from 16 features computed at contact preparation.  Trained on the
 // GPU by the kernels below from contact samples that plain AVBD logs.
 //
-// Every product is a 16x16 MFMA tile C += A(16 x K) B(K x 16); one-pass
-// kernels read the operands from LDS through strides, training from rows.
+// Every product is a 16x16 MFMA tile C += A(16 x K) B(K x 16).  The forward
+// passes and training read both operands as padded rows along K, four values
+// in one 8-byte LDS access (200000 rows forward: 143 us with 2-byte reads at
+// strides whose rows share a bank, now 101); the gradients of one minibatch
+// read transposed operands through strides.
 // Lane l supplies A[l % 16][k0 + 4(l / 16) + j] and B[k0 + 4(l / 16) + j][l % 16]
 // (j = 0..3) and receives C[4(l / 16) + e][l % 16] (e = 0..3).
 
@@ -53,24 +56,38 @@ __device__ __forceinline__ f32x4 mma_tile(const uint16_t *A, int sai, int sak, c
     return acc;
 }
 
+constexpr int kRow = 68;                       // halves per 64-wide row: 34 banks apart
+constexpr int kNarrow = 20;                    // halves per 16-wide row
+// One tile: rows of A and rows of B (the right operand transposed), both along K.
+template <int K>
+__device__ __forceinline__ f32x4 mma_rows(const uint16_t *A, int sa, const uint16_t *B, int sb, f32x4 acc) {
+    const int l = threadIdx.x & 63, r = l & 15, q = (l >> 4) * 4;
+#pragma unroll
+    for (int k0 = 0; k0 < K; k0 += 16) {
+        const bf16x4 a = *reinterpret_cast<const bf16x4 *>(A + r * sa + k0 + q);
+        const bf16x4 b = *reinterpret_cast<const bf16x4 *>(B + r * sb + k0 + q);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    }
+    return acc;
+}
 // Operands of one 64-sample pass, bf16 in LDS.
-struct MlpShared {
-    uint16_t w1[kMlpHidden * kMlpIn];          // [out][in]
-    uint16_t w2[kMlpHidden * kMlpHidden];      // [out][in]
-    uint16_t w3[16 * kMlpHidden];              // [out][in], rows 2..15 zero
+struct alignas(16) MlpShared {
+    uint16_t w1[kMlpHidden * kNarrow];         // [out][in]
+    uint16_t w2[kMlpHidden * kRow];            // [out][in]
+    uint16_t w3[16 * kRow];                    // [out][in], rows 2..15 zero
     float b1[kMlpHidden], b2[kMlpHidden], b3[16];
-    uint16_t x[64 * kMlpIn];                   // [sample][feature]
-    uint16_t h1[64 * kMlpHidden], h2[64 * kMlpHidden];
+    uint16_t x[64 * kNarrow];                  // [sample][feature]
+    uint16_t h1[64 * kRow], h2[64 * kRow];
     uint16_t dy[64 * 16];                      // [sample][out], cols 2..15 zero
-    uint16_t dz2[64 * kMlpHidden], dz1[64 * kMlpHidden];
+    uint16_t dz2[64 * kRow], dz1[64 * kRow];
     float y[64 * kMlpOut], t[64 * kMlpOut];
 };
 
 __device__ void load_weights(MlpShared &S, const float *p) {
     const int l = threadIdx.x;
-    for (int k = l; k < kMlpHidden * kMlpIn; k += 64) S.w1[k] = to_bf16(p[kMlpW1 + k]);
-    for (int k = l; k < kMlpHidden * kMlpHidden; k += 64) S.w2[k] = to_bf16(p[kMlpW2 + k]);
-    for (int k = l; k < 16 * kMlpHidden; k += 64) S.w3[k] = k < kMlpOut * kMlpHidden ? to_bf16(p[kMlpW3 + k]) : 0;
+    for (int k = l; k < kMlpHidden * kMlpIn; k += 64) S.w1[k / kMlpIn * kNarrow + k % kMlpIn] = to_bf16(p[kMlpW1 + k]);
+    for (int k = l; k < kMlpHidden * kMlpHidden; k += 64) S.w2[k / kMlpHidden * kRow + k % kMlpHidden] = to_bf16(p[kMlpW2 + k]);
+    for (int k = l; k < 16 * kMlpHidden; k += 64) S.w3[k / kMlpHidden * kRow + k % kMlpHidden] = k < kMlpOut * kMlpHidden ? to_bf16(p[kMlpW3 + k]) : 0;
     for (int k = l; k < kMlpHidden; k += 64) {
         S.b1[k] = p[kMlpB1 + k];
         S.b2[k] = p[kMlpB2 + k];
@@ -84,29 +101,28 @@ __device__ void forward(MlpShared &S) {
     for (int mi = 0; mi < 4; ++mi)
         for (int nj = 0; nj < 4; ++nj) {
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            acc = mma_tile(S.x + mi * 16 * kMlpIn, kMlpIn, 1, S.w1 + nj * 16 * kMlpIn, 1, kMlpIn, kMlpIn, acc);
+            acc = mma_rows<kMlpIn>(S.x + mi * 16 * kNarrow, kNarrow, S.w1 + nj * 16 * kNarrow, kNarrow, acc);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int s = mi * 16 + q + e, o = nj * 16 + r;
-                S.h1[s * kMlpHidden + o] = to_bf16(fmaxf(acc[e] + S.b1[o], 0.0f));
+                S.h1[s * kRow + o] = to_bf16(fmaxf(acc[e] + S.b1[o], 0.0f));
             }
         }
     __syncthreads();
     for (int mi = 0; mi < 4; ++mi)
         for (int nj = 0; nj < 4; ++nj) {
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            acc = mma_tile(S.h1 + mi * 16 * kMlpHidden, kMlpHidden, 1, S.w2 + nj * 16 * kMlpHidden, 1, kMlpHidden,
-                           kMlpHidden, acc);
+            acc = mma_rows<kMlpHidden>(S.h1 + mi * 16 * kRow, kRow, S.w2 + nj * 16 * kRow, kRow, acc);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int s = mi * 16 + q + e, o = nj * 16 + r;
-                S.h2[s * kMlpHidden + o] = to_bf16(fmaxf(acc[e] + S.b2[o], 0.0f));
+                S.h2[s * kRow + o] = to_bf16(fmaxf(acc[e] + S.b2[o], 0.0f));
             }
         }
     __syncthreads();
     for (int mi = 0; mi < 4; ++mi) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        acc = mma_tile(S.h2 + mi * 16 * kMlpHidden, kMlpHidden, 1, S.w3, 1, kMlpHidden, kMlpHidden, acc);
+        acc = mma_rows<kMlpHidden>(S.h2 + mi * 16 * kRow, kRow, S.w3, kRow, acc);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int s = mi * 16 + q + e;
@@ -139,7 +155,7 @@ __device__ float backward(MlpShared &S, uint32_t count, float *g) {
     // dW3 = dY^T H2, db3
     for (int nj = 0; nj < 4; ++nj) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        acc = mma_tile(S.dy, 1, 16, S.h2 + nj * 16, kMlpHidden, 1, 64, acc);
+        acc = mma_tile(S.dy, 1, 16, S.h2 + nj * 16, kRow, 1, 64, acc);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (q + e < kMlpOut) g[kMlpW3 + (q + e) * kMlpHidden + nj * 16 + r] = acc[e];
@@ -153,11 +169,11 @@ __device__ float backward(MlpShared &S, uint32_t count, float *g) {
     for (int mi = 0; mi < 4; ++mi)
         for (int nj = 0; nj < 4; ++nj) {
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            acc = mma_tile(S.dy + mi * 16 * 16, 16, 1, S.w3 + nj * 16, kMlpHidden, 1, 16, acc);
+            acc = mma_tile(S.dy + mi * 16 * 16, 16, 1, S.w3 + nj * 16, kRow, 1, 16, acc);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int s = mi * 16 + q + e, o = nj * 16 + r;
-                S.dz2[s * kMlpHidden + o] = from_bf16(S.h2[s * kMlpHidden + o]) > 0.0f ? to_bf16(acc[e]) : 0;
+                S.dz2[s * kRow + o] = from_bf16(S.h2[s * kRow + o]) > 0.0f ? to_bf16(acc[e]) : 0;
             }
         }
     __syncthreads();
@@ -165,38 +181,37 @@ __device__ float backward(MlpShared &S, uint32_t count, float *g) {
     for (int mi = 0; mi < 4; ++mi)
         for (int nj = 0; nj < 4; ++nj) {
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            acc = mma_tile(S.dz2 + mi * 16, 1, kMlpHidden, S.h1 + nj * 16, kMlpHidden, 1, 64, acc);
+            acc = mma_tile(S.dz2 + mi * 16, 1, kRow, S.h1 + nj * 16, kRow, 1, 64, acc);
 #pragma unroll
             for (int e = 0; e < 4; ++e) g[kMlpW2 + (mi * 16 + q + e) * kMlpHidden + nj * 16 + r] = acc[e];
         }
     {
         float b = 0.0f;
-        for (int s = 0; s < 64; ++s) b += from_bf16(S.dz2[s * kMlpHidden + l]);
+        for (int s = 0; s < 64; ++s) b += from_bf16(S.dz2[s * kRow + l]);
         g[kMlpB2 + l] = b;
     }
     // dZ1 = (dZ2 W2) .* [H1 > 0]
     for (int mi = 0; mi < 4; ++mi)
         for (int nj = 0; nj < 4; ++nj) {
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            acc = mma_tile(S.dz2 + mi * 16 * kMlpHidden, kMlpHidden, 1, S.w2 + nj * 16, kMlpHidden, 1, kMlpHidden,
-                           acc);
+            acc = mma_tile(S.dz2 + mi * 16 * kRow, kRow, 1, S.w2 + nj * 16, kRow, 1, kMlpHidden, acc);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int s = mi * 16 + q + e, o = nj * 16 + r;
-                S.dz1[s * kMlpHidden + o] = from_bf16(S.h1[s * kMlpHidden + o]) > 0.0f ? to_bf16(acc[e]) : 0;
+                S.dz1[s * kRow + o] = from_bf16(S.h1[s * kRow + o]) > 0.0f ? to_bf16(acc[e]) : 0;
             }
         }
     __syncthreads();
     // dW1 = dZ1^T X, db1
     for (int mi = 0; mi < 4; ++mi) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        acc = mma_tile(S.dz1 + mi * 16, 1, kMlpHidden, S.x, kMlpIn, 1, 64, acc);
+        acc = mma_tile(S.dz1 + mi * 16, 1, kRow, S.x, kNarrow, 1, 64, acc);
 #pragma unroll
         for (int e = 0; e < 4; ++e) g[kMlpW1 + (mi * 16 + q + e) * kMlpIn + r] = acc[e];
     }
     {
         float b = 0.0f;
-        for (int s = 0; s < 64; ++s) b += from_bf16(S.dz1[s * kMlpHidden + l]);
+        for (int s = 0; s < 64; ++s) b += from_bf16(S.dz1[s * kRow + l]);
         g[kMlpB1 + l] = b;
     }
     // summed squared error over the wave
@@ -210,7 +225,7 @@ __device__ void load_samples(MlpShared &S, const float *samples, uint32_t first,
     const int l = threadIdx.x;
     const bool live = uint32_t(l) < count;
     const float *row = samples + size_t(first + (live ? l : 0)) * kMlpSample;
-    for (int f = 0; f < kMlpIn; ++f) S.x[l * kMlpIn + f] = live ? to_bf16(row[f]) : 0;
+    for (int f = 0; f < kMlpIn; ++f) S.x[l * kNarrow + f] = live ? to_bf16(row[f]) : 0;
     for (int o = 0; o < kMlpOut; ++o) S.t[l * kMlpOut + o] = live ? row[kMlpIn + o] : 0.0f;
     __syncthreads();
 }
@@ -239,10 +254,8 @@ __global__ void __launch_bounds__(64) k_mlp_gradients(const float *samples, uint
 // operands and the parameters in memory took 85 us per minibatch, this 7.1
 // (8.3 with the samples' indices looked up in the stage that needs them and
 // the bias corrections' powers after the update).
-constexpr int kRow = 68;                       // halves per 64-wide row: 34 banks apart
-constexpr int kNarrow = 20;                    // halves per 16-wide row
 constexpr int kTrainThreads = 1024;
-struct TrainShared {
+struct alignas(16) TrainShared {
     // weights: [out][in], and transposed where the backward pass reads them along out
     uint16_t w1[kMlpHidden * kNarrow], w2[kMlpHidden * kRow], w2t[kMlpHidden * kRow], w3[16 * kRow],
         w3t[kMlpHidden * kNarrow];
@@ -255,18 +268,6 @@ struct TrainShared {
     float c1, c2;                              // Adam's bias corrections of the step
 };
 
-// One tile: rows of A and rows of B (the right operand transposed), both along K.
-template <int K>
-__device__ __forceinline__ f32x4 mma_rows(const uint16_t *A, int sa, const uint16_t *B, int sb, f32x4 acc) {
-    const int l = threadIdx.x & 63, r = l & 15, q = (l >> 4) * 4;
-#pragma unroll
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        const bf16x4 a = *reinterpret_cast<const bf16x4 *>(A + r * sa + k0 + q);
-        const bf16x4 b = *reinterpret_cast<const bf16x4 *>(B + r * sb + k0 + q);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-    }
-    return acc;
-}
 // Four values of a column (rows q .. q + 3) into [row][column] and, as one
 // 8-byte store, into [column][row].
 __device__ __forceinline__ void put_tile(uint16_t *rows, uint16_t *cols, int row, int col, const uint16_t *v) {
@@ -525,7 +526,7 @@ __global__ void __launch_bounds__(64) k_mlp_infer(const uint32_t *count_ptr, con
     for (uint32_t first = blockIdx.x * 64; first < total; first += gridDim.x * 64) {
         const uint32_t count = min(64u, total - first);
         const bool live = uint32_t(l) < count;
-        for (int f = 0; f < kMlpIn; ++f) S.x[l * kMlpIn + f] = live ? to_bf16(feat[size_t(first + l) * kMlpIn + f]) : 0;
+        for (int f = 0; f < kMlpIn; ++f) S.x[l * kNarrow + f] = live ? to_bf16(feat[size_t(first + l) * kMlpIn + f]) : 0;
         __syncthreads();
         forward(S);
         if (live) {
@@ -571,7 +572,7 @@ __global__ void __launch_bounds__(64) k_mlp_forward(const float *x, uint32_t n, 
     for (uint32_t first = blockIdx.x * 64; first < n; first += gridDim.x * 64) {
         const uint32_t count = min(64u, n - first);
         const bool live = uint32_t(l) < count;
-        for (int f = 0; f < kMlpIn; ++f) S.x[l * kMlpIn + f] = live ? to_bf16(x[size_t(first + l) * kMlpIn + f]) : 0;
+        for (int f = 0; f < kMlpIn; ++f) S.x[l * kNarrow + f] = live ? to_bf16(x[size_t(first + l) * kMlpIn + f]) : 0;
         __syncthreads();
         forward(S);
         if (live)
