@@ -94,7 +94,7 @@ constexpr uint32_t kFlowUsed = 7;
 constexpr int kLoadAgent = 16;   // buffer load cache policy: sc1
 typedef uint32_t flow_pair __attribute__((ext_vector_type(4)));   // two words: value, stamp, value, stamp
 __device__ __forceinline__ flow_pair flow_load(__amdgpu_buffer_rsrc_t box, uint32_t body, int pair) {
-    return __builtin_amdgcn_raw_buffer_load_b128(box, int(body * (kFlowWords * 8u)), 16 * pair, kLoadAgent);
+    return __builtin_amdgcn_raw_buffer_load_b128(box, int(flow_offset(body)), 16 * pair, kLoadAgent);
 }
 
 // Sum over a converged wavefront (every lane active).
@@ -1123,7 +1123,7 @@ __device__ __forceinline__ void load_disp(const float4 *disp, uint32_t i, float 
     d[0] = a.x; d[1] = a.y; d[2] = a.z; d[3] = b.x; d[4] = b.y; d[5] = b.z;
 }
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t flow_box(const SolveArgs &a) {
-    return __builtin_amdgcn_make_buffer_rsrc(a.flow, 0, int(a.n * (kFlowWords * 8u)), 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(a.flow, 0, int(flow_offset(a.n)), 0x00020000);
 }
 
 // Dataflow sweep: waits until body j has published this sweep's displacement
@@ -3104,7 +3104,7 @@ PmhResult Solver::each_buffer(uint32_t bodies, uint32_t pairs, uint32_t points, 
     R(color_bodies, positions); R(bp_start, positions + 1); R(anchored, bodies); R(mean, bodies);
     R(members, bodies); R(mean_list, bodies);
     R(jdeg, bodies + 1); R(jstart, bodies + 1); R(jcursor, bodies); R(joint_head, bodies);
-    R(prev_vel, bodies); R(flow, kFlowWords * (size_t)bodies);
+    R(prev_vel, bodies); R(flow, flow_words(bodies));
     R(code, pairs); R(ab, pairs); R(m_count, pairs + 1); R(m_start, pairs + 1); R(m_slot, pairs + 1);
     R(m_impact, pairs); R(m_face, pairs); R(m_init_rel, pairs); R(adj, 2 * (size_t)pairs);
     R(tri_list, pairs); R(face_list, pairs);
@@ -3121,12 +3121,12 @@ PmhResult Solver::each_buffer(uint32_t bodies, uint32_t pairs, uint32_t points, 
 PmhResult Solver::reserve(uint32_t bodies, uint32_t pairs, uint32_t points) {
     // Zeroed when first allocated: the velocity history, the sweep's
     // mailboxes, the counters and the running totals.
-    const bool fresh_prev = prev_vel.n < bodies, fresh_flow = flow.n < kFlowWords * (size_t)bodies;
+    const bool fresh_prev = prev_vel.n < bodies, fresh_flow = flow.n < flow_words(bodies);
     const bool fresh_ctr = !counters.p, fresh_totals = !totals.p;
     PmhResult r = each_buffer(bodies, pairs, points, [](auto &buf, size_t count) { return buf.reserve(count); });
     if (r != PMH_SUCCESS) return r;
     if (fresh_prev) PMH_CHECK(hipMemset(prev_vel.p, 0, sizeof(float4) * bodies));
-    if (fresh_flow) PMH_CHECK(hipMemset(flow.p, 0, sizeof(unsigned long long) * kFlowWords * bodies));
+    if (fresh_flow) PMH_CHECK(hipMemset(flow.p, 0, sizeof(unsigned long long) * flow_words(bodies)));
     if (fresh_ctr) PMH_CHECK(hipMemset(counters.p, 0, sizeof(StepCounters)));
     if (fresh_totals) PMH_CHECK(hipMemset(totals.p, 0, sizeof(SolveTotals)));
     ecap = 2 * (size_t)points;
@@ -3479,7 +3479,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
         };
         // Dataflow sweep: one launch per iteration, as many resident
         // wavefronts as fit (tickets hand out the positions).
-        const bool flow = sp.dataflow;
+        const bool flow = sp.dataflow && flow_fits(n);
         const uint32_t positions = v.host_color_start[colors];
         auto launch_sweep = [&](SolveArgs &af, uint32_t phase, uint32_t it, hipEvent_t start,
                                 hipEvent_t stop) -> hipError_t {
@@ -3538,7 +3538,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
                 if (flow) {
                     SolveArgs af = a;
                     if (++v.sweep_stamp == 0u) {   // stamps wrapped: no stale stamp may match
-                        PMH_CHECK(hipMemsetAsync(v.flow.p, 0, sizeof(unsigned long long) * kFlowWords * n, s));
+                        PMH_CHECK(hipMemsetAsync(v.flow.p, 0, sizeof(unsigned long long) * flow_words(n), s));
                         v.sweep_stamp = 1u;
                     }
                     af.flow_stamp = v.sweep_stamp;

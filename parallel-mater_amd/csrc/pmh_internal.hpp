@@ -120,6 +120,14 @@ struct SolveTotals {
 
 constexpr uint32_t kMaxBodies = 0x3fffffffu;   // body indices leave two bits of a word for flags
 constexpr uint32_t kFlowWords = 8;             // 64-bit mailbox words per body of the dataflow sweep
+// The sweep reads the mailboxes through one buffer descriptor, whose size and
+// offsets are 32-bit byte counts: 67 108 863 bodies.  One launch per colour
+// needs no mailboxes and takes larger worlds.
+constexpr uint32_t kFlowBytes = kFlowWords * 8u;
+constexpr uint32_t kFlowBodies = 0xffffffffu / kFlowBytes;
+constexpr bool flow_fits(uint32_t bodies) { return bodies <= kFlowBodies; }
+constexpr size_t flow_words(uint32_t bodies) { return flow_fits(bodies) ? kFlowWords * size_t(bodies) : 0; }
+__host__ __device__ constexpr uint32_t flow_offset(uint32_t body) { return body * kFlowBytes; }   // body n: the size
 constexpr uint32_t kMaxColors = 256;
 // A body the colouring gave up on (a wait ran out) holds this value: not a
 // colour, so no solve stage sees it, and published, so nobody waits on it.
