@@ -387,6 +387,12 @@ PmhResult pmhWorldSetColorWaitLimit(PmhWorld world, uint32_t polls);
  * path without a stalled device. */
 PmhResult pmhWorldSetSweepWaitLimit(PmhWorld world, uint32_t polls);
 
+/* Vertices that a clipped polygon of the convex face path may have on a row
+ * of 16 lanes (default and most: 16); wider ones are clipped on one lane, with
+ * the same results.  No counterpart in the reference; a small limit lets a
+ * test take that path with shapes whose polygons hardly ever get there. */
+PmhResult pmhWorldSetFaceRowLimit(PmhWorld world, uint32_t vertices);
+
 /* pmCmdCopyRigidStates / pmCmdSetRigidStates (src/api/resources.cpp:1293;
  * runtime_rigid.cu.inc:147-195: a set-state resets AVBD history and the
  * contact cache). */

@@ -734,35 +734,6 @@ __device__ __forceinline__ PairFrames pair_frames(const HingeFrame *frames, cons
     return f;
 }
 
-// rigid_reduce_face_patch, geometry.slang:1228-1270.
-__device__ void reduce_face_patch(Manifold &m, float tol) {
-    const float t2 = tol * tol;
-    bool removed = true;
-    while (removed) {
-        removed = false;
-        for (uint32_t cand = 0; cand < m.count && !removed; ++cand) {
-            const V3 p = m.c[cand].point;
-            for (uint32_t f = 0; f < m.count && !removed; ++f) {
-                if (f == cand) continue;
-                for (uint32_t s = f + 1; s < m.count; ++s) {
-                    if (s == cand) continue;
-                    const V3 e = sub(m.c[s].point, m.c[f].point);
-                    const float e2 = len2(e);
-                    if (e2 <= t2) continue;
-                    const float t = dot(sub(p, m.c[f].point), e) / e2;
-                    if (t <= 1.0e-4f || t >= 0.9999f) continue;
-                    const V3 cl = add(m.c[f].point, mul(e, t));
-                    if (len2(sub(p, cl)) > t2) continue;
-                    for (uint32_t k = cand + 1; k < m.count; ++k) m.c[k - 1] = m.c[k];
-                    --m.count;
-                    removed = true;
-                    break;
-                }
-            }
-        }
-    }
-}
-
 __device__ float rotational_motion_bound(const PmhRigidBodyState &p, const PmhRigidBodyState &c,
                                          const ShapeDev &s) {
     const Q d = relative_quaternion(sq(p.orientation), sq(c.orientation), false);
@@ -770,168 +741,6 @@ __device__ float rotational_motion_bound(const PmhRigidBodyState &p, const PmhRi
     const V3 ma = {smax(fabsf(s.mn[0]), fabsf(s.mx[0])), smax(fabsf(s.mn[1]), fabsf(s.mx[1])),
                    smax(fabsf(s.mn[2]), fabsf(s.mx[2]))};
     return 2.0f * len(ma) * sh;
-}
-
-// rigid_convex_face_manifold, geometry.slang:1606-1745.
-__device__ bool convex_face_manifold(const PmhRigidBodyState &bs, const ShapeView &bm,
-                                     const PmhRigidBodyState &cs, const ShapeView &cm, float margin,
-                                     float reach_corr, Manifold &out) {
-    out.count = 0;
-    out.face_patch = 0;
-    const float rest = smin(margin, 1.0e-3f);
-    const float reach = margin + reach_corr;
-    float best = -3.402823466e+38f;
-    uint32_t ref_face = 0;
-    bool ref_is_body = false;
-    for (uint32_t side = 0; side < 2; ++side) {
-        const ShapeView &rm = side == 0 ? cm : bm;
-        const PmhRigidBodyState &rs = side == 0 ? cs : bs;
-        const ShapeView &im = side == 0 ? bm : cm;
-        const PmhRigidBodyState &is = side == 0 ? bs : cs;
-        const Q rq = sq(rs.orientation), iq = sq(is.orientation);
-        const V3 rel = sub(sv(is.position), sv(rs.position));
-        for (uint32_t f = 0; f < rm.s.idx_count / 3; ++f) {
-            const float4 pl = rm.plane(f);
-            const V3 nrm = rotate(rq, v3(pl));
-            const V3 inn = inv_rotate(iq, nrm);
-            float support = 3.402823466e+38f;
-            for (uint32_t k = 0; k < im.s.vtx_count; ++k) support = smin(support, dot(inn, im.vert(k)));
-            const float sep = support + dot(nrm, rel) - pl.w;
-            if (sep > best) { best = sep; ref_face = f; ref_is_body = side != 0; }
-        }
-    }
-    if (best > reach) return true;
-    const ShapeView &rm = ref_is_body ? bm : cm;
-    const PmhRigidBodyState &rs = ref_is_body ? bs : cs;
-    const ShapeView &im = ref_is_body ? cm : bm;
-    const PmhRigidBodyState &is = ref_is_body ? cs : bs;
-    const Q rq = sq(rs.orientation);
-    const float4 reference = rm.plane(ref_face);
-    const V3 rn = v3(reference);
-    const V3 outward = rotate(rq, rn);
-    const V3 iaxis = inv_rotate(sq(is.orientation), outward);
-    float alignment = 1.0f;
-    uint32_t inc_face = 0;
-    for (uint32_t f = 0; f < im.s.idx_count / 3; ++f) {
-        const float val = dot(iaxis, v3(im.plane(f)));
-        if (val < alignment) { alignment = val; inc_face = f; }
-    }
-    const V3 normal = mul(outward, ref_is_body ? -1.0f : 1.0f);
-    const float4 incident = im.plane(inc_face);
-    const uint32_t rfaces = rm.s.idx_count / 3;
-    for (uint32_t t = 0; t < im.s.idx_count / 3; ++t) {
-        const float4 face = im.plane(t);
-        if (dot(v3(face), v3(incident)) < 0.99999f || fabsf(face.w - incident.w) > 1.0e-5f) continue;
-        // The polygon is clipped back and forth between two buffers.
-        V3 buf[2][36];
-        V3 *poly = buf[0], *clipped = buf[1];
-        uint32_t count = 3;
-        for (uint32_t c = 0; c < 3; ++c)
-            poly[c] = inv_rotate(rq, sub(transform_point(is, im.vert(im.index(t * 3 + c))), sv(rs.position)));
-        for (uint32_t pi = 0; pi < rfaces && count != 0; ++pi) {
-            const float4 pl = rm.plane(pi);
-            const V3 pn = v3(pl);
-            const float off = pl.w + (dot(pn, rn) > 0.99999f ? reach : 0.0f);
-            uint32_t cc = 0;
-            V3 prev = poly[count - 1];
-            float pd = dot(pn, prev) - off;
-            for (uint32_t k = 0; k < count; ++k) {
-                const V3 cur = poly[k];
-                const float d = dot(pn, cur) - off;
-                if ((d <= 0.0f) != (pd <= 0.0f) && cc < 36)
-                    clipped[cc++] = add(prev, mul(sub(cur, prev), pd / (pd - d)));
-                if (d <= 0.0f && cc < 36) clipped[cc++] = cur;
-                prev = cur;
-                pd = d;
-            }
-            count = cc;
-            V3 *const t_ = poly;
-            poly = clipped;
-            clipped = t_;
-        }
-        for (uint32_t k = 0; k < count; ++k) {
-            const float d = dot(rn, poly[k]) - reference.w;
-            if (d > reach) continue;
-            Contact c;
-            c.normal = normal;
-            c.point = transform_point(rs, sub(poly[k], mul(rn, d * 0.5f)));
-            c.pen = rest - d + 1.0e-5f;
-            c.impact_fraction = 1.0f;
-            add_contact(out, c, smax(margin * 2.0f, 1.0e-4f));
-        }
-    }
-    if (out.count == 0u) return false;
-    reduce_face_patch(out, smax(1.0e-6f, margin * 1.0e-3f));
-    out.face_patch = 1u;
-    return true;
-}
-
-// rigid_swept_convex_face_manifold, geometry.slang:1751-1853.
-__device__ bool swept_convex_face_manifold(const PmhRigidBodyState &pb, const PmhRigidBodyState &b,
-                                           const ShapeView &bm, const PmhRigidBodyState &pc,
-                                           const PmhRigidBodyState &c, const ShapeView &cm, float margin,
-                                           Manifold &out) {
-    out.count = 0;
-    out.face_patch = 0;
-    const Q bd = relative_quaternion(sq(pb.orientation), sq(b.orientation), false);
-    const Q cd = relative_quaternion(sq(pc.orientation), sq(c.orientation), false);
-    if (bd.x != 0.0f || bd.y != 0.0f || bd.z != 0.0f || cd.x != 0.0f || cd.y != 0.0f || cd.z != 0.0f)
-        return false;
-    const V3 bmo = sub(sv(b.position), sv(pb.position)), cmo = sub(sv(c.position), sv(pc.position));
-    const float rest = smin(margin, 1.0e-3f);
-    float entry = 0.0f, exit_time = 1.0f;
-    V3 entry_normal = {0.0f, 0.0f, 0.0f};
-    for (uint32_t side = 0; side < 2; ++side) {
-        const ShapeView &rm = side == 0 ? cm : bm;
-        const ShapeView &im = side == 0 ? bm : cm;
-        const PmhRigidBodyState &rs = side == 0 ? pc : pb;
-        const PmhRigidBodyState &is = side == 0 ? pb : pc;
-        const V3 rel = side == 0 ? sub(bmo, cmo) : sub(cmo, bmo);
-        for (uint32_t f = 0; f < rm.s.idx_count / 3; ++f) {
-            const float4 pl = rm.plane(f);
-            const V3 nrm = rotate(sq(rs.orientation), v3(pl));
-            const V3 inn = inv_rotate(sq(is.orientation), nrm);
-            float support = 3.402823466e+38f;
-            for (uint32_t k = 0; k < im.s.vtx_count; ++k) support = smin(support, dot(inn, im.vert(k)));
-            const float gap = support + dot(nrm, sub(sv(is.position), sv(rs.position))) - pl.w;
-            const float speed = dot(nrm, rel);
-            if (speed == 0.0f) {
-                if (gap > rest) return true;
-            } else {
-                const float crossing = (rest - gap) / speed;
-                if (speed < 0.0f && crossing > entry) {
-                    entry = crossing;
-                    entry_normal = mul(nrm, side == 0 ? 1.0f : -1.0f);
-                }
-                if (speed > 0.0f) exit_time = smin(exit_time, crossing);
-            }
-        }
-    }
-    if (entry > exit_time || entry > 1.0f || exit_time < 0.0f) return true;
-    if (entry == 0.0f) {
-        const bool clipped = convex_face_manifold(b, bm, c, cm, margin, 0.0f, out);
-        if (clipped && out.count != 0u) return true;
-        if (!convex_face_manifold(pb, bm, pc, cm, margin, 0.0f, out) || out.count == 0u) return false;
-        for (uint32_t p = 0; p < out.count; ++p) {
-            const float closing = -dot(sub(bmo, cmo), out.c[p].normal);
-            if (closing <= 0.0f) return false;
-            out.c[p].pen += closing;
-            out.c[p].impact_fraction = 0.0f;
-        }
-        return true;
-    }
-    PmhRigidBodyState ib = pb, ic = pc;
-    ib.position = pv(add(sv(pb.position), mul(bmo, entry)));
-    ic.position = pv(add(sv(pc.position), mul(cmo, entry)));
-    if (!convex_face_manifold(ib, bm, ic, cm, rest + 1.0e-5f, 0.0f, out) || out.count == 0u) return false;
-    for (uint32_t p = 0; p < out.count; ++p) {
-        Contact &ct = out.c[p];
-        if (dot(ct.normal, entry_normal) < 0.99999f) return false;
-        const float remaining = -dot(sub(bmo, cmo), ct.normal) * (1.0f - entry);
-        ct.pen = smax(0.0f, remaining + ct.pen) + rest + 1.0e-5f;
-        ct.impact_fraction = entry;
-    }
-    return true;
 }
 
 __device__ bool requires_swept(const PmhRigidBodyState &pa, const PmhRigidBodyState &a, const ShapeDev &ma,
@@ -1818,11 +1627,13 @@ __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t lan
 // A row of 16 lanes works on one pair, so that a small world's few pairs do
 // not each wait for one lane's serial search: the separating axes run over
 // the lanes, a clipped polygon has one vertex per lane and a manifold one
-// contact per lane.  The results are those of the serial functions above
+// contact per lane.  The results are those of the reference's serial search
 // (the same operations on each value, ties decided by the serial order).
 constexpr uint32_t kFaceLanes = 16;
+constexpr uint32_t kFacePolygon = 36;   // vertices of a clipped polygon (the reference's capacity)
 struct FaceShared {
     float v[kFaceLanes][3];     // polygon vertices on their way to the next plane; contact points
+    float wide[2][kFacePolygon][3];   // a polygon of more vertices than lanes, before and after a plane
 };
 
 __device__ __forceinline__ uint32_t row_bits(bool p) {   // one bit per lane of the row
@@ -1929,7 +1740,7 @@ __device__ __forceinline__ void row_add_contact(RowManifold &m, uint32_t lane, V
     }
 }
 
-// reduce_face_patch for a row: the 28 pairs (f, s) of at most 8 contacts are
+// rigid_reduce_face_patch (geometry.slang:1228-1270) for a row: the 28 pairs (f, s) of at most 8 contacts are
 // shared out over the lanes.
 __device__ __forceinline__ void row_reduce_patch(RowManifold &m, uint32_t lane, FaceShared &S, float tol) {
     const float t2 = tol * tol;
@@ -1972,7 +1783,8 @@ __device__ __forceinline__ void row_reduce_patch(RowManifold &m, uint32_t lane, 
     }
 }
 
-// The separating-axis search of convex_face_manifold for a row: the face of
+// The separating-axis search of rigid_convex_face_manifold
+// (geometry.slang:1606-1745) for a row: the face of
 // the largest separation (the collider's faces first), kFaceApart past reach.
 constexpr uint32_t kFaceApart = 0xffffffffu;
 __device__ __forceinline__ uint32_t row_axis(const FaceGeometry &geo, const FaceSide &body, const FaceSide &collider,
@@ -1994,12 +1806,48 @@ __device__ __forceinline__ uint32_t row_axis(const FaceGeometry &geo, const Face
     return best_at == 0xffffu ? 0u : best_at;
 }
 
-// The rest of convex_face_manifold for a row.  kFaceWide: a clipped polygon
-// grew past one vertex per lane.
-enum : uint32_t { kFaceDeclined = 0, kFaceSolved = 1, kFaceWide = 2 };
-__device__ __forceinline__ uint32_t row_clip(const FaceGeometry &geo, const FaceSide &body, const FaceSide &collider,
-                                             float margin, float reach, uint32_t best_at, uint32_t lane, FaceShared &S,
-                                             RowManifold &out) {
+// Clips the polygon in S.wide[0] by the planes from `pi` on, on one lane;
+// returns its vertices and, in `buf`, the buffer they end in.
+__device__ __forceinline__ uint32_t clip_wide(const float4 *planes, uint32_t pi, uint32_t count_planes, V3 rn, float reach,
+                                              uint32_t count, FaceShared &S, uint32_t &buf) {
+    buf = 0;
+#pragma unroll 1
+    for (; pi < count_planes && count != 0u; ++pi) {
+        const float4 pl = planes[pi];
+        const V3 pn = v3(pl);
+        const float off = pl.w + (dot(pn, rn) > 0.99999f ? reach : 0.0f);
+        float (*const from)[3] = S.wide[buf], (*const to)[3] = S.wide[buf ^ 1u];
+        uint32_t next = 0;
+        V3 prev = {from[count - 1][0], from[count - 1][1], from[count - 1][2]};
+        float pd = dot(pn, prev) - off;
+        auto put = [&](V3 x) {
+            if (next >= kFacePolygon) return;
+            to[next][0] = x.x; to[next][1] = x.y; to[next][2] = x.z;
+            ++next;
+        };
+#pragma unroll 1
+        for (uint32_t k = 0; k < count; ++k) {
+            const V3 cur = {from[k][0], from[k][1], from[k][2]};
+            const float d = dot(pn, cur) - off;
+            if ((d <= 0.0f) != (pd <= 0.0f)) put(add(prev, mul(sub(cur, prev), pd / (pd - d))));
+            if (d <= 0.0f) put(cur);
+            prev = cur;
+            pd = d;
+        }
+        count = next;
+        buf ^= 1u;
+    }
+    return count;
+}
+
+// The rest of rigid_convex_face_manifold for a row; false where it finds no
+// contact.  A polygon that grows past `widest` vertices (at most one per lane)
+// goes on in LDS, its planes on one lane.  A plane adds at most one vertex to
+// a convex polygon, so that is expected of shapes of more than 13 triangles;
+// rounded distances can cut a sliver more than twice in any.
+__device__ __forceinline__ bool row_clip(const FaceGeometry &geo, const FaceSide &body, const FaceSide &collider,
+                                         float margin, float reach, uint32_t best_at, uint32_t widest,
+                                         uint32_t lane, FaceShared &S, RowManifold &out) {
     const float rest = smin(margin, 1.0e-3f);
     const uint32_t nc = collider.faces;
     const bool ref_is_body = best_at >= nc;
@@ -2033,7 +1881,7 @@ __device__ __forceinline__ uint32_t row_clip(const FaceGeometry &geo, const Face
         }
         for (uint32_t todo = row_bits(same); todo != 0u; todo &= todo - 1u) {
             const uint32_t t = t0 + __builtin_ctz(todo);
-            uint32_t count = 3;
+            uint32_t count = 3, wide = 2u;           // 2: one vertex per lane
             V3 cur = {0.0f, 0.0f, 0.0f};
             if (lane < 3u) {
                 const V3 local = geo.verts[im.verts + geo.idx[im.indices + t * 3 + lane]];
@@ -2053,7 +1901,18 @@ __device__ __forceinline__ uint32_t row_clip(const FaceGeometry &geo, const Face
                 const uint32_t before = ((in << 1) | (in >> (count - 1u))) & all;
                 const uint32_t cut = in ^ before;
                 const uint32_t next = __builtin_popcount(in) + __builtin_popcount(cut);
-                if (next > kFaceLanes) return kFaceWide;
+                if (next > widest) {
+                    row_sync();
+                    if (lane < count) {
+                        S.wide[0][lane][0] = cur.x; S.wide[0][lane][1] = cur.y; S.wide[0][lane][2] = cur.z;
+                    }
+                    row_sync();
+                    if (lane == 0u) count = clip_wide(rp, pi, rfaces, rn, reach, count, S, wide);
+                    row_sync();
+                    count = uint32_t(__shfl(int(count), 0, 16));
+                    wide = uint32_t(__shfl(int(wide), 0, 16));
+                    break;
+                }
                 const uint32_t prev_lane = lane == 0u ? count - 1u : lane - 1u;
                 const V3 prev = row_get(cur, prev_lane);
                 const float pd = __shfl(d, int(prev_lane), 16);
@@ -2072,21 +1931,29 @@ __device__ __forceinline__ uint32_t row_clip(const FaceGeometry &geo, const Face
                 count = next;
                 cur = {S.v[lane][0], S.v[lane][1], S.v[lane][2]};
             }
-            const float d = dot(rn, cur) - reference.w;
-            const V3 point = add(rm.pos, rotate(rq, sub(cur, mul(rn, d * 0.5f))));
-            const float pen = rest - d + 1.0e-5f;
-            for (uint32_t keep = row_bits(lane < count && !(d > reach)); keep != 0u; keep &= keep - 1u) {
-                const uint32_t k = __builtin_ctz(keep);
-                row_add_contact(out, lane, row_get(point, k), __shfl(pen, int(k), 16), smax(margin * 2.0f, 1.0e-4f));
+#pragma unroll 1
+            for (uint32_t k0 = 0; k0 < count; k0 += kFaceLanes) {
+                if (wide < 2u) {
+                    const float *q = S.wide[wide][min(k0 + lane, kFacePolygon - 1u)];
+                    cur = {q[0], q[1], q[2]};
+                }
+                const float d = dot(rn, cur) - reference.w;
+                const V3 point = add(rm.pos, rotate(rq, sub(cur, mul(rn, d * 0.5f))));
+                const float pen = rest - d + 1.0e-5f;
+                for (uint32_t keep = row_bits(k0 + lane < count && !(d > reach)); keep != 0u; keep &= keep - 1u) {
+                    const uint32_t k = __builtin_ctz(keep);
+                    row_add_contact(out, lane, row_get(point, k), __shfl(pen, int(k), 16), smax(margin * 2.0f, 1.0e-4f));
+                }
             }
         }
     }
-    if (out.count == 0u) return kFaceDeclined;
+    if (out.count == 0u) return false;
     row_reduce_patch(out, lane, S, smax(1.0e-6f, margin * 1.0e-3f));
-    return kFaceSolved;
+    return true;
 }
 
-// The separating-axis half of swept_convex_face_manifold for a row.
+// The separating-axis half of rigid_swept_convex_face_manifold
+// (geometry.slang:1751-1853) for a row.
 enum : uint32_t { kSweptDecline = 0, kSweptEmpty = 1, kSweptTouching = 2, kSweptImpact = 3 };
 __device__ __forceinline__ uint32_t row_swept_entry(const FaceGeometry &geo, const FaceSide &pb, const FaceSide &b,
                                                     const FaceSide &pc, const FaceSide &c, float margin, uint32_t lane,
@@ -2217,8 +2084,7 @@ __global__ void __launch_bounds__(kNarrowBlock) k_narrowphase(const uint32_t *np
 // The queued mesh pairs, one row of 16 lanes each.  The face path runs at
 // most twice on the swept side (at the predicted states, then at the previous
 // ones, or at the time of impact) and once without; the rows of a wavefront
-// may be at different ones of these.  Pairs whose polygon outgrows the row
-// are queued for k_face_wide.
+// may be at different ones of these.
 //
 // One lane per pair took 213 us on a 55-box pyramid and 716 us on a heap of
 // 32768 bodies (one lane's serial search and clipping in scratch memory, too
@@ -2241,7 +2107,7 @@ struct FaceResult {                     // in the place of the input of a pair t
     float normal[3], impact;
     uint32_t count, face_patch, kind, start;
 };
-enum : uint32_t { kResultEmit = 0, kResultTriangles = 1, kResultWide = 2 };
+enum : uint32_t { kResultEmit = 0, kResultTriangles = 1 };
 struct FaceRecord {
     union {
         FaceInput in;
@@ -2265,7 +2131,7 @@ __global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_
                                                            const ShapeDev *shapes, FaceGeometry geo,
                                                            const PmhRigidBodyState *prev, const PmhRigidBodyState *pred,
                                                            const uint2 *ab, NarrowOut o, uint32_t *tri_list,
-                                                           uint32_t *wide_list, const HingeFrame *frames) {
+                                                           const HingeFrame *frames, uint32_t widest) {
     __shared__ FaceShared shared_rows[kFaceRows];
     __shared__ FaceRecord records[kFaceChunk];
     __shared__ uint8_t list[kFaceChunk];
@@ -2276,7 +2142,7 @@ __global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_
     // One pair per row while blocks are left, then more per block.
     const uint32_t share = (F + gridDim.x - 1) / gridDim.x;
     const uint32_t chunk = min(max((share + kFaceRows - 1) / kFaceRows * kFaceRows, kFaceRows), kFaceChunk);
-    enum : uint32_t { kPlain, kAtEnd, kAtStart, kAtImpact, kDone, kWide, kListed };
+    enum : uint32_t { kPlain, kAtEnd, kAtStart, kAtImpact, kDone, kListed };
     for (uint32_t base = blockIdx.x * chunk; base < F; base += gridDim.x * chunk) {
         const uint32_t pairs = min(chunk, F - base);
         if (threadIdx.x < pairs) {
@@ -2329,7 +2195,7 @@ __global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_
             const uint32_t todo = stage == 0u ? pairs : listed;
             for (uint32_t k = row; k < todo; k += kFaceRows) {
                 FaceRecord &r = records[stage == 0u ? k : list[k]];
-                const uint32_t m = r.pair, flags = r.flags;
+                const uint32_t flags = r.flags;
                 const float margin = r.in.margin, rest = smin(margin, 1.0e-3f);
                 const bool swept = (flags & kFaceSwept) != 0u;
                 RowManifold man;
@@ -2366,7 +2232,7 @@ __global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_
                     const float reach = mg + (at == kPlain ? r.in.reach : 0.0f);
                     if (search) axis = row_axis(geo, a, b, reach, lane);
                     search = true;
-                    uint32_t got = kFaceSolved;
+                    bool ok = true;
                     man.count = 0;
                     man.impact = 1.0f;
                     if (axis != kFaceApart) {
@@ -2383,13 +2249,10 @@ __global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_
                             at = kListed;
                             break;
                         }
-                        got = row_clip(geo, a, b, mg, reach, axis, lane, S, man);
+                        ok = row_clip(geo, a, b, mg, reach, axis, widest, lane, S, man);
                     }
-                    const bool ok = got == kFaceSolved;
                     face_patch = ok && man.count != 0u ? 1u : 0u;
-                    if (got == kFaceWide) {
-                        at = kWide;
-                    } else if (at == kPlain) {
+                    if (at == kPlain) {
                         face = ok && !(swept && man.count == 0u);
                         at = kDone;
                     } else if (!ok || man.count == 0u) {
@@ -2423,8 +2286,8 @@ __global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_
                 if (lane == 0u) {
                     r.out.normal[0] = man.normal.x; r.out.normal[1] = man.normal.y; r.out.normal[2] = man.normal.z;
                     r.out.impact = man.impact;
-                    r.out.kind = at == kWide ? kResultWide : face ? kResultEmit : kResultTriangles;
-                    r.out.count = at != kWide && face ? man.count : 0u;
+                    r.out.kind = face ? kResultEmit : kResultTriangles;
+                    r.out.count = face ? man.count : 0u;
                     r.out.face_patch = face_patch;
                 }
             }
@@ -2438,24 +2301,20 @@ __global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_
             FaceRecord &r = records[live ? threadIdx.x : 0u];
             const uint32_t kind = live ? r.out.kind : kResultEmit;
             uint32_t count = live ? r.out.count : 0u;
-            const uint64_t tri = __ballot(kind == kResultTriangles), wide = __ballot(kind == kResultWide);
+            const uint64_t tri = __ballot(kind == kResultTriangles);
             const uint32_t before = wave_exclusive_scan(count, threadIdx.x), total = wave_sum(count);
-            uint32_t at_point = 0, at_tri = 0, at_wide = 0;
+            uint32_t at_point = 0, at_tri = 0;
             if (threadIdx.x == 0u) {
                 if (total) at_point = atomicAdd(&o.ctr->point_alloc, total);
                 if (tri) at_tri = atomicAdd(&o.ctr->tri_pairs, uint32_t(__popcll(tri)));
-                if (wide) at_wide = atomicAdd(&o.ctr->wide_pairs, uint32_t(__popcll(wide)));
             }
             const uint64_t below = (1ull << threadIdx.x) - 1ull;
             const uint32_t start = __shfl(at_point, 0, 64) + before;
             at_tri = __shfl(at_tri, 0, 64) + uint32_t(__popcll(tri & below));
-            at_wide = __shfl(at_wide, 0, 64) + uint32_t(__popcll(wide & below));
             if (live) {
                 const uint32_t m = r.pair;
                 if (kind == kResultTriangles) {
                     tri_list[at_tri] = m;
-                } else if (kind == kResultWide) {
-                    wide_list[at_wide] = m;
                 } else {
                     if (count && start + count > o.point_cap) {
                         atomicOr(&o.ctr->status, kStatusPointOverflow);
@@ -2495,49 +2354,6 @@ __global__ void __launch_bounds__(kFaceBlock) k_face_pairs(const uint32_t *face_
             o.c_pair[i] = m;
         }
         __syncthreads();
-    }
-}
-
-// Listed pairs one lane each, with the serial functions: a polygon clipped by
-// more planes than lanes can hold vertices for.  A plane adds at most one
-// vertex to a triangle's three, so only shapes of more than 13 triangles get
-// here.
-constexpr uint32_t kRowFaces = kFaceLanes - 3;
-__global__ void __launch_bounds__(128) k_face_wide(const uint32_t *wide_list, const PmhBodyParameters *P,
-                                                   const ShapeDev *shapes, const V3 *verts, const uint32_t *idx,
-                                                   const float4 *planes, const PmhRigidBodyState *prev,
-                                                   const PmhRigidBodyState *pred, const uint2 *ab, NarrowOut o,
-                                                   uint32_t *tri_list, const HingeFrame *frames,
-                                                   const float4 *frame_ref) {
-    const uint32_t F = o.ctr->wide_pairs;
-    for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < F; f += gridDim.x * blockDim.x) {
-        const uint32_t m = wide_list[f];
-        const uint2 p = ab[m];
-        const PmhBodyParameters pa = P[p.x], pb = P[p.y];
-        ShapeView sa{shapes[pa.mesh_index], verts, idx, planes};
-        ShapeView sb{shapes[pb.mesh_index], verts, idx, planes};
-        const PmhRigidBodyState A0 = prev[p.x], A = pred[p.x], B0 = prev[p.y], B = pred[p.y];
-        const float margin = pa.collision_margin + pb.collision_margin;
-        const float cr = correction_reach(pa, sa.s) + correction_reach(pb, sb.s);
-        const PairFrames fr = pair_frames(frames, frame_ref, pa, pb, p, A0, A);
-        Manifold man;
-        man.count = 0;
-        man.face_patch = 0;
-        bool face = false;
-        // A guided pair leaves the face path (geometry.slang:2779).
-        if (sa.s.convex_face && sb.s.convex_face && !guided_pair(fr.ha, fr.hb)) {
-            const bool swept = requires_swept(A0, A, sa.s, B0, B, sb.s, margin);
-            if (swept) face = swept_convex_face_manifold(A0, A, sa, B0, B, sb, margin, man);
-            if (!face) {
-                face = convex_face_manifold(A, sa, B, sb, margin, cr, man);
-                if (swept && man.count == 0u) face = false;
-            }
-        }
-        if (!face) {
-            tri_list[wave_reserve(&o.ctr->tri_pairs, 1u)] = m;
-            continue;
-        }
-        emit_manifold(o, m, man, A, B, persistent_pair(sa.s, sb.s, pb), fr.ha, fr.hb);
     }
 }
 
@@ -3148,7 +2964,6 @@ __global__ void k_step_begin(StepCounters *ctr) {
     ctr->tri_pairs = 0;
     ctr->tri_hits = 0;
     ctr->face_pairs = 0;
-    ctr->wide_pairs = 0;
     ctr->fallback_pairs = 0;
     ctr->cell_size_bits = 0.0f;
 }
@@ -3255,13 +3070,9 @@ PmhResult World::step_once(uint32_t k_step, bool warm_infer) {
     k_narrowphase<<<blocks_for(v.pair_cap, kNarrowBlock, 2048), kNarrowBlock, 0, s>>>(&ctr->pairs, params.p, shapes_dev.p, prev, pred,
                                                                     v.ab.p, out, v.face_list.p, frames, frame_ref);
     const FaceGeometry geo{verts_dev.p, idx_dev.p, planes_dev.p};
-    // The list of wide pairs lies in the impact flags, written later.
     k_face_pairs<<<blocks_for(v.pair_cap, kFaceRows, 4096), kFaceBlock, 0, s>>>(
-        v.face_list.p, params.p, shapes_dev.p, geo, prev, pred, v.ab.p, out, v.tri_list.p, v.m_impact.p, frames);
-    if (face_triangles > kRowFaces)
-        k_face_wide<<<blocks_for(v.pair_cap, 128, 1024), 128, 0, s>>>(
-            v.m_impact.p, params.p, shapes_dev.p, verts_dev.p, idx_dev.p, planes_dev.p, prev, pred, v.ab.p, out,
-            v.tri_list.p, frames, frame_ref);
+        v.face_list.p, params.p, shapes_dev.p, geo, prev, pred, v.ab.p, out, v.tri_list.p, frames,
+        std::min(face_row_limit, kFaceLanes));
     // The face list is free by now, the adjacency not yet in use.
     auto *hit_mask = reinterpret_cast<unsigned long long *>(v.adj.p);
     k_triangle_screen<<<blocks_for(v.pair_cap, kScreenBlock, 1024), kScreenBlock, 0, s>>>(

@@ -109,7 +109,6 @@ struct StepCounters {
     uint32_t sweep_ticket[2];  // work tickets of the dataflow sweep, alternating per sweep
     uint32_t sweep_failed;     // a dataflow-sweep wait ran out; stays set until the host reports it
     uint32_t face_pairs;       // mesh pairs queued for the convex face path
-    uint32_t wide_pairs;       // of those, pairs whose clipped polygon outgrew a row of lanes
 };
 
 // Running totals over every step since the last reset.

@@ -309,10 +309,8 @@ PmhResult World::ensure_device() {
         std::vector<float4> planes, shell;
         std::vector<BvhDev> nodes;
         std::vector<uint32_t> leaves;
-        face_triangles = 0;
         for (HostShape &s : shapes) {
             ShapeDev d = s.info;
-            if (d.convex_face) face_triangles = std::max(face_triangles, d.idx_count / 3);
             d.vtx_off = uint32_t(verts.size());
             d.idx_off = uint32_t(idx.size());
             d.plane_off = uint32_t(planes.size());
@@ -915,6 +913,12 @@ PmhResult pmhWorldSetGravity(PmhWorld world, const float gravity[3]) {
 PmhResult pmhWorldSetSweepWaitLimit(PmhWorld world, uint32_t polls) {
     if (!world) return PMH_ERROR_INVALID_ARGUMENT;
     W(world)->sweep_wait_limit = polls;
+    return PMH_SUCCESS;
+}
+
+PmhResult pmhWorldSetFaceRowLimit(PmhWorld world, uint32_t vertices) {
+    if (!world) return PMH_ERROR_INVALID_ARGUMENT;
+    W(world)->face_row_limit = vertices;
     return PMH_SUCCESS;
 }
 

@@ -18,6 +18,7 @@ struct World {
     float residual_tolerance = 0.0f;
     uint32_t color_wait_limit = kColorWaitLimit;
     uint32_t sweep_wait_limit = kColorWaitLimit;
+    uint32_t face_row_limit = 16;     // vertices of a clipped polygon on the face path's rows
     int device = 0;
     hipStream_t stream = nullptr;
 
@@ -74,7 +75,6 @@ struct World {
     DBuf<float4> proxy_mn, proxy_mx;
     DBuf<int4> cell_of;
     uint32_t table_size = 0;
-    uint32_t face_triangles = 0;      // most triangles of a shape on the convex face path
     float grid_cell = 1.0f;
     DBuf<uint32_t> bucket_count, bucket_start, large, cand_count, cand_offset;
     // Per bucket entry, in entry order: the body's cell (w: 1 if dynamic), its

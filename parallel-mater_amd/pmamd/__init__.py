@@ -102,6 +102,7 @@ def lib():
         "pmhWorldStep": (i32, [_P, _U]),
         "pmhWorldSetColorWaitLimit": (i32, [_P, _U]),
         "pmhWorldSetSweepWaitLimit": (i32, [_P, _U]),
+        "pmhWorldSetFaceRowLimit": (i32, [_P, _U]),
         "pmhWorldApplyRigidInputs": (i32, [_P, _U, _P]),
         "pmhWorldSetKinematicTargets": (i32, [_P, _U, _U, _P]),
         "pmhWorldAddJoints": (i32, [_P, _U, _P]),
@@ -347,6 +348,11 @@ class World:
         """Polls of one dataflow-sweep wait before it fails the step
         (default 2**22); 0 fails at the first unmet wait."""
         _check(lib().pmhWorldSetSweepWaitLimit(self._h, polls), "pmhWorldSetSweepWaitLimit")
+
+    def set_face_row_limit(self, vertices):
+        """Vertices of a clipped polygon on the face path's rows (default
+        and most: 16); wider ones are clipped on one lane."""
+        _check(lib().pmhWorldSetFaceRowLimit(self._h, vertices), "pmhWorldSetFaceRowLimit")
 
     def residuals(self, maximum=False):
         """(per-iteration RMS constraint residuals [2, 64], NaN where no
