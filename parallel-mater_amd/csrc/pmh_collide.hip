@@ -1378,9 +1378,11 @@ __device__ __forceinline__ void merge_contact(const TrianglePair &P, Manifold &m
     else add_contact(m, c, spacing);
 }
 
-// rigid_collide_triangle_ranges: triangles in order, body-major.
+// rigid_collide_triangle_ranges: triangles in order, body-major.  Called on
+// the four lanes of a closest-point search, which share the manifold: one of
+// them (`writer`) reads and writes it.
 __device__ void collide_triangle_ranges(const TrianglePair &P, uint32_t a_first, uint32_t a_count,
-                                        uint32_t b_first, uint32_t b_count, Manifold &m) {
+                                        uint32_t b_first, uint32_t b_count, Manifold &m, bool writer) {
     if (guided_pair(P.f.ha, P.f.hb)) return;   // geometry.slang:1371
     bool inside_a, inside_b;
     inside_flags(P, inside_a, inside_b);
@@ -1392,13 +1394,13 @@ __device__ void collide_triangle_ranges(const TrianglePair &P, uint32_t a_first,
             const uint32_t bt = b_first + bi;
             if (3u * bt + 2u >= P.bm.s.idx_count) break;
             Contact c;
-            if (triangle_pair_contact(P, at, bt, inside_a, inside_b, c)) add_contact(m, c, spacing);
+            if (triangle_pair_contact(P, at, bt, inside_a, inside_b, c) && writer) add_contact(m, c, spacing);
         }
     }
 }
 
 __device__ void collide_triangle_ranges_swept(const TrianglePair &P, uint32_t a_first, uint32_t a_count,
-                                              uint32_t b_first, uint32_t b_count, Manifold &m) {
+                                              uint32_t b_first, uint32_t b_count, Manifold &m, bool writer) {
     bool inside_a, inside_b;
     inside_flags(P, inside_a, inside_b);
     const float spacing = smax(P.margin * 2.0f, 1.0e-4f);
@@ -1409,7 +1411,7 @@ __device__ void collide_triangle_ranges_swept(const TrianglePair &P, uint32_t a_
             const uint32_t bt = b_first + bi;
             if (3u * bt + 2u >= P.bm.s.idx_count) break;
             Contact c;
-            if (triangle_pair_swept_contact(P, at, bt, inside_a, inside_b, c)) merge_contact(P, m, c, spacing);
+            if (triangle_pair_swept_contact(P, at, bt, inside_a, inside_b, c) && writer) merge_contact(P, m, c, spacing);
         }
     }
 }
@@ -1447,16 +1449,18 @@ __device__ __forceinline__ void node_bounds(const BvhDev &nd, const BoundsFrame 
 }
 
 __device__ __forceinline__ void collide_leaf_ranges(const TrianglePair &P, bool swept, const BvhDev &na,
-                                                    const BvhDev &nb, Manifold &m) {
-    collide_triangle_ranges(P, na.first, na.count, nb.first, nb.count, m);
-    if (swept) collide_triangle_ranges_swept(P, na.first, na.count, nb.first, nb.count, m);
+                                                    const BvhDev &nb, Manifold &m, bool writer) {
+    collide_triangle_ranges(P, na.first, na.count, nb.first, nb.count, m, writer);
+    if (swept) collide_triangle_ranges_swept(P, na.first, na.count, nb.first, nb.count, m, writer);
 }
 
 // rigid_collide_meshes: simultaneous descent with a 64-entry stack, all
 // triangles when the stack would overflow.
-__device__ __noinline__ void collide_meshes(const TrianglePair &P, bool swept, Manifold &m) {
-    m.count = 0;
-    m.face_patch = 0;
+__device__ __noinline__ void collide_meshes(const TrianglePair &P, bool swept, Manifold &m, bool writer) {
+    if (writer) {
+        m.count = 0;
+        m.face_patch = 0;
+    }
     const BoundsFrame fa = bounds_frame(P.a), fb = bounds_frame(P.b);
     const BoundsFrame pfa = swept ? bounds_frame(P.ap) : BoundsFrame{};
     const BoundsFrame pfb = swept ? bounds_frame(P.bp) : BoundsFrame{};
@@ -1479,7 +1483,7 @@ __device__ __noinline__ void collide_meshes(const TrianglePair &P, bool swept, M
         if (!boxes_touch(amn, amx, bmn, bmx)) continue;
         const bool la = na.count != 0u, lb = nb.count != 0u;
         if (la && lb) {
-            collide_leaf_ranges(P, swept, na, nb, m);
+            collide_leaf_ranges(P, swept, na, nb, m, writer);
             continue;
         }
         const uint32_t need = la || lb ? 2u : 4u;
@@ -1498,10 +1502,12 @@ __device__ __noinline__ void collide_meshes(const TrianglePair &P, bool swept, M
         }
     }
     if (overflow) {
-        m.count = 0;
-        m.face_patch = 0;
-        collide_triangle_ranges(P, 0, P.am.s.idx_count / 3u, 0, P.bm.s.idx_count / 3u, m);
-        if (swept) collide_triangle_ranges_swept(P, 0, P.am.s.idx_count / 3u, 0, P.bm.s.idx_count / 3u, m);
+        if (writer) {
+            m.count = 0;
+            m.face_patch = 0;
+        }
+        collide_triangle_ranges(P, 0, P.am.s.idx_count / 3u, 0, P.bm.s.idx_count / 3u, m, writer);
+        if (swept) collide_triangle_ranges_swept(P, 0, P.am.s.idx_count / 3u, 0, P.bm.s.idx_count / 3u, m, writer);
     }
 }
 
@@ -2465,17 +2471,20 @@ __device__ uint32_t traversal_list(const TrianglePair &P, bool swept, uint2 *lis
 }
 
 // Serial evaluation for the rare pairs whose leaf list does not fit in
-// LDS: the same candidate order and merge rule on one lane (four lanes of
-// the same data, which the closest-point search is laid out for).  Leaf
+// LDS: the same candidate order and merge rule, the contacts computed on four
+// lanes of the same data (which the closest-point search is laid out for) and
+// merged by one of them (`writer`), which alone touches the manifolds.  Leaf
 // candidates come from the motion test alone (`swept`); the ranges of a
 // guided pair always take the swept pass (`swept_eval`).
 __device__ void triangle_pair_serial(const TrianglePair &tp, bool swept, bool swept_eval, bool leaf_mode,
-                                     Manifold &man, Manifold &local) {
-    man.count = 0;
-    man.face_patch = 0;
+                                     Manifold &man, Manifold &local, bool writer) {
     if (!leaf_mode) {
-        collide_meshes(tp, swept_eval, man);
+        collide_meshes(tp, swept_eval, man, writer);
         return;
+    }
+    if (writer) {
+        man.count = 0;
+        man.face_patch = 0;
     }
     const BoundsFrame fa = bounds_frame(tp.a), fb = bounds_frame(tp.b);
     const BoundsFrame pfa = swept ? bounds_frame(tp.ap) : BoundsFrame{};
@@ -2486,10 +2495,13 @@ __device__ void triangle_pair_serial(const TrianglePair &tp, bool swept, bool sw
         for (uint64_t f = w; f < cells; f += 128u) {
             uint2 nodes;
             if (!leaf_cell_overlaps(tp, swept, fa, fb, pfa, pfb, f, nodes)) continue;
-            local.count = 0;
-            local.face_patch = 0;
-            collide_leaf_ranges(tp, swept_eval, tp.am.node(nodes.x), tp.bm.node(nodes.y), local);
-            for (uint32_t k = 0; k < local.count; ++k) merge_contact(tp, man, local.c[k], spacing);
+            if (writer) {
+                local.count = 0;
+                local.face_patch = 0;
+            }
+            collide_leaf_ranges(tp, swept_eval, tp.am.node(nodes.x), tp.bm.node(nodes.y), local, writer);
+            if (writer)
+                for (uint32_t k = 0; k < local.count; ++k) merge_contact(tp, man, local.c[k], spacing);
         }
 }
 
@@ -2699,7 +2711,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         wave_sync();
         // 2. Contacts.
         if (nlist == kListOverflow) {
-            if (lane < 4u && !(wide && wv != 0)) triangle_pair_serial(tp, swept, swept_eval, leaf_mode, S.man, S.local);
+            if (lane < 4u && !(wide && wv != 0)) triangle_pair_serial(tp, swept, swept_eval, leaf_mode, S.man, S.local, lane == 0);
         } else {
             if (lane == 0) {
                 S.man.count = 0;
