@@ -1126,14 +1126,24 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t flow_box(const SolveArgs &a) {
     return __builtin_amdgcn_make_buffer_rsrc(a.flow, 0, int(flow_offset(a.n)), 0x00020000);
 }
 
+// After an unmet poll of a dataflow sweep's wait: whether the wait ends there.
+// One that runs out raises the abort flag, which ends every other wait of the
+// step, and marks the status and the sweep (kept until the host reports it),
+// so the step keeps its states and fails instead of hanging.  The abort flag
+// is read every 256th poll only: thousands of waiting lanes reading one
+// address on every poll would queue on one memory channel, and the waits would
+// slow down the bodies they wait for.
+__device__ __forceinline__ bool flow_gives_up(const SolveArgs &a, uint32_t polls) {
+    if (polls > a.flow_limit) {
+        st_relaxed(&a.ctr->color_abort, 1u);
+        st_relaxed(&a.ctr->sweep_failed, 1u);
+        atomicOr(&a.ctr->status, kStatusColorTimeout);
+        return true;
+    }
+    return (polls & 255u) == 0u && ld_relaxed(&a.ctr->color_abort) != 0u;
+}
 // Dataflow sweep: waits until body j has published this sweep's displacement
-// and takes it.  Bounded: a wait that runs out raises the abort flag, which
-// ends every other wait of the step, and marks the status and the sweep
-// (kept until the host reports it), so the step keeps its states and fails
-// instead of hanging.  The abort flag is read every 256th poll only:
-// thousands of waiting lanes reading one address on every poll would queue on
-// one memory channel, and the waits would slow down the bodies they wait for.
-// kW: the rotation delta's w with it, in d[6].
+// and takes it.  kW: the rotation delta's w with it, in d[6].
 template <bool kW = false>
 __device__ __forceinline__ void flow_take(const SolveArgs &a, __amdgpu_buffer_rsrc_t box, uint32_t j, float *d) {
     flow_pair w0, w1, w2, w3;
@@ -1146,13 +1156,7 @@ __device__ __forceinline__ void flow_take(const SolveArgs &a, __amdgpu_buffer_rs
         else w3[1] = s;
         if (((w0[1] ^ s) | (w0[3] ^ s) | (w1[1] ^ s) | (w1[3] ^ s) | (w2[1] ^ s) | (w2[3] ^ s) |
              (w3[1] ^ s)) == 0u) break;
-        if (polls > a.flow_limit) {
-            st_relaxed(&a.ctr->color_abort, 1u);
-            st_relaxed(&a.ctr->sweep_failed, 1u);
-            atomicOr(&a.ctr->status, kStatusColorTimeout);
-            break;
-        }
-        if ((polls & 255u) == 0u && ld_relaxed(&a.ctr->color_abort) != 0u) break;
+        if (flow_gives_up(a, polls)) break;
         // The mailbox is read again, not kept from the last poll.
         asm volatile("s_sleep 1" ::: "memory");
     }
@@ -1165,7 +1169,7 @@ __device__ __forceinline__ float flow_take_w(const SolveArgs &a, __amdgpu_buffer
     flow_pair w3;
     for (uint32_t polls = 1;; ++polls) {
         w3 = flow_load(box, j, 3);
-        if (w3[1] == a.flow_stamp || polls > a.flow_limit || ld_relaxed(&a.ctr->color_abort) != 0u) break;
+        if (w3[1] == a.flow_stamp || flow_gives_up(a, polls)) break;
         asm volatile("s_sleep 1" ::: "memory");
     }
     return __uint_as_float(w3[0]);
