@@ -1470,12 +1470,13 @@ __device__ __forceinline__ void solve_group(const SolveArgs &a, uint32_t base, u
             }
         }
     }
-    // From here to the mailbox the wavefront is on the chain over the
-    // colours; wavefronts that wait or update duals give way.
-    if constexpr (kFlow && L >= 16) __builtin_amdgcn_s_setprio(3);
     // Joint rows follow the contact rows (solve.slang:401-430), each
     // joint in one lane's partial block.
     if (kJoints && active) body_joint_rows<kFlow, L>(a, i, phase, blk, lane, dI, dq.w);
+    // Every wait is over: from here to the mailbox the wavefront is on the
+    // chain over the colours (with joints, from the last joint's wait on);
+    // wavefronts that wait or update duals give way.
+    if constexpr (kFlow && L >= 16) __builtin_amdgcn_s_setprio(3);
     group_reduce<L>(blk);
     float update[6];
     bool solved = false;
@@ -2044,6 +2045,11 @@ __device__ __forceinline__ void body_joint_rows(const SolveArgs &a, uint32_t i, 
         const uint32_t k = ent.x & ~kSideFirst, other = ent.y & kEntryBody;
         PmhRigidConstraint &j = a.joints[k];
         const bool wait = kFlow && (ent.y & kEntryLower) != 0u;
+        // A wait gives way to the wavefronts it may be waiting for.
+        if constexpr (kFlow && L >= 16) __builtin_amdgcn_s_setprio(0);
+        auto waited = [] {
+            if constexpr (kFlow && L >= 16) __builtin_amdgcn_s_setprio(3);
+        };
         float dO[7];
         JointEnds ends;
         auto pair_ends = [&]() {
@@ -2066,6 +2072,7 @@ __device__ __forceinline__ void body_joint_rows(const SolveArgs &a, uint32_t i, 
                 load_disp(a.disp, other, dO);
                 dO[6] = a.dq[other].w;
             }
+            waited();
             pair_ends();
             float unused = 0.0f;
             const PmhRigidBodyState sI = pose_at(tp, tq, {dI[0], dI[1], dI[2]},
@@ -2080,6 +2087,7 @@ __device__ __forceinline__ void body_joint_rows(const SolveArgs &a, uint32_t i, 
         PmhAvbdRow row = j.rows[0];
         if (wait) flow_take(a, flow_box(a), other, dO);
         else load_disp(a.disp, other, dO);
+        waited();
         dO[6] = 1.0f;
         pair_ends();
 #pragma unroll 1
