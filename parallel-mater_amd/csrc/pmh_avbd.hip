@@ -88,8 +88,10 @@ __device__ __forceinline__ T wave_fold(T x, F f) {
 // between data and flag: a word whose stamp is this sweep's holds this
 // sweep's value.  Written by 64-bit agent-scope stores, read two words per
 // 16-byte agent-scope load (the sc1 bit: the L2 caches of the eight XCDs are
-// not coherent with each other inside a kernel); each word is consistent in
-// itself and the stamps tell whether all of them have arrived.
+// not coherent with each other inside a kernel); the stamps tell whether all
+// words have arrived.  That such a load returns each aligned 8-byte word whole,
+// as one store left it, is an assumption about gfx950: the language promises it
+// of 8-byte atomics only.
 constexpr uint32_t kFlowUsed = 7;
 constexpr int kLoadAgent = 16;   // buffer load cache policy: sc1
 typedef uint32_t flow_pair __attribute__((ext_vector_type(4)));   // two words: value, stamp, value, stamp
@@ -102,14 +104,6 @@ __device__ __forceinline__ uint32_t wave_total(uint32_t v) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
     return v;
-}
-
-// Adds each lane's value to one counter with one atomic per wavefront
-// (every lane active).  Same-address atomics from every lane serialise in
-// one L2 channel; the counters here are read only after the kernel.
-__device__ __forceinline__ void wave_counter_add(uint32_t *counter, uint32_t v) {
-    const uint32_t t = wave_total(v);
-    if ((threadIdx.x & 63) == 0 && t) atomicAdd(counter, t);
 }
 
 // Adds each thread's K values to K counters with one atomic per counter and
@@ -320,12 +314,11 @@ __global__ void k_body_init(uint32_t n, const PmhBodyParameters *P, const PmhRig
                             float4 *tv, float4 *tw, float4 *disp, float4 *dq, float4 *inertia,
                             float4 *prev_vel, uint32_t *color, uint32_t *parent, uint32_t *impact,
                             uint32_t *deg, uint32_t *anchored, uint32_t *adj_cursor, uint32_t *members,
-                            float4 *mean, uint32_t *jdeg, uint32_t *jcursor) {
+                            float4 *mean, uint32_t *jdeg) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     members[i] = 0;
     jdeg[i] = 0;
-    jcursor[i] = 0;
     mean[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const PmhRigidBodyState s = st[i];
     tpos[i] = f4(sv(s.position), 0.0f);
@@ -453,7 +446,7 @@ __global__ void k_contact_init(const uint32_t *npairs, const PmhBodyParameters *
 // Graph: adjacency (dynamic endpoints only), islands, impact, colouring.
 // ---------------------------------------------------------------------
 __global__ void k_degree(const uint32_t *npairs, const PmhBodyParameters *P, const uint2 *ab,
-                         const uint32_t *m_count, uint32_t *deg, uint32_t *anchored_edge, StepCounters *ctr) {
+                         const uint32_t *m_count, uint32_t *deg, StepCounters *ctr) {
     const uint32_t M = *npairs;
     uint32_t local = 0, m1 = 0, m2 = 0, p1 = 0, p2 = 0;
     for (uint32_t m = blockIdx.x * blockDim.x + threadIdx.x; m < M; m += gridDim.x * blockDim.x) {
@@ -468,7 +461,6 @@ __global__ void k_degree(const uint32_t *npairs, const PmhBodyParameters *P, con
     uint32_t *const counters[5] = {&ctr->manifolds, &ctr->m1, &ctr->m2, &ctr->p1, &ctr->p2};
     const uint32_t values[5] = {local, m1, m2, p1, p2};
     block_counters_add<5>(counters, values);
-    (void)anchored_edge;
 }
 
 __global__ void k_adj_fill(const uint32_t *npairs, const PmhBodyParameters *P, const uint2 *ab,
@@ -866,8 +858,6 @@ __global__ void __launch_bounds__(64 * kColorWaveBlock) k_color_wave(uint32_t n,
     }
 }
 
-// Wave-aggregated histogram: one atomic per distinct colour per wavefront
-// (a few colours, tens of thousands of bodies).
 // Histogram and placement by blocks of 1024 bodies, each adding once per
 // colour it holds: atomics on one address serialise at 10 ns, and one per
 // colour and wavefront took 62 us each over 47000 bodies, now 5.
@@ -3115,7 +3105,7 @@ PmhResult Solver::each_buffer(uint32_t bodies, uint32_t pairs, uint32_t points, 
     R(impact, bodies); R(deg, positions + 1); R(adj_start, bodies + 1); R(adj_cursor, bodies);
     R(color_bodies, positions); R(bp_start, positions + 1); R(anchored, bodies); R(mean, bodies);
     R(members, bodies); R(mean_list, bodies);
-    R(jdeg, bodies + 1); R(jstart, bodies + 1); R(jcursor, bodies); R(joint_head, bodies);
+    R(jdeg, bodies + 1); R(jstart, bodies + 1); R(joint_head, bodies);
     R(prev_vel, bodies); R(flow, flow_words(bodies));
     R(code, pairs); R(ab, pairs); R(m_count, pairs + 1); R(m_start, pairs + 1); R(m_slot, pairs + 1);
     R(m_impact, pairs); R(m_face, pairs); R(m_init_rel, pairs); R(adj, 2 * (size_t)pairs);
@@ -3204,7 +3194,7 @@ void Solver::release() {
     inertia.release(); prev_vel.release(); color.release(); parent.release(); impact.release();
     deg.release(); adj_start.release(); adj_cursor.release(); color_bodies.release();
     bp_start.release(); anchored.release(); mean.release(); members.release(); mean_list.release(); flow.release();
-    jdeg.release(); jstart.release(); jcursor.release(); joint_head.release(); jadj.release();
+    jdeg.release(); jstart.release(); joint_head.release(); jadj.release();
     jent.release(); jstep.release(); code.release(); ab.release();
     m_count.release(); m_start.release(); m_slot.release(); m_impact.release(); m_face.release();
     m_init_rel.release(); adj.release(); tri_list.release(); face_list.release(); c_np.release(); c_pt.release(); c_aa.release();
@@ -3307,7 +3297,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
     k_body_init<<<bg, 256, 0, s>>>(n, P, previous, states, dt, sp.gravity, v.tpos.p, v.tq.p, v.tv.p, v.tw.p,
                                    v.disp.p, v.dq.p, v.inertia.p, v.prev_vel.p, v.color.p, v.parent.p,
                                    v.impact.p, v.deg.p, v.anchored.p, v.adj_cursor.p, v.members.p, v.mean.p,
-                                   v.jdeg.p, v.jcursor.p);
+                                   v.jdeg.p);
     k_contact_init<<<pg, 256, 0, s>>>(npairs, P, previous, states, v.ab.p, v.m_count.p, v.m_start.p, v.c_np.p,
                                       v.c_pt.p, v.c_aa.p, v.c_ab.p, v.c_err.p, v.c_lam.p, v.c_pen.p, v.c_flags.p,
                                       v.m_impact.p, v.c_entry.p, dt, sp.profile);
@@ -3327,7 +3317,7 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
     // Counting passes over the pairs: a smaller grid, so fewer blocks add
     // to the step's counters.
     const uint32_t count_g = std::min<uint32_t>(pg, 2u * uint32_t(device_compute_units()));
-    k_degree<<<count_g, 256, 0, s>>>(npairs, P, v.ab.p, v.m_count.p, v.deg.p, nullptr, ctr);
+    k_degree<<<count_g, 256, 0, s>>>(npairs, P, v.ab.p, v.m_count.p, v.deg.p, ctr);
     PmhResult r = exclusive_scan(s, v.deg.p, v.adj_start.p, n, nullptr, nullptr, v.scan_tmp);
     if (r != PMH_SUCCESS) return r;
     k_adj_fill<<<pg, 256, 0, s>>>(npairs, P, v.ab.p, v.m_count.p, v.adj_start.p, v.adj_cursor.p, v.adj.p);

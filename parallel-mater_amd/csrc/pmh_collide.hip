@@ -871,8 +871,7 @@ __device__ bool analytic_manifold(const PmhRigidBodyState &as, const ShapeDev &a
 // swept variant (geometry.slang:949-1117, 1272-1584, 1855-2154), the
 // leaf-pair candidate order of pm_generate_rigid_leaf_pairs (:2303-2492),
 // the per-candidate merge of pm_evaluate_rigid_leaf_pairs (:2525-2706)
-// and the BVH traversal of rigid_collide_meshes (:2156-2285).  One thread
-// per listed pair.
+// and the BVH traversal of rigid_collide_meshes (:2156-2285).
 // ---------------------------------------------------------------------
 __device__ __forceinline__ float normal_speed(const PmhRigidBodyState &b, const PmhRigidBodyState &c, V3 p, V3 n) {
     const V3 bv = add(sv(b.linear_velocity), cross(sv(b.angular_velocity), sub(p, sv(b.position))));
@@ -1511,23 +1510,6 @@ __device__ __noinline__ void collide_meshes(const TrianglePair &P, bool swept, M
     }
 }
 
-// Number of (body leaf, collider leaf) pairs whose motion bounds overlap.
-__device__ uint32_t count_leaf_candidates(const TrianglePair &P, bool swept, const BoundsFrame &fa,
-                                          const BoundsFrame &fb, const BoundsFrame &pfa, const BoundsFrame &pfb) {
-    const uint32_t la = P.am.s.leaf_count, lb = P.bm.s.leaf_count;
-    uint32_t total = 0;
-    for (uint32_t i = 0; i < la; ++i) {
-        V3 amn, amx;
-        node_bounds(P.am.node(P.am.leaf(i)), pfa, fa, swept, P.margin, amn, amx);
-        for (uint32_t j = 0; j < lb; ++j) {
-            V3 bmn, bmx;
-            node_bounds(P.bm.node(P.bm.leaf(j)), pfb, fb, swept, 0.0f, bmn, bmx);
-            total += boxes_touch(amn, amx, bmn, bmx) ? 1u : 0u;
-        }
-    }
-    return total;
-}
-
 // Narrowphase outputs: per-pair records and the point arrays, into which
 // each non-empty manifold writes a contiguous range.
 struct NarrowOut {
@@ -1676,9 +1658,6 @@ struct FaceSide {
     Q rot;
     uint32_t planes, verts, vert_count, indices, faces;
 };
-__device__ __forceinline__ FaceSide face_side(const PmhRigidBodyState &s, const ShapeDev &m) {
-    return {sv(s.position), sq(s.orientation), m.plane_off, m.vtx_off, m.vtx_count, m.idx_off, m.idx_count / 3};
-}
 __device__ __forceinline__ FaceSide pick(bool first, const FaceSide &a, const FaceSide &b) {
     FaceSide r;
     r.pos = {first ? a.pos.x : b.pos.x, first ? a.pos.y : b.pos.y, first ? a.pos.z : b.pos.z};

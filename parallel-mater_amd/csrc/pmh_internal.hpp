@@ -269,7 +269,7 @@ struct Solver {
     PmhRigidConstraint *joints = nullptr;
     uint32_t nj = 0;
     bool hinges = false;                 // some joint is a hinge (anchor projection)
-    DBuf<uint32_t> jdeg, jstart, jcursor, jadj, joint_head;
+    DBuf<uint32_t> jdeg, jstart, jadj, joint_head;
     DBuf<uint2> jent;                    // jadj's ends: joint and side, other body and flags
     DBuf<JointStep> jstep;               // one per joint
     // Every body's candidate joints (alive, both ids valid) in descending
