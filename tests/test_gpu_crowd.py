@@ -1,7 +1,8 @@
 # SPDX-License-Identifier: MIT
 """The grid query against the oracle's pairs: crowds in which a body has as
-many candidates as the group's memory holds, one less, one more and far more,
-and a wide moving body above a multiple of the chunks of the large scan."""
+many candidates as its segment of the pool holds (96 by default, 128 where the
+pair pool is larger: what the group's memory holds), one less, one more and far
+more, and a wide moving body above a multiple of the chunks of the large scan."""
 import numpy as np
 import pytest
 
@@ -35,12 +36,13 @@ def crowd(n, seed, wide):
     return S.Scene(shapes, p, st)
 
 
-@pytest.mark.parametrize("n", [2, 33, 64, 65, 128, 129, 130, 170])
+@pytest.mark.parametrize("n", [2, 33, 64, 65, 96, 97, 98, 128, 129, 130, 170])
 @pytest.mark.parametrize("wide", [False, True])
-def test_crowds_give_the_oracles_pairs(n, wide):
-    print("crowd", n, wide, flush=True)
+@pytest.mark.parametrize("pairs_per_body", [96, 192])
+def test_crowds_give_the_oracles_pairs(n, wide, pairs_per_body):
+    print("crowd", n, wide, pairs_per_body, flush=True)
     s = crowd(n, n, wide)
-    g = s.build(pmamd.World(profile=1))
+    g = s.build(pmamd.World(profile=1, pairs_per_body=pairs_per_body))
     o = s.build(O.OracleWorld(profile=1, lanes=32))
     g.step(1)
     o.step(1)
