@@ -387,6 +387,11 @@ PmhResult pmhWorldSetColorWaitLimit(PmhWorld world, uint32_t polls);
  * path without a stalled device. */
 PmhResult pmhWorldSetSweepWaitLimit(PmhWorld world, uint32_t polls);
 
+/* Number of the last sweep (32 bits, which wrap): the next ones count on from
+ * it.  It can be raised by an even count.  No counterpart in the reference; a
+ * test steps across the wrap with it. */
+PmhResult pmhWorldSetSweepStamp(PmhWorld world, uint32_t stamp);
+
 /* Vertices that a clipped polygon of the convex face path may have on a row
  * of 16 lanes (default and most: 16); wider ones are clipped on one lane, with
  * the same results.  No counterpart in the reference; a small limit lets a

@@ -3539,9 +3539,9 @@ PmhResult avbd_prepare_solve(hipStream_t s, Solver &v, const PmhBodyParameters *
             for (uint32_t it = 0; it < budget; ++it) {
                 if (flow) {
                     SolveArgs af = a;
-                    if (++v.sweep_stamp == 0u) {   // stamps wrapped: no stale stamp may match
-                        PMH_CHECK(hipMemsetAsync(v.flow.p, 0, sizeof(unsigned long long) * flow_words(n), s));
-                        v.sweep_stamp = 1u;
+                    if (++v.sweep_stamp == 0u) {   // stamps wrapped: no stale stamp may match, of a larger call either
+                        PMH_CHECK(hipMemsetAsync(v.flow.p, 0, sizeof(unsigned long long) * v.flow.n, s));
+                        v.sweep_stamp = 2u;   // even: the ticket counter that the last (odd) sweep cleared
                     }
                     af.flow_stamp = v.sweep_stamp;
                     hipEvent_t e0 = nullptr, e1 = nullptr;

@@ -916,6 +916,13 @@ PmhResult pmhWorldSetSweepWaitLimit(PmhWorld world, uint32_t polls) {
     return PMH_SUCCESS;
 }
 
+PmhResult pmhWorldSetSweepStamp(PmhWorld world, uint32_t stamp) {
+    if (!world || stamp < W(world)->solver.sweep_stamp || ((stamp ^ W(world)->solver.sweep_stamp) & 1u) != 0u)
+        return PMH_ERROR_INVALID_ARGUMENT;
+    W(world)->solver.sweep_stamp = stamp;
+    return PMH_SUCCESS;
+}
+
 PmhResult pmhWorldSetFaceRowLimit(PmhWorld world, uint32_t vertices) {
     if (!world) return PMH_ERROR_INVALID_ARGUMENT;
     W(world)->face_row_limit = vertices;

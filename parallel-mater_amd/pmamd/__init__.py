@@ -102,6 +102,7 @@ def lib():
         "pmhWorldStep": (i32, [_P, _U]),
         "pmhWorldSetColorWaitLimit": (i32, [_P, _U]),
         "pmhWorldSetSweepWaitLimit": (i32, [_P, _U]),
+        "pmhWorldSetSweepStamp": (i32, [_P, _U]),
         "pmhWorldSetFaceRowLimit": (i32, [_P, _U]),
         "pmhWorldApplyRigidInputs": (i32, [_P, _U, _P]),
         "pmhWorldSetKinematicTargets": (i32, [_P, _U, _U, _P]),
@@ -348,6 +349,11 @@ class World:
         """Polls of one dataflow-sweep wait before it fails the step
         (default 2**22); 0 fails at the first unmet wait."""
         _check(lib().pmhWorldSetSweepWaitLimit(self._h, polls), "pmhWorldSetSweepWaitLimit")
+
+    def set_sweep_stamp(self, stamp):
+        """Number of the last dataflow sweep (32 bits, which wrap); it can
+        be raised by an even count."""
+        _check(lib().pmhWorldSetSweepStamp(self._h, stamp), "pmhWorldSetSweepStamp")
 
     def set_face_row_limit(self, vertices):
         """Vertices of a clipped polygon on the face path's rows (default
