@@ -2073,8 +2073,8 @@ __global__ void __launch_bounds__(kNarrowBlock) k_narrowphase(const uint32_t *np
 //
 // One lane per pair took 213 us on a 55-box pyramid and 716 us on a heap of
 // 32768 bodies (one lane's serial search and clipping in scratch memory, too
-// few wavefronts in flight to hide it), and 538 us on 1024 scenes; rows take 30,
-// 186 and 194 us.
+// few wavefronts in flight to hide it), and 538 us on 1024 scenes; rows take 31,
+// 188 and 194 us.
 //
 // A block first reads its pairs one lane each (bodies, shapes, whether the
 // pair is swept) into records in LDS, then its rows take the records one by
